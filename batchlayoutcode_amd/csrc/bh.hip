@@ -24,9 +24,11 @@
 //                  with a shared stack of (node, lane mask): the vertex's own position is
 //                  the iteration-start one (it only moves in its own batch step), so all
 //                  n traversals run in one launch
-//   8. k_attract_move  one workgroup walks the ceil(n/B) batches in order: attraction
-//                  over every CSR entry with live positions (:1055-1058), minus the
-//                  repulsion, then the unit-step move (:1062-1066)
+//   8. the walk    attraction over every CSR entry with live positions (:1055-1058), minus the
+//                  repulsion, then the unit-step move (:1062-1066), as if batch after batch: in
+//                  FP64 mode k_attract_move, one workgroup walking the ceil(n/B) batches in
+//                  order; else by dependence levels (walk_level.hip) or, where a graph has too
+//                  many of them, one of the batch walks
 //   9. energy      sum of |F_i|^2
 //
 // FP32 mode evaluates the opening test D/|c-v| < theta in FP32 with a relative guard
@@ -1365,17 +1367,31 @@ constexpr size_t wrow_lds(bool has_w) {
            sizeof(int) * (2 * WROW_CAP + 4 * WROW_T) + (has_w ? sizeof(float) * 2 * WROW_CAP : 0);
 }
 
-// Whether k_walk_row can take batches of B vertices of graph g, and if so the early/late
-// split of the CSR on the device (both cached per batch size).  Early entries of a batch
-// must fit the walk's stage.
-bool row_walk_fits(bl_graph *g, int B) {
-    if (g->row_walk_batch == B) return g->row_walk_ok;
-    g->row_walk_batch = B;
-    g->row_walk_ok = false;
+// Whether k_walk_row can take batches of B vertices of graph g: early entries of a batch must fit
+// the walk's stage (cached per batch size).
+bool row_walk_takes(bl_graph *g, int B) {
+    if (g->row_takes_batch == B) return g->row_takes;
+    g->row_takes_batch = B;
+    g->row_takes = false;
     const int n = g->n;
     if (!(B <= WROW_T && g->nnz > 0 && g->max_row <= WROW_MAXDEG && (int)g->h_rowptr.size() == n + 1 &&
           (int64_t)g->h_colids.size() == g->nnz))
         return false;
+    batch_scan(g, B);
+    for (int c : g->batch_early)
+        if (c > WROW_CAP) return false;
+    g->row_takes = true;
+    return true;
+}
+
+// k_walk_row's early/late split of the CSR on the device (cached per batch size), where it takes
+// the graph.
+bool row_walk_fits(bl_graph *g, int B) {
+    if (g->row_walk_batch == B) return g->row_walk_ok;
+    g->row_walk_batch = B;
+    g->row_walk_ok = false;
+    if (!row_walk_takes(g, B)) return false;
+    const int n = g->n;
     const bool hw = !g->h_w.empty();
     std::vector<int32_t> erp(n + 1, 0), lrp(n + 1, 0), eci, lci;
     std::vector<float> ew, lw;
@@ -1391,8 +1407,6 @@ bool row_walk_fits(bl_graph *g, int B) {
         erp[i + 1] = (int32_t)eci.size();
         lrp[i + 1] = (int32_t)lci.size();
     }
-    for (int b0 = 0; b0 < n; b0 += B)
-        if (erp[std::min(n, b0 + B)] - erp[b0] > WROW_CAP) return false;
     // the walk reads index 0 of an empty list (clamped loads): keep one valid entry
     if (eci.empty()) eci.push_back(0), ew.push_back(0.0f);
     if (lci.empty()) lci.push_back(0), lw.push_back(0.0f);
@@ -1630,6 +1644,11 @@ __global__ __launch_bounds__(2 * WROW_T) void k_walk_row(const int *__restrict__
 constexpr int GW_T = 1024;
 constexpr int GW_G = 24;  // 8..32 measured on the R-MAT walk: 24 is fastest
 constexpr int GW_K = 4;  // entries per thread loaded a batch ahead
+// Measured times (us): a level of the walk by levels, on its own launch (5 to 25 with its size;
+// 5 where it decides) and in a run of small levels; a step of the lagged walk of 256 and of 512
+// vertices; a batch of the row walk.  The other walks take 4 us a batch or more, and there are never
+// more levels than batches.
+constexpr double LEVEL_US = 5.0, LEVEL_RUN_US = 2.3, LAG_US = 0.5, LAG512_US = 0.7, ROW_US = 2.2;
 constexpr int GW_MIN_ENTRIES = 4096;  // mean CSR entries per batch from which it is used
 
 struct GridWalk {
@@ -2174,6 +2193,27 @@ int launch_walk_grid(bl_graph *g, double2 *pos, const bl_params *p, double step,
 }
 }  // namespace
 
+void batch_scan(bl_graph *g, int B) {
+    if (g->batch_scan_of == B) return;
+    const int n = g->n, nb = (n + B - 1) / B;
+    g->batch_early.assign(nb, 0);
+    g->batch_top.assign(nb, -1);
+    for_ranges(nb, [&](int k0, int k1) {
+        for (int b = k0; b < k1; ++b) {
+            const int b0 = b * B;
+            int c = 0, top = -1;
+            for (int e = g->h_rowptr[b0]; e < g->h_rowptr[std::min(n, b0 + B)]; ++e) {
+                const int j = g->h_colids[e];
+                c += j < b0;
+                top = j < b0 ? std::max(top, j) : top;
+            }
+            g->batch_early[b] = c;
+            g->batch_top[b] = top;
+        }
+    }, n);
+    g->batch_scan_of = B;
+}
+
 int bh_build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s) {
     return build_tree(w, d_pos, n, s, nullptr, nullptr, false);
 }
@@ -2197,26 +2237,23 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     const int nbt = (n + p->batch - 1) / p->batch;
     bool use_grid = p->precision != BL_PREC_FP64 && p->batch <= WALK_MAXB &&
                     (double)g->nnz / (double)nbt >= (double)GW_MIN_ENTRIES;
-    bool use_row = p->precision != BL_PREC_FP64 && row_walk_fits(g, p->batch);
+    bool use_row = p->precision != BL_PREC_FP64 && row_walk_takes(g, p->batch);
     // where the multi-workgroup walk would run, the wide lagged walk (helper workgroups) runs
     // instead when its plan fits; BL_WALK=grid keeps the multi-workgroup walk, BL_WALK=wide
     // takes the wide walk wherever it fits
     bool want_wide = use_grid;
-    if (const char *wenv = getenv("BL_WALK")) {
+    const char *wenv = getenv("BL_WALK");
+    if (wenv) {
         if (!strcmp(wenv, "grid")) use_grid = p->precision != BL_PREC_FP64 && p->batch <= WALK_MAXB, want_wide = false;
         else if (!strcmp(wenv, "single")) use_grid = false, want_wide = false;
         else if (!strcmp(wenv, "pf")) use_grid = false, use_row = false, want_wide = false;
         else if (!strcmp(wenv, "row")) use_grid = false, want_wide = false;
         else if (!strcmp(wenv, "wide")) want_wide = p->precision != BL_PREC_FP64;
     }
-    const bool use_wide = want_wide && wide_walk_fits(g, p->batch);
+    int wide_d = 0;
+    bool use_wide = want_wide && wide_walk_takes(g, p->batch, &wide_d);
     int wide_h = 255;
     if (const char *v = getenv("BL_WIDE_H")) wide_h = std::max(1, atoi(v));
-    if (use_wide) {
-        rc = wide_walk_prepare(g->has_w);
-        if (rc) return rc;
-        use_grid = false;
-    }
     if (use_grid || use_wide) use_row = false;
     // the lagged walk (helper workgroups) where the row walk fits and the graph has enough batches;
     // BL_LAG_D / BL_LAG_H set its lag and helper count
@@ -2224,14 +2261,37 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     if (const char *v = getenv("BL_LAG_D")) lag_d = atoi(v);
     if (const char *v = getenv("BL_LAG_H")) lag_h = std::max(0, atoi(v));
     if (use_row && lag_d == 0) lag_d = lag_walk_choose(g, p->batch);
-    bool use_lag = use_row && lag_d > 0 && lag_walk_fits(g, p->batch, lag_d);
-    if (const char *wenv = getenv("BL_WALK"))  // row and single: one workgroup, no helpers
-        if (!strcmp(wenv, "row") || !strcmp(wenv, "single")) use_lag = false;
-    if (use_lag) {
-        rc = lag_walk_prepare(g->has_w);
-        if (rc) return rc;
+    int lag_w = 0;
+    int lag_steps = use_row && lag_d > 0 ? lag_walk_steps(g, p->batch, lag_d, &lag_w) : 0;
+    if (wenv && (!strcmp(wenv, "row") || !strcmp(wenv, "single"))) lag_steps = 0;  // no helpers
+    bool use_lag = lag_steps > 0;
+    // by dependence levels, whichever walk the graph's shape selects (its switches keep it)
+    const char *lenv = getenv("BL_LEVELS");
+    bool use_level = p->precision != BL_PREC_FP64 && iters > 0 && !wenv && !getenv("BL_LAG_D") && !getenv("BL_LAG_H") &&
+                     !getenv("BL_WIDE_D") && !getenv("BL_WIDE_H") && !(lenv && !strcmp(lenv, "0")) &&
+                     level_walk_plan(g, p->batch, use_lag ? lag_d : 0);
+    // The lagged walk stays on graphs whose ids follow the edges: a 1000 x 1000 grid in row order at
+    // -batch 256 has 1,001 levels and 3,907 steps, 2.26 against 1.98 ms (at -batch 64: 2.27 against
+    // 7.84); without such an order 24 levels against 976 steps, 0.12 against 0.53 ms (250k random
+    // geometric graph).
+    if (use_level && (use_lag || use_row) && !lenv)
+        use_level = LEVEL_US * g->lev_big + LEVEL_RUN_US * g->lev_small <
+                    (!use_lag ? ROW_US * nbt : (lag_w == 512 ? LAG512_US : LAG_US) * lag_steps);
+    if (!use_level) {
+        if (use_wide) use_wide = wide_walk_fits(g, p->batch);
+        if (use_wide) {
+            rc = wide_walk_prepare(g->has_w);
+            if (rc) return rc;
+            use_grid = false;
+        }
+        if (use_row) use_row = row_walk_fits(g, p->batch);
+        use_lag = use_lag && use_row && lag_walk_fits(g, p->batch, lag_d);
+        if (use_lag) {
+            rc = lag_walk_prepare(g->has_w);
+            if (rc) return rc;
+        }
     }
-    if (use_row) {
+    if (use_row && !use_level) {
         const size_t lb = wrow_lds(g->has_w);
         BL_HIP(hipFuncSetAttribute(g->has_w ? reinterpret_cast<const void *>(k_walk_row<true>)
                                             : reinterpret_cast<const void *>(k_walk_row<false>),
@@ -2283,7 +2343,12 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
                       : launch_rep(g->bh, n, theta, p->precision, s);
         prof.end();
         if (rc) return rc;
-        if (p->precision != BL_PREC_FP64 && !use_grid && use_row) {
+        if (use_level) {
+            prof.begin(5);
+            rc = launch_level_late(g, pos, p, s);
+            prof.end();
+            if (rc) return rc;
+        } else if (p->precision != BL_PREC_FP64 && !use_grid && use_row) {
             // the row walk's pre-pass: attraction of the neighbours in the same or a later batch
             prof.begin(5);
             hipLaunchKernelGGL(k_late_attract, dim3((n + 255) / 256), dim3(256), 0, s, g->late_rp.as<int>(),
@@ -2298,6 +2363,11 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
                                g->has_w ? g->w_edge.as<float>() : nullptr, p->weight, pos, g->bh.rep.as<double2>(),
                                g->scratch.as<double2>(), n, p->batch, STEP, g->eterm.as<double>(),
                                g->bh.misc.as<int>());
+        } else if (use_level) {
+            walk = use_wide ? BL_WALK_WIDE : use_grid ? BL_WALK_GRID : use_lag ? BL_WALK_LAG
+                   : use_row ? BL_WALK_ROW : p->batch <= WALK_MAXB ? BL_WALK_PF : BL_WALK_SPLIT;
+            rc = launch_walk_level(g, pos, p, STEP, s);
+            if (rc) return rc;
         } else if (use_wide) {
             walk = BL_WALK_WIDE;
             rc = launch_walk_wide(g, pos, p, STEP, wide_h, s);
@@ -2339,8 +2409,8 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     unsigned long long cells = 0;
     if (far_mode && far_mode != FAR_EXACT && iters > 0)
         BL_HIP(hipMemcpyAsync(&cells, ncells, sizeof(cells), hipMemcpyDeviceToHost, s));
-    int helped = 0;
-    if (walk == BL_WALK_LAG) BL_HIP(hipMemcpyAsync(&helped, lag_walk_helped(g), sizeof(int), hipMemcpyDeviceToHost, s));
+    int helped = use_level && walk == BL_WALK_LAG ? lag_steps : 0;
+    if (walk == BL_WALK_LAG && !use_level) BL_HIP(hipMemcpyAsync(&helped, lag_walk_helped(g), sizeof(int), hipMemcpyDeviceToHost, s));
     int model_iters = far_mode == FAR_LEARNED ? iters : 0;
     float judge_err[2] = {0.0f, 0.0f};
     if (judged && iters > 0) {
@@ -2355,7 +2425,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     }
     int gerr = 0, werr = 0, waited = 0;
     if (g->bh.gwalk_used) BL_HIP(hipMemcpyAsync(&gerr, gwalk_err(g->bh), sizeof(int), hipMemcpyDeviceToHost, s));
-    if (walk == BL_WALK_WIDE && (rc = wide_walk_read(g, &werr, &waited, s))) return rc;
+    if (walk == BL_WALK_WIDE && !use_level && (rc = wide_walk_read(g, &werr, &waited, s))) return rc;
     BL_HIP(hipStreamSynchronize(s));
     if (status & ST_DUPKEY) return BL_E_DUPKEY;
     if (gerr) return BL_E_DEVICE;  // a grid barrier timed out (the walk stopped early)
@@ -2368,7 +2438,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         st->far_cells = (int64_t)cells;
         st->far_model_iters = model_iters;
         st->walk_helped = helped;
-        st->walk_lag = walk == BL_WALK_LAG ? lag_d : walk == BL_WALK_WIDE ? g->wide_dmax : 0;
+        st->walk_lag = walk == BL_WALK_LAG ? lag_d : walk == BL_WALK_WIDE ? wide_d : 0;
         st->far_judge_err[0] = judge_err[0];
         st->far_judge_err[1] = judge_err[1];
         st->energy = E;

@@ -78,10 +78,16 @@ __device__ __forceinline__ void seg_step(double2 &v, int key) {
 // (ax, ay), with |d| = |d|^2 / sqrt(|d|^2) from rsqrt2 (coincident or nearly coincident vertices,
 // |d| < 2^-450, add nothing, where the reference adds at most 2^-900 W).  The walks with helper
 // workgroups use it in the walker and in the helpers alike, so their sums agree bit for bit.
-__device__ __forceinline__ void attr_add(double2 pj, double2 v, double Wk, double &ax, double &ay) {
-    const double dx = pj.x - v.x, dy = pj.y - v.y;
+__device__ __forceinline__ void attr_factors(double2 pj, double2 v, double Wk, double &dx, double &dy, double &sc) {
+    dx = pj.x - v.x;
+    dy = pj.y - v.y;
     const double d2 = dx * dx + dy * dy;
-    const double sc = d2 > 0x1p-900 ? Wk * (d2 * rsqrt2(d2)) : 0.0;
+    const double s = Wk * (d2 * rsqrt2(d2));  // formed whatever d2: a select, no branch
+    sc = d2 > 0x1p-900 ? s : 0.0;
+}
+__device__ __forceinline__ void attr_add(double2 pj, double2 v, double Wk, double &ax, double &ay) {
+    double dx, dy, sc;
+    attr_factors(pj, v, Wk, dx, dy, sc);
     ax = fma(dx, sc, ax);
     ay = fma(dy, sc, ay);
 }
@@ -96,22 +102,39 @@ constexpr int ST_DUPKEY = 1;
 // itself (far_cells_of).
 int bh_build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s);
 
-// The lagged batch walk (walk_lag.hip): lag_walk_fits builds the settled / recent split for
+// Per batch of B vertices: its early entries (neighbour in an earlier batch; g->batch_early) and the
+// largest early neighbour (-1: none; g->batch_top).  Cached per batch size.
+void batch_scan(bl_graph *g, int B);
+
+// The walk by dependence levels (walk_level.hip): level_walk_plan builds the plan for batch size B
+// (D > 0: with the sums of the lagged walk at lag D); launch_level_late sums the late attraction
+// into the repulsion, launch_walk_level runs one iteration's walk after it.
+bool level_walk_plan(bl_graph *g, int B, int D);
+int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, hipStream_t s);
+int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, double step, hipStream_t s);
+
+// The lagged batch walk (walk_lag.hip): lag_walk_choose gives the default lag for batches of B
+// vertices (0: not taken), lag_walk_steps the walk's steps at lag D (0: not taken) and their width,
+// lag_walk_groups the step of every vertex; lag_walk_fits builds the settled / recent split for
 // batch size B and lag D (false: the walk does not take this graph and batch size);
 // launch_walk_lag runs one iteration's walk with `helpers` helper workgroups (after
 // k_late_attract); lag_walk_prepare sets the kernels' LDS limit.
 int lag_walk_choose(bl_graph *g, int B);
+int lag_walk_steps(bl_graph *g, int B, int D, int *width);
+std::vector<int32_t> lag_walk_groups(bl_graph *g, int B);
 bool lag_walk_fits(bl_graph *g, int B, int D);
 int launch_walk_lag(bl_graph *g, double2 *pos, const bl_params *p, double step, int helpers, hipStream_t s);
 int lag_walk_prepare(bool has_w);
 int *lag_walk_helped(bl_graph *g);
 
-// The wide lagged batch walk (walk_wide.hip): wide_walk_fits builds the near / far split and
+// The wide lagged batch walk (walk_wide.hip): wide_walk_takes tells whether it takes the graph (and
+// its largest lag); wide_walk_fits builds the near / far split and
 // the helpers' chunks for batch size B (largest lag from BL_WIDE_D; false: the walk does not
 // take this graph and batch size); launch_walk_wide runs one iteration's walk (no pre-pass)
 // with up to `helpers` helper workgroups; wide_walk_read queues the copies of the error flag
 // and of the number of batches the walker waited for (valid after the stream synchronizes);
 // wide_walk_prepare sets the kernels' LDS limit.
+bool wide_walk_takes(const bl_graph *g, int B, int *dmax);
 bool wide_walk_fits(bl_graph *g, int B);
 int launch_walk_wide(bl_graph *g, double2 *pos, const bl_params *p, double step, int helpers, hipStream_t s);
 int wide_walk_read(bl_graph *g, int *err, int *waited, hipStream_t s);

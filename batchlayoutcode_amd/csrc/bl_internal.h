@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <thread>
 #include <vector>
 
 #include "batchlayout.h"
@@ -50,6 +52,22 @@ struct BHWork {
     void release();
 };
 
+// Lists of the walk by levels (walk_level.hip): short rows (in slices of 64 vertices, or a few lanes
+// each) and longer ones.
+struct LevelLists {
+    DevBuf head, vid, ids, w;  // slices: {first entry, columns}, vertices, entries
+    DevBuf row, rids, rw;      // longer rows: {vertex, first entry, past the last}, entries
+    void release() {
+        for (DevBuf *b : {&head, &vid, &ids, &w, &row, &rids, &rw}) b->release();
+    }
+};
+// One launch: levels [l0, l1) of slices from vertex slot v0 and entry block e0, or one level (l1 ==
+// l0): nn waves of rows of 4 lanes, nw of 8, then from row r0 nr rows of a wave and nh of a workgroup.
+struct LevelLaunch {
+    int32_t l0, l1, v0, nn, nw, r0, nr, nh;
+    uint32_t e0;
+};
+
 }  // namespace bl
 
 struct bl_graph {
@@ -63,6 +81,10 @@ struct bl_graph {
     std::vector<int32_t> h_rowptr, h_colids;  // host copy of the CSR (walk selection and split)
     std::vector<float> h_w;
     int32_t max_row = 0;            // longest CSR row
+    int32_t batch_scan_of = 0;      // batch size batch_early and batch_top were computed for
+    std::vector<int32_t> batch_early, batch_top;
+    int32_t row_takes_batch = 0;    // batch size row_takes was computed for
+    bool row_takes = false;
     int32_t row_walk_batch = 0;     // batch size row_walk_ok and the split were computed for
     bool row_walk_ok = false;
     // the CSR split for the one-workgroup row walk at batch size row_walk_batch: "early"
@@ -82,6 +104,7 @@ struct bl_graph {
     // per-vertex sums and per-group flags (launch generations)
     int32_t lag_batch = 0, lag_d = 0, lag_gen = 0, lag_width = 0, lag_ng = 0, lag_rcap = 0;
     int32_t lag_auto_batch = 0, lag_auto_d = 0;  // the default lag for batch size lag_auto_batch
+    int32_t lag_step_batch = 0, lag_steps = 0, lag_step_width = 0;  // the walk's steps at batch size lag_step_batch
     bool lag_ok = false;
     bl::DevBuf lag_erp, lag_esp, lag_eci, lag_ew, lag_rofs, lag_rw, lag_pre, lag_ready, lag_ring_of, lag_gstart,
         lag_sink;
@@ -93,6 +116,14 @@ struct bl_graph {
     bool wide_ok = false;
     bl::DevBuf wide_near_rp, wide_near_code, wide_near_w, wide_npa, wide_npb, wide_ring_of, wide_far_rp,
         wide_far_ci, wide_far_w, wide_chunks, wide_cfr, wide_nch, wide_pre, wide_cnt, wide_sink;
+    // the walk by dependence levels (walk_level.hip) at batch size lev_batch, with the sums of the
+    // lagged walk at lag lev_d (0: each row's early entries in CSR order)
+    int32_t lev_batch = 0, lev_d = 0, lev_big = 0, lev_small = 0, lev_late_slices = 0, lev_late_rows = 0,
+            lev_late_hubs = 0;
+    bool lev_ok = false;
+    bl::LevelLists lev_early, lev_late;
+    bl::DevBuf lev_start;
+    std::vector<bl::LevelLaunch> lev_launch;
     // the neighbours the reference's merge pointer actually meets (algorithms.cpp:758-762),
     // as a CSR of strictly increasing column ids per row (+ their weights)
     bl::DevBuf eff_rowptr, eff_colids, eff_w;
@@ -111,6 +142,23 @@ struct bl_graph {
 };
 
 namespace bl {
+
+// f(i0, i1) over [0, n) in contiguous ranges, on up to 8 host threads (one for small work, in
+// vertices): the passes over a graph's CSR that build the walks' plans.
+template <class F>
+void for_ranges(int n, F f, int work = -1) {
+    const int k = (work < 0 ? n : work) < (1 << 16) ? 1 : (int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
+    auto cut = [&](int t) { return (int)((int64_t)n * t / k); };
+    std::vector<std::thread> ts;
+    int t = 1;
+    try {
+        for (; t < k; ++t) ts.emplace_back(f, cut(t), cut(t + 1));
+    } catch (...) {  // no more threads: the rest here
+    }
+    f(0, cut(1));
+    if (t < k) f(cut(t), n);
+    for (std::thread &x : ts) x.join();
+}
 
 // Optional per-launch timing with HIP events on the launch stream (bl_params.profile).
 struct Prof {

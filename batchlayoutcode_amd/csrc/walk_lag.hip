@@ -61,6 +61,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <atomic>
 #include <vector>
 
 #include "bh_common.h"
@@ -465,16 +466,7 @@ std::vector<int32_t> lag_groups(const bl_graph *g, int B, int T) {
     std::vector<int32_t> gs{0};
     int cur0 = 0, size = 1;  // the open group: first vertex and batches
     for (int b = 1; b < nb; ++b) {
-        bool join = size < gmax;
-        for (int i = b * B; join && i < std::min(n, b * B + B); ++i)
-            for (int e = g->h_rowptr[i]; e < g->h_rowptr[i + 1]; ++e) {
-                const int j = g->h_colids[e];
-                if (j >= cur0 && j < b * B) {
-                    join = false;
-                    break;
-                }
-            }
-        if (join) {
+        if (size < gmax && g->batch_top[b] < cur0) {
             ++size;
         } else {
             gs.push_back(b * B);
@@ -488,7 +480,8 @@ std::vector<int32_t> lag_groups(const bl_graph *g, int B, int T) {
 
 // The group width for batches of B: 512 when its groups are at most four fifths as many as the
 // batches, else 256 (one batch a step for B > 128).
-int lag_width(const bl_graph *g, int B, std::vector<int32_t> *groups) {
+int lag_width(bl_graph *g, int B, std::vector<int32_t> *groups) {
+    batch_scan(g, B);
     const int nb = (g->n + B - 1) / B;
     std::vector<int32_t> gs = lag_groups(g, B, 512);
     int T = 512;
@@ -542,7 +535,34 @@ bool lag_ring_fits(const bl_graph *g, const std::vector<int32_t> &gs, const std:
     return true;
 }
 
+bool lag_takes(const bl_graph *g, int B, int D) {
+    return B <= LAG_BMAX && D >= 4 && D <= LAG_DMAX && g->nnz > 0 && g->max_row <= LAG_MAXDEG &&
+           (int)g->h_rowptr.size() == g->n + 1 && (int64_t)g->h_colids.size() == g->nnz;
+}
+bool lag_enough(int ng, int D) { return ng >= 2 * D && ng >= LAG_LEAD + 4; }
+
 }  // namespace
+
+// The walk's steps (groups) for batches of B vertices at the default lag D (lag_walk_choose), and
+// the group width; 0: the walk does not take the graph.
+int lag_walk_steps(bl_graph *g, int B, int D, int *width) {
+    if (!lag_takes(g, B, D)) return 0;
+    if (g->lag_step_batch != B) {
+        std::vector<int32_t> gs;
+        g->lag_step_width = lag_width(g, B, &gs);
+        g->lag_steps = (int)gs.size() - 1;
+        g->lag_step_batch = B;
+    }
+    *width = g->lag_step_width;
+    return lag_enough(g->lag_steps, D) ? g->lag_steps : 0;
+}
+
+// The step of every vertex.
+std::vector<int32_t> lag_walk_groups(bl_graph *g, int B) {
+    std::vector<int32_t> gs;
+    lag_width(g, B, &gs);
+    return group_of(gs, g->n);
+}
 
 // Whether the lagged walk takes batches of B vertices of graph g with lag D (groups), and if so
 // the groups, the settled / recent split of the early entries and the ring slots on the device
@@ -553,13 +573,11 @@ bool lag_walk_fits(bl_graph *g, int B, int D) {
     g->lag_d = D;
     g->lag_ok = false;
     const int n = g->n;
-    if (!(B <= LAG_BMAX && D >= 4 && D <= LAG_DMAX && g->nnz > 0 && g->max_row <= LAG_MAXDEG &&
-          (int)g->h_rowptr.size() == n + 1 && (int64_t)g->h_colids.size() == g->nnz))
-        return false;
+    if (!lag_takes(g, B, D)) return false;
     std::vector<int32_t> gs;
     const int T = lag_width(g, B, &gs);
     const int ng = (int)gs.size() - 1;
-    if (!(ng >= 2 * D && ng >= LAG_LEAD + 4)) return false;
+    if (!lag_enough(ng, D)) return false;
     const bool hw = !g->h_w.empty();
     const int rcap = lag_rcap(hw, T);
     const std::vector<int32_t> go = group_of(gs, n);
@@ -636,22 +654,30 @@ int lag_walk_choose(bl_graph *g, int B) {
     const int T = lag_width(g, B, &gs);
     const int ng = (int)gs.size() - 1;
     const std::vector<int32_t> go = group_of(gs, n);
-    int D = std::min(LAG_DMAX, ng / 2);
+    const int D0 = std::min(LAG_DMAX, ng / 2);
+    std::atomic<int> least{D0};
     static_assert(LAG_RS == 4, "the fifth-nearest gap bounds the lag");
-    for (int i = 0; i < n && D >= 4; ++i) {
-        const int gi = go[i], b0 = (i / B) * B;
-        int gap[LAG_RS + 1], cnt = 0;  // the five smallest gaps gi - gj >= 1, ascending
-        for (int e = g->h_rowptr[i]; e < g->h_rowptr[i + 1]; ++e) {
-            const int j = g->h_colids[e];
-            if (j >= b0) continue;  // late
-            const int k = gi - go[j];
-            if (cnt == LAG_RS + 1 && k >= gap[LAG_RS]) continue;
-            int m = cnt < LAG_RS + 1 ? cnt++ : LAG_RS;
-            while (m > 0 && gap[m - 1] > k) gap[m] = gap[m - 1], --m;
-            gap[m] = k;
+    for_ranges(n, [&](int i0, int i1) {
+        int D = D0;
+        for (int i = i0; i < i1 && D >= 4; ++i) {
+            const int gi = go[i], b0 = (i / B) * B;
+            int gap[LAG_RS + 1], cnt = 0;  // the five smallest gaps gi - gj >= 1, ascending
+            for (int e = g->h_rowptr[i]; e < g->h_rowptr[i + 1]; ++e) {
+                const int j = g->h_colids[e];
+                if (j >= b0) continue;  // late
+                const int k = gi - go[j];
+                if (cnt == LAG_RS + 1 && k >= gap[LAG_RS]) continue;
+                int m = cnt < LAG_RS + 1 ? cnt++ : LAG_RS;
+                while (m > 0 && gap[m - 1] > k) gap[m] = gap[m - 1], --m;
+                gap[m] = k;
+            }
+            if (cnt == LAG_RS + 1) D = std::min(D, gap[LAG_RS]);  // recent: gaps 1 .. D - 1
         }
-        if (cnt == LAG_RS + 1) D = std::min(D, gap[LAG_RS]);  // recent: gaps 1 .. D - 1
-    }
+        int old = least.load();
+        while (D < old && !least.compare_exchange_weak(old, D)) {
+        }
+    });
+    int D = least.load();
     const int rcap = lag_rcap(!g->h_w.empty(), T);
     if (D >= 4 && !lag_ring_fits(g, gs, go, B, D, rcap, nullptr)) {  // the largest D that fits
         int lo = 3, hi = D;  // fits(lo) or lo == 3; !fits(hi)

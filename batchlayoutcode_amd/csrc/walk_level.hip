@@ -1,0 +1,687 @@
+// The batch walk of the Barnes-Hut family (algorithms.cpp:1050-1066) by dependence levels.
+//
+// A vertex's new position is a function of its iteration-start position, its repulsion, the new
+// positions of its neighbours in earlier batches ("early") and the iteration-start positions of
+// the others ("late").  So the sequential batches are a dependence graph of vertices, not of
+// batches: level(i) = 1 + the largest level of an early neighbour (0 without one), and the
+// vertices of one level move at once whatever their batches.  There are never more levels than
+// batches, and on graphs with unordered ids there are about as many as the longest chain of
+// neighbours in increasing batch order: 18 on a triangulation of 1.66M points at -batch 256 (6,497
+// batches), 24 on the 250k random geometric graph (976), 199 on the R-MAT graph of scale 20
+// at -batch 1024 (534).  The result is the sequential walk's: the late terms are summed first,
+// for all vertices (k_level_late), before any vertex moves.
+//
+//   f_i = (sum over early, in list order) - rep'_i,    rep'_i = rep_i - sum over late
+//
+// What bounds a small level is its launch and its chain of dependent loads, about 5 us together, not
+// its arithmetic; a large one is bound by its random 16-byte reads and writes (25 us for 200k
+// vertices).  So a level's rows are laid out for two round trips, the vertices with their entries
+// and then every position these name:
+//   - rows of up to 4 entries take 4 lanes each, rows of up to 8 take 8, at an address that the lane's
+//     number gives: a lane forms the factors of one entry, and the lanes' products are added one after
+//     another by DPP moves;
+//   - rows of up to LV_WAVE entries one a wave, longer ones (hubs) one a workgroup, the row's header
+//     first.
+// One lane an entry also keeps the code short: with one lane a row, eight terms unrolled, a level
+// waited longer for its instructions (cold after every launch) than for its data (10 us against 5
+// for the small levels of the triangulation).
+// A level of more than LV_RUN vertices, or with a row beyond 8 entries, is one launch.  Runs of
+// smaller levels are one launch of one workgroup, which takes the levels one after another with a
+// barrier between them and loads a level's vertices and entries two levels ahead.
+//
+// Walk per iteration, with the late sums, before and after: triangulation of 1.66M points at -batch
+// 256 2.65 -> 0.28 ms (lagged walk), 250k random geometric graph 0.54 -> 0.13 ms (lagged walk),
+// R-MAT scale 20 at -batch 1024 2.07 -> 1.09 ms (wide walk), a 1000 x 1000 grid in row order at
+// -batch 64 7.84 -> 2.29 ms (lagged walk) and at -batch 1024 5.20 -> 0.15 ms (entry-split walk).
+//
+// Graphs for which the lagged walk (walk_lag.hip) is chosen keep its sums bit for bit: the
+// early neighbours at least D groups back ("settled") are summed first, the repulsion is
+// subtracted, then the others ("recent", marked in the entry) are added.
+#include <math.h>
+#include <stdlib.h>
+
+#include <algorithm>
+#include <new>
+#include <vector>
+
+#include "bh_common.h"
+#include "pair_math.h"
+
+namespace bl {
+namespace {
+
+constexpr int LV_NARROW = 4, LV_WIDE = 8;  // lanes of a short row
+constexpr int LV_WAVE = 512;      // longest row of one wave: 8 entries a lane (1, in list order)
+constexpr int LV_T = 512;         // threads of a level's workgroups: 8 slices or rows, or one hub
+constexpr int LV_WAVES = LV_T / 64;
+constexpr int LV_RUN = 2048;      // largest level of a run: 2 slices per wave of 1024 threads
+constexpr int LV_RUNS = 8;        // shortest run: a level in it takes 2-3 us, after about 15 us to start
+constexpr int LV_MAXLEVELS = 1 << 16;
+constexpr int LV_LATE = 32;       // longest row of a slice of the late lists
+constexpr int LV_WINDOW = 4096;   // where rows are longer, these lists are sorted by length within such windows
+constexpr unsigned LV_PAD = 0x7fffffffu, LV_RECENT = 0x80000000u;
+constexpr int64_t LV_SHORT = (int64_t)1 << 62;  // host: marks a short row's place
+
+struct LevelArgs {
+    const int2 *head;      // late slices: first entry, columns
+    const int *vid;        // vertices of the slices and short rows (-1: none)
+    const unsigned *ids;   // their entries: column id, LV_RECENT, or LV_PAD; a slice's as [column][64], a
+                           // short row's consecutive
+    const float *w;
+    const int4 *row;       // longer rows: vertex, first entry, past the last
+    const unsigned *rids;
+    const float *rw;
+    const int *lstart;     // the run kernel: first slice of each level in its run
+    double W, step;
+    double2 *pos, *rep;
+    double *eterm;
+    const int *status;
+};
+
+// One launch of a level: nn waves of rows of 4 lanes (16 a wave), then nw of rows of 8 (8 a wave),
+// from vertex slot v0 and entry block e0 (64 entries each), then nr rows from row r0, one a wave,
+// then hubs, one a workgroup.
+struct LevelShape {
+    int v0, nn, nw, r0, nr;
+    unsigned e0;
+};
+
+// x_i += (F/|F|) * STEP (:1062-1066), the unit vector F * rsqrt2(|F|^2): the lagged walk's operations.
+__device__ __forceinline__ void move_vertex(const LevelArgs &a, int i, double2 v, double2 f) {
+    const double m2 = f.x * f.x + f.y * f.y;
+    const double r = rsqrt2(m2) * a.step;
+    a.pos[i] = make_double2(fma(f.x, r, v.x), fma(f.y, r, v.y));
+    a.eterm[i] = m2;
+}
+
+// The late term: |d| by the IEEE square root where the graph keeps the lagged walk's sums.
+template <bool IEEE>
+__device__ __forceinline__ void late_add(double2 pj, double2 v, double Wk, double &ax, double &ay) {
+    if constexpr (IEEE) {
+        const double dx = pj.x - v.x, dy = pj.y - v.y;
+        const double sc = Wk * sqrt(dx * dx + dy * dy);
+        ax = fma(dx, sc, ax);
+        ay = fma(dy, sc, ay);
+    } else {
+        attr_add(pj, v, Wk, ax, ay);
+    }
+}
+
+// The sums so far and one more term, kept if `on`.
+__device__ __forceinline__ void add_if(bool on, double2 pj, double2 v, double Wk, double2 &f) {
+    double x = f.x, y = f.y;
+    attr_add(pj, v, Wk, x, y);
+    f.x = on ? x : f.x;
+    f.y = on ? y : f.y;
+}
+
+// Early sum of one vertex: settled entries, then - r at the first recent one (or at the end).
+struct EarlySum {
+    double2 f{0.0, 0.0};
+    bool less = false;
+    __device__ __forceinline__ void subtract(bool on, double2 r) {
+        f.x = on ? f.x - r.x : f.x;
+        f.y = on ? f.y - r.y : f.y;
+        less = less || on;
+    }
+    __device__ __forceinline__ void add(unsigned c, double2 pj, double2 v, double2 r, double Wk) {
+        subtract(c >= LV_RECENT && !less, r);
+        add_if(c != LV_PAD, pj, v, Wk, f);
+    }
+    __device__ __forceinline__ double2 total(double2 r) {
+        subtract(!less, r);
+        return f;
+    }
+};
+
+// N columns of a slice from entry e (the lane's in the first column), of which the first `have`
+// exist (the last again past them), and the positions they name (padding names the own vertex).
+template <bool HAS_W, int N>
+__device__ __forceinline__ void slice_ids(const LevelArgs &a, size_t e, int have, unsigned *c, float *w) {
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+        const size_t k = e + 64 * (size_t)min(g, have - 1);
+        c[g] = g < have ? a.ids[k] : LV_PAD;
+        w[g] = HAS_W ? a.w[k] : 0.0f;
+    }
+}
+template <int N>
+__device__ __forceinline__ void slice_pos(const LevelArgs &a, const unsigned *c, int own, double2 *p) {
+#pragma unroll
+    for (int g = 0; g < N; ++g) p[g] = a.pos[c[g] == LV_PAD ? own : (int)(c[g] & LV_PAD)];
+}
+
+// v of the lane before (row_shr:1; lane 0 of 16 gets 0, which no short row's lane takes).
+__device__ __forceinline__ double lane_before(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x111, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x111, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
+// A wave of short rows, N lanes each: entry block `block`, the rows' vertices from slot vs.  Lane k
+// of a row forms entry k's factors and adds its product to the sum of the lanes before it, in the
+// k-th of N steps; the repulsion is subtracted before the first recent entry, else at the end.
+template <bool HAS_W, int N>
+__device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t block, int bad) {
+    const int lane = threadIdx.x & 63, k = lane & (N - 1);
+    const int id = a.vid[vs + lane / N], i = max(id, 0);
+    const size_t e = block * 64 + lane;
+    const unsigned c = a.ids[e];
+    const double Wk = HAS_W ? a.W * (double)a.w[e] : a.W;
+    const bool real = c != LV_PAD;
+    const double2 v = a.pos[i], r = a.rep[i];
+    const double2 pj = a.pos[real ? (int)(c & LV_PAD) : i];
+    double dx, dy, sc;
+    attr_factors(pj, v, Wk, dx, dy, sc);
+    const unsigned rec = (unsigned)(__ballot(c >= LV_RECENT) >> (lane - k)) & ((1u << N) - 1);
+    const bool first = rec != 0 && (int)__builtin_ctz(rec) == k;
+    const double rx = first ? r.x : 0.0, ry = first ? r.y : 0.0;
+    double2 f = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int g = 0; g < N; ++g) {
+        double px = g > 0 ? lane_before(f.x) : 0.0, py = g > 0 ? lane_before(f.y) : 0.0;
+        px -= rx;
+        py -= ry;
+        const double sx = fma(dx, sc, px), sy = fma(dy, sc, py);
+        if (k == g) f = make_double2(real ? sx : px, real ? sy : py);
+    }
+    if (k != N - 1 || id < 0 || bad) return;
+    if (rec == 0) f = make_double2(f.x - r.x, f.y - r.y);
+    move_vertex(a, i, v, f);
+}
+
+// This thread's share of a row's sum: entries t, t + T, ..., eight loads in flight.
+template <bool HAS_W, int T>
+__device__ __forceinline__ double2 row_share(const LevelArgs &a, int4 row, int t, double2 v) {
+    constexpr int N = 8;
+    double2 f = make_double2(0.0, 0.0);
+    for (int e = row.y + t; e < row.z; e += N * T) {
+        unsigned c[N];
+        double2 p[N];
+        float w[N];
+#pragma unroll
+        for (int g = 0; g < N; ++g) {
+            const int k = min(e + g * T, row.z - 1);
+            c[g] = a.rids[k] & LV_PAD;
+            w[g] = HAS_W ? a.rw[k] : 0.0f;
+        }
+#pragma unroll
+        for (int g = 0; g < N; ++g) p[g] = a.pos[c[g]];
+#pragma unroll
+        for (int g = 0; g < N; ++g)
+            add_if(e + g * T < row.z, p[g], v, HAS_W ? a.W * (double)w[g] : a.W, f);
+    }
+    return f;
+}
+
+__device__ __forceinline__ double lane_of(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// The total force of a row of at most 64 entries with its sums in list order, in every lane: lane
+// k forms the factors of entry k, then the products are added one after another.
+template <bool HAS_W>
+__device__ __forceinline__ double2 row_in_order(const LevelArgs &a, int4 row, int lane, double2 v, double2 r) {
+    const int cnt = row.z - row.y, k = row.y + min(lane, cnt - 1);
+    const unsigned c = a.rids[k];
+    const double Wk = HAS_W ? a.W * (double)a.rw[k] : a.W;
+    const double2 pj = a.pos[c & LV_PAD];
+    double dx, dy, sc;
+    attr_factors(pj, v, Wk, dx, dy, sc);
+    const uint64_t rec = __ballot(c >= LV_RECENT && lane < cnt);
+    const int from = rec ? (int)__builtin_ctzll(rec) : cnt;  // the first recent entry
+    double2 f = make_double2(0.0, 0.0);
+    for (int e = 0; e < cnt; ++e) {
+        if (e == from) f = make_double2(f.x - r.x, f.y - r.y);
+        const double s = lane_of(sc, e);
+        f.x = fma(lane_of(dx, e), s, f.x);
+        f.y = fma(lane_of(dy, e), s, f.y);
+    }
+    return from == cnt ? make_double2(f.x - r.x, f.y - r.y) : f;
+}
+
+// A row's wave or workgroup has its sum f in `one` thread: the late sum, or the move.
+template <bool LATE>
+__device__ __forceinline__ void finish_row(const LevelArgs &a, bool one, int i, double2 v, double2 r, double2 f, int bad) {
+    if (!one || bad) return;
+    if constexpr (LATE)
+        a.rep[i] = make_double2(r.x - f.x, r.y - f.y);
+    else
+        move_vertex(a, i, v, make_double2(f.x - r.x, f.y - r.y));
+}
+
+// Rows by workgroup b past the slices' workgroups: nr rows from row r0 one a wave, then hubs (a
+// fixed order of the sums: per lane, over the wave by DPP, over the waves in turn).
+template <bool HAS_W, bool LATE, bool SEQ>
+__device__ __forceinline__ void long_rows(const LevelArgs &a, int b, int r0, int nr, int bad) {
+    __shared__ double2 red[LV_WAVES];
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int rb = (nr + LV_WAVES - 1) / LV_WAVES;
+    if (b < rb) {
+        const int k = b * LV_WAVES + wave;
+        if (k >= nr) return;
+        const int4 row = a.row[r0 + k];  // wave-uniform
+        const double2 v = a.pos[row.x], r = a.rep[row.x];
+        if constexpr (SEQ) {
+            const double2 f = row_in_order<HAS_W>(a, row, lane, v, r);
+            if (lane == 0 && !bad) move_vertex(a, row.x, v, f);
+            return;
+        }
+        double2 f = row_share<HAS_W, 64>(a, row, lane, v);
+        f.x = wave_sum(f.x);
+        f.y = wave_sum(f.y);
+        finish_row<LATE>(a, lane == 0, row.x, v, r, f, bad);
+        return;
+    }
+    const int4 row = a.row[r0 + nr + b - rb];
+    const double2 v = a.pos[row.x], r = a.rep[row.x];
+    double2 f = row_share<HAS_W, LV_T>(a, row, (int)threadIdx.x, v);
+    f.x = wave_sum(f.x);
+    f.y = wave_sum(f.y);
+    if (lane == 0) red[wave] = f;
+    __syncthreads();
+    f = red[0];
+#pragma unroll
+    for (int k = 1; k < LV_WAVES; ++k) f = add2(f, red[k]);
+    finish_row<LATE>(a, threadIdx.x == 0, row.x, v, r, f, bad);
+}
+
+// One level (SEQ: every row's sum in list order).  The status word is looked at last, so that no
+// load waits for it.
+template <bool HAS_W, bool SEQ>
+__global__ __launch_bounds__(LV_T) void k_level(LevelArgs a, LevelShape q) {
+    const int bad = *a.status;
+    const int nsb = (q.nn + q.nw + LV_WAVES - 1) / LV_WAVES;
+    if ((int)blockIdx.x < nsb) {
+        const int k = __builtin_amdgcn_readfirstlane((int)blockIdx.x * LV_WAVES + ((int)threadIdx.x >> 6));
+        constexpr int RN = 64 / LV_NARROW, RW = 64 / LV_WIDE;  // rows a wave
+        if (k < q.nn)
+            short_rows<HAS_W, LV_NARROW>(a, q.v0 + RN * k, (size_t)q.e0 + k, bad);
+        else if (k < q.nn + q.nw)
+            short_rows<HAS_W, LV_WIDE>(a, q.v0 + RN * q.nn + RW * (k - q.nn), (size_t)q.e0 + k, bad);
+        return;
+    }
+    long_rows<HAS_W, false, SEQ>(a, (int)blockIdx.x - nsb, q.r0, q.nr, bad);
+}
+
+// The late sums of all vertices, folded into the repulsion: ns slices, then the rows.
+template <bool HAS_W, bool IEEE>
+__global__ __launch_bounds__(LV_T) void k_level_late(LevelArgs a, int ns, int nr) {
+    const int bad = *a.status;
+    const int nsb = (ns + LV_WAVES - 1) / LV_WAVES;
+    if ((int)blockIdx.x < nsb) {
+        constexpr int N = 4;
+        const int lane = threadIdx.x & 63;
+        const int s = __builtin_amdgcn_readfirstlane((int)blockIdx.x * LV_WAVES + ((int)threadIdx.x >> 6));
+        if (s >= ns) return;
+        const int2 h = a.head[s];
+        const int id = a.vid[s * 64 + lane], i = max(id, 0);
+        const double2 v = a.pos[i], r = a.rep[i];
+        double ax = 0.0, ay = 0.0;
+        for (int k0 = 0; k0 < h.y; k0 += N) {
+            unsigned c[N];
+            float w[N];
+            double2 p[N];
+            slice_ids<HAS_W, N>(a, (size_t)h.x + 64 * (size_t)k0 + lane, h.y - k0, c, w);
+            slice_pos<N>(a, c, i, p);
+#pragma unroll
+            for (int g = 0; g < N; ++g)
+                if (c[g] != LV_PAD) late_add<IEEE>(p[g], v, HAS_W ? a.W * (double)w[g] : a.W, ax, ay);
+        }
+        if (id >= 0 && !bad) a.rep[i] = make_double2(r.x - ax, r.y - ay);
+        return;
+    }
+    long_rows<HAS_W, true, false>(a, (int)blockIdx.x - nsb, 0, nr, bad);
+}
+
+// Levels [l0, l1) of at most LV_RUN vertices in slices of 8 columns (the run's first vertex slot is
+// v0, its entry block e0), by one workgroup: wave w takes slices w and w + 16 of a level.  What does
+// not change during the walk is loaded ahead, the vertices and entries two levels and the vertex's
+// own position (only its own level moves it) and repulsion one; after the barrier a level is one
+// round trip for its neighbours' positions, the sums and the stores.  The workgroup's waves share
+// one L1, so a barrier after the stores is all the order they need.
+template <bool HAS_W>
+__global__ __launch_bounds__(1024) void k_level_run(LevelArgs a, int l0, int l1, int v0, unsigned e0) {
+    constexpr int PER = LV_RUN / 1024, G = LV_WIDE;
+    if (__builtin_amdgcn_readfirstlane(*a.status)) return;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    struct Slice {
+        int id = -1;
+        unsigned c[G];
+        float w[G];
+    } cur[PER], nxt[PER];
+    double2 v[PER], r[PER];
+    auto entries = [&](int l, Slice *x) {
+        const int b = l < l1 ? a.lstart[l] : 0, e = l < l1 ? a.lstart[l + 1] : 0;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int s = b + wv + 16 * j;
+            x[j].id = -1;
+            if (s < e) {
+                x[j].id = a.vid[v0 + s * 64 + lane];
+                slice_ids<HAS_W, G>(a, ((size_t)e0 + (size_t)G * s) * 64 + lane, G, x[j].c, x[j].w);
+            } else {
+#pragma unroll
+                for (int g = 0; g < G; ++g) x[j].c[g] = LV_PAD, x[j].w[g] = 0.0f;
+            }
+        }
+    };
+    auto own = [&](const Slice *x) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = max(x[j].id, 0);
+            v[j] = a.pos[i];
+            r[j] = a.rep[i];
+        }
+    };
+    entries(l0, cur);
+    own(cur);
+    entries(l0 + 1, nxt);
+    for (int l = l0; l < l1; ++l) {
+        double2 f[PER], vo[PER];
+        int ido[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            ido[j] = cur[j].id;
+            vo[j] = v[j];
+            f[j] = make_double2(0.0, 0.0);
+            if (__builtin_amdgcn_readfirstlane(__ballot(ido[j] >= 0) != 0)) {
+                double2 p[G];
+                slice_pos<G>(a, cur[j].c, max(ido[j], 0), p);
+                EarlySum sum;
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    if (!__ballot(cur[j].c[g] != LV_PAD)) break;  // rows fill the columns in order
+                    sum.add(cur[j].c[g], p[g], v[j], r[j], HAS_W ? a.W * (double)cur[j].w[g] : a.W);
+                }
+                f[j] = sum.total(r[j]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PER; ++j) cur[j] = nxt[j];
+        own(cur);
+        entries(l + 2, nxt);
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (ido[j] >= 0) move_vertex(a, ido[j], vo[j], f[j]);
+        __syncthreads();
+    }
+}
+
+template <class T>
+bool put(DevBuf &d, const std::vector<T> &h) {
+    if (d.ensure(sizeof(T) * std::max<size_t>(h.size(), 64))) return false;
+    return h.empty() || hipMemcpy(d.p, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice) == hipSuccess;
+}
+
+// Slices and longer rows, as on the device.
+struct Lists {
+    std::vector<int2> head;
+    std::vector<int32_t> vid;
+    std::vector<uint32_t> ids, rids;
+    std::vector<float> w, rw;
+    std::vector<int4> row;
+    bool upload(LevelLists &d, bool has_w) const {
+        return put(d.head, head) && put(d.vid, vid) && put(d.ids, ids) && put(d.row, row) && put(d.rids, rids) &&
+               (!has_w || (put(d.w, w) && put(d.rw, rw)));
+    }
+};
+
+}  // namespace
+
+namespace {
+bool build_plan(bl_graph *g, int B, int D) {
+    const int n = g->n;
+    if ((int)g->h_rowptr.size() != n + 1 || (int64_t)g->h_colids.size() != g->nnz) return false;
+    const int32_t *rp = g->h_rowptr.data(), *ci = g->h_colids.data();
+    const float *gw = g->h_w.empty() ? nullptr : g->h_w.data();
+    const std::vector<int32_t> go = D > 0 ? lag_walk_groups(g, B) : std::vector<int32_t>();
+    // levels and numbers of early entries
+    std::vector<int32_t> lev(n), ec(n);
+    int nl = 0;
+    for (int b0 = 0; b0 < n; b0 += B)
+        for (int i = b0; i < std::min(n, b0 + B); ++i) {
+            int top = -1, c = 0;
+            for (int e = rp[i]; e < rp[i + 1]; ++e)
+                if (ci[e] < b0) {
+                    top = std::max(top, lev[ci[e]]);
+                    ++c;
+                }
+            lev[i] = top + 1;
+            ec[i] = c;
+            nl = std::max(nl, top + 2);
+        }
+    if (nl > LV_MAXLEVELS) return false;
+    // within a level: rows for slices of 4 and of 8 columns, rows of a wave, hubs (the lagged walk's
+    // rows, whose sums stay in list order, have at most 64 entries)
+    constexpr int K = 4;
+    if (D > 0 && g->max_row > 64) return false;
+    auto cls = [&](int i) {
+        return (size_t)lev[i] * K + (ec[i] <= LV_NARROW ? 0 : ec[i] <= LV_WIDE ? 1 : ec[i] <= LV_WAVE ? 2 : 3);
+    };
+    std::vector<int32_t> first((size_t)nl * K + 1, 0), order(n);
+    for (int i = 0; i < n; ++i) ++first[cls(i) + 1];
+    for (size_t k = 0; k < (size_t)nl * K; ++k) first[k + 1] += first[k];
+    {
+        std::vector<int32_t> at(first.begin(), first.end() - 1);
+        for (int i = 0; i < n; ++i) order[at[cls(i)]++] = i;
+    }
+    constexpr int64_t cap = ((int64_t)1 << 31) - 1;
+    // Where every vertex's entries go: slot >= 0 the first of its column in a slice (stride 64), < 0
+    // ~ the first of a longer row, or of a short row (marked LV_SHORT).
+    struct Build {
+        Lists L;
+        std::vector<int64_t> slot;
+        int64_t nid = 0, nrid = 0;
+        void slices(const int32_t *vs, int m, int W) {
+            const size_t vat = L.vid.size();
+            L.vid.resize(vat + (size_t)(m + 63) / 64 * 64, -1);
+            for (int t = 0; t < m; ++t) {
+                L.vid[vat + t] = vs[t];
+                slot[vs[t]] = nid + (int64_t)(t >> 6) * W * 64 + (t & 63);
+            }
+            nid += (int64_t)((m + 63) / 64) * W * 64;
+        }
+        // short rows of W lanes, to whole waves; their number of waves
+        int short_rows(const int32_t *vs, int m, int W) {
+            const int per = 64 / W, waves = (m + per - 1) / per;
+            const size_t vat = L.vid.size();
+            L.vid.resize(vat + (size_t)waves * per, -1);
+            for (int t = 0; t < m; ++t) {
+                L.vid[vat + t] = vs[t];
+                slot[vs[t]] = ~((nid + (int64_t)t * W) | LV_SHORT);
+            }
+            nid += (int64_t)waves * 64;
+            return waves;
+        }
+        void row(int i, int len) {
+            slot[i] = ~nrid;
+            L.row.push_back(make_int4(i, (int)nrid, (int)(nrid + len), 0));
+            nrid += len;
+        }
+        void allocate(bool weights) {
+            L.ids.assign((size_t)nid, LV_PAD);
+            L.rids.resize((size_t)nrid);
+            if (weights) L.w.assign((size_t)nid, 0.0f), L.rw.resize((size_t)nrid);
+        }
+        struct Cursor {
+            int64_t at;
+            int stride;
+            bool row;
+        };
+        Cursor at(int i) const {
+            if (slot[i] >= 0) return {slot[i], 64, false};
+            const int64_t k = ~slot[i];
+            return {k & ~LV_SHORT, 1, !(k & LV_SHORT)};
+        }
+        void put(Cursor &c, uint32_t id, const float *gw, int e) {
+            (c.row ? L.rids : L.ids)[c.at] = id;
+            if (gw) (c.row ? L.rw : L.w)[c.at] = gw[e];
+            c.at += c.stride;
+        }
+    } E, L;
+    E.slot.resize(n);
+    L.slot.resize(n);
+    // the levels' launches: on their own, or runs of small levels without longer rows
+    std::vector<int32_t> start;  // of each level of the runs, its first slice in its run, and the run's end
+    auto count = [&](int l, int c) { return first[(size_t)l * K + c + 1] - first[(size_t)l * K + c]; };
+    auto small = [&](int l) { return count(l, 0) + count(l, 1) <= LV_RUN && count(l, 2) + count(l, 3) == 0; };
+    g->lev_launch.clear();
+    g->lev_big = g->lev_small = 0;
+    for (int l = 0; l < nl;) {
+        int e = l;
+        while (e < nl && small(e)) ++e;
+        LevelLaunch q{};
+        q.v0 = (int)E.L.vid.size();
+        q.e0 = (uint32_t)(E.nid / 64);
+        const int32_t *vs = order.data() + first[(size_t)l * K];
+        if (e - l >= LV_RUNS) {
+            q.l0 = (int)start.size();
+            q.l1 = q.l0 + e - l;
+            int at = 0;  // slices of the run
+            for (; l < e; ++l) {
+                const int m = count(l, 0) + count(l, 1);
+                start.push_back(at);
+                E.slices(order.data() + first[(size_t)l * K], m, LV_WIDE);
+                at += (m + 63) / 64;
+            }
+            start.push_back(at);
+            g->lev_small += q.l1 - q.l0;
+        } else {
+            q.nn = E.short_rows(vs, count(l, 0), LV_NARROW);
+            q.nw = E.short_rows(vs + count(l, 0), count(l, 1), LV_WIDE);
+            vs += count(l, 0) + count(l, 1);
+            q.r0 = (int)E.L.row.size();
+            q.nr = count(l, 2);
+            q.nh = count(l, 3);
+            for (int t = 0; t < q.nr + q.nh; ++t) E.row(vs[t], ec[vs[t]]);
+            ++g->lev_big;
+            ++l;
+        }
+        g->lev_launch.push_back(q);
+        if (E.nid > cap * 32 || (int64_t)E.L.vid.size() > cap) return false;
+    }
+    // the late lists: slices in vertex order, sorted by length within windows where rows are long
+    std::vector<int32_t> win, rows, hubs;
+    auto late_len = [&](int i) { return rp[i + 1] - rp[i] - ec[i]; };
+    const bool sorted = g->max_row > LV_LATE;
+    for (int w0 = 0; w0 < n; w0 += LV_WINDOW) {
+        win.clear();
+        for (int i = w0; i < std::min(n, w0 + LV_WINDOW); ++i) {
+            const int c = late_len(i);
+            if (c > LV_WAVE) hubs.push_back(i);
+            else if (c > LV_LATE) rows.push_back(i);
+            else if (c > 0) win.push_back(i);
+        }
+        if (sorted)
+            std::stable_sort(win.begin(), win.end(), [&](int x, int y) { return late_len(x) < late_len(y); });
+        for (size_t t = 0; t < win.size(); t += 64) {
+            const int m = (int)std::min<size_t>(64, win.size() - t);
+            int W = 0;
+            for (int q = 0; q < m; ++q) W = std::max(W, late_len(win[t + q]));
+            L.L.head.push_back(make_int2((int)L.nid, W));
+            L.slices(win.data() + t, m, W);
+        }
+        if (L.nid > cap - 2 * LV_WINDOW * LV_LATE) return false;
+    }
+    for (int i : rows) L.row(i, late_len(i));
+    for (int i : hubs) L.row(i, late_len(i));
+    E.allocate(gw != nullptr);
+    L.allocate(gw != nullptr);
+    for_ranges(n, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i) {
+            const int b0 = (i / B) * B, lim = D > 0 ? go[i] - D : 0;
+            auto early = E.at(i), late = L.at(i);
+            bool recent = false;
+            for (int e = rp[i]; e < rp[i + 1]; ++e) {
+                const int j = ci[e];
+                if (j >= b0) L.put(late, (uint32_t)j, gw, e);
+                else if (D > 0 && go[j] > lim) recent = true;
+                else E.put(early, (uint32_t)j, gw, e);
+            }
+            if (!recent) continue;
+            for (int e = rp[i]; e < rp[i + 1]; ++e)
+                if (ci[e] < b0 && go[ci[e]] > lim) E.put(early, (uint32_t)ci[e] | LV_RECENT, gw, e);
+        }
+    });
+    if (!E.L.upload(g->lev_early, gw) || !L.L.upload(g->lev_late, gw) || !put(g->lev_start, start)) return false;
+    g->lev_late_slices = (int)L.L.head.size();
+    g->lev_late_rows = (int)rows.size();
+    g->lev_late_hubs = (int)hubs.size();
+    return true;
+}
+}  // namespace
+
+// The plan for batches of B vertices (cached per batch size and lag): levels, their slices and
+// hubs, the late lists, and the launches.  D > 0: the sums of the lagged walk with lag D and
+// the groups of lag_walk_groups.  False: too many levels, or lists past 2^31 entries.
+bool level_walk_plan(bl_graph *g, int B, int D) {
+    if (g->lev_batch == B && g->lev_d == D) return g->lev_ok;
+    g->lev_batch = B;
+    g->lev_d = D;
+    try {
+        g->lev_ok = build_plan(g, B, D);
+    } catch (const std::bad_alloc &) {
+        g->lev_ok = false;
+    }
+    return g->lev_ok;
+}
+
+namespace {
+LevelArgs level_args(const bl_graph *g, const LevelLists &d, double2 *pos, const bl_params *p, double step) {
+    LevelArgs a;
+    a.head = d.head.as<int2>();
+    a.vid = d.vid.as<int>();
+    a.ids = d.ids.as<unsigned>();
+    a.w = g->has_w ? d.w.as<float>() : nullptr;
+    a.row = d.row.as<int4>();
+    a.rids = d.rids.as<unsigned>();
+    a.rw = g->has_w ? d.rw.as<float>() : nullptr;
+    a.lstart = g->lev_start.as<int>();
+    a.W = p->weight;
+    a.step = step;
+    a.pos = pos;
+    a.rep = g->bh.rep.as<double2>();
+    a.eterm = g->eterm.as<double>();
+    a.status = g->bh.misc.as<int>();
+    return a;
+}
+int level_blocks(int slices, int rows, int hubs) {
+    return (slices + LV_WAVES - 1) / LV_WAVES + (rows + LV_WAVES - 1) / LV_WAVES + hubs;
+}
+}  // namespace
+
+// The late sums, before any vertex moves.
+int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, hipStream_t s) {
+    const LevelArgs a = level_args(g, g->lev_late, pos, p, 0.0);
+    const int ns = g->lev_late_slices, nr = g->lev_late_rows;
+    const int grid = level_blocks(ns, nr, g->lev_late_hubs);
+    if (grid > 0) {
+        const bool ieee = g->lev_d > 0;
+        auto k = g->has_w ? (ieee ? k_level_late<true, true> : k_level_late<true, false>)
+                          : (ieee ? k_level_late<false, true> : k_level_late<false, false>);
+        hipLaunchKernelGGL(k, dim3(grid), dim3(LV_T), 0, s, a, ns, nr);
+    }
+    BL_HIP(hipGetLastError());
+    return BL_OK;
+}
+
+// One iteration's walk (after launch_level_late).
+int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, double step, hipStream_t s) {
+    const LevelArgs a = level_args(g, g->lev_early, pos, p, step);
+    auto k = g->has_w ? (g->lev_d > 0 ? k_level<true, true> : k_level<true, false>)
+                      : (g->lev_d > 0 ? k_level<false, true> : k_level<false, false>);
+    for (const LevelLaunch &q : g->lev_launch) {
+        if (q.l1 > q.l0)
+            hipLaunchKernelGGL(g->has_w ? k_level_run<true> : k_level_run<false>, dim3(1), dim3(1024), 0, s, a, q.l0,
+                               q.l1, q.v0, q.e0);
+        else
+            hipLaunchKernelGGL(k, dim3(level_blocks(q.nn + q.nw, q.nr, q.nh)), dim3(LV_T), 0, s, a,
+                               LevelShape{q.v0, q.nn, q.nw, q.r0, q.nr, q.e0});
+    }
+    BL_HIP(hipGetLastError());
+    return BL_OK;
+}
+
+}  // namespace bl

@@ -524,6 +524,16 @@ void first_rows(const int32_t *off, int nr, int E, int c, int *out) {
 
 }  // namespace
 
+// Whether the wide walk takes batches of B vertices (a lag of WD_DMIN always fits the ring), and its
+// largest lag.
+bool wide_walk_takes(const bl_graph *g, int B, int *dmax) {
+    *dmax = WD_DMAX;
+    if (const char *v = getenv("BL_WIDE_D")) *dmax = atoi(v);
+    const int n = g->n;
+    return !(B < 64 || B > WD_T || *dmax < WD_DMIN || n < 8 * B || g->nnz <= 0 || g->nnz >= WD_MASK ||
+             (int)g->h_rowptr.size() != n + 1 || (int64_t)g->h_colids.size() != g->nnz);
+}
+
 // The plan of the wide walk for batches of B vertices (cached per batch size and largest lag):
 //   1. the lag D_b of each batch: the largest lag (BL_WIDE_D, default WD_DMAX), reduced where
 //      the ring cannot hold the moved positions the batch reads as near: the vertices a later
@@ -536,16 +546,14 @@ void first_rows(const int32_t *off, int nr, int E, int c, int *out) {
 //      tables, and each exported vertex's slot;
 //   3. far entries (CSR order within a row, settled ones marked), cut into chunks of whole rows.
 bool wide_walk_fits(bl_graph *g, int B) {
-    int dmax = WD_DMAX;
-    if (const char *v = getenv("BL_WIDE_D")) dmax = atoi(v);
+    int dmax;
+    const bool takes = wide_walk_takes(g, B, &dmax);
     if (g->wide_batch == B && g->wide_dmax == dmax) return g->wide_ok;
     g->wide_batch = B;
     g->wide_dmax = dmax;
     g->wide_ok = false;
     const int n = g->n;
-    if (B < 64 || B > WD_T || dmax < WD_DMIN || n < 8 * B || g->nnz <= 0 || g->nnz >= WD_MASK ||
-        (int)g->h_rowptr.size() != n + 1 || (int64_t)g->h_colids.size() != g->nnz)
-        return false;
+    if (!takes) return false;
     const int nb = (n + B - 1) / B;
     const int32_t *rp = g->h_rowptr.data(), *ci = g->h_colids.data();
     const bool hw = !g->h_w.empty();

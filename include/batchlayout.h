@@ -100,8 +100,10 @@ typedef struct {
        [7] unused */
     double kernel_ms[8];
     int32_t kernel_launches[8];
-    /* Barnes-Hut family (algos 4, 6, 40-43): the batch walk of the last iteration, one of BL_WALK_*
-       (0 for the all-pairs algorithms) */
+    /* Barnes-Hut family (algos 4, 6, 40-43): the batch walk that the graph's shape and the batch size
+       select, one of BL_WALK_* (0 for the all-pairs algorithms).  Outside FP64 mode its batches move
+       by dependence levels where these are few (the same layout up to the order of partial sums;
+       for BL_WALK_LAG the same bits); the value names the selected walk either way */
     int32_t walk;
     /* algos 40, 42, 43: cells the far-field traversal accepted in the last iteration (with the
        learned model, the number of model evaluations); 0 otherwise */
@@ -114,7 +116,8 @@ typedef struct {
     /* BL_WALK_LAG: batches of the last iteration whose sums over long-moved neighbours came from the
        helper workgroups (the walker formed the others itself), and the lag D it ran with.
        BL_WALK_WIDE: batches of the last iteration whose helper sums were ready when the walker
-       reached them (it waited for the others), and the largest lag */
+       reached them (it waited for the others), and the largest lag.  By dependence levels no
+       walker forms or waits for a sum: every group or batch counts */
     int32_t walk_helped;
     int32_t walk_lag;
     /* vertices whose final position is not finite (NaN or infinite).  The reference's move
