@@ -56,25 +56,6 @@ struct BatchedArgs {
 
 typedef __attribute__((address_space(3))) const double lds_double;
 
-// Dense repulsion of position pi against positions [j0, j1) of `src` (x, y interleaved, in LDS
-// or global memory; with an LDS-typed pointer the loads are LDS broadcasts instead of generic
-// loads).
-template <bool REFINE, class Src>
-__device__ __forceinline__ void dense_range(Src src, int j0, int j1, double2 pi, double &ax, double &ay) {
-    int u = j0;
-    for (; u + 8 <= j1; u += 8) {  // eight positions in flight per load batch
-        double qx[8], qy[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            qx[k] = src[2 * (u + k)];
-            qy[k] = src[2 * (u + k) + 1];
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) pair_rep<REFINE>(qx[k], qy[k], pi.x, pi.y, ax, ay);
-    }
-    for (; u < j1; ++u) pair_rep<REFINE>(src[2 * u], src[2 * u + 1], pi.x, pi.y, ax, ay);
-}
-
 // Pairwise combination in a fixed tree: leaves arrive left to right, level l holds the pending
 // left subtree of 2^l leaves; after 2^L leaves (L <= 4) level L holds their sum,
 // ((v0 + v1) + (v2 + v3)) + ...  Named registers and uniform branches (the leaf count k is the
@@ -136,11 +117,11 @@ __device__ void layout_graph(const BatchedArgs &a, int g, double2 *P, double2 *r
                 PairTree t;
                 for (int c = js * cpt; c < (js + 1) * cpt; ++c) {  // this subgroup's subtree
                     const int j0 = min(n, c * sub), j1 = min(n, j0 + sub);
-                    double cx = 0.0, cy = 0.0;
+                    double cx, cy;
                     if (in_lds)
-                        dense_range<REFINE>((lds_double *)P, j0, j1, pi, cx, cy);
+                        dense_sum<REFINE, 8>((lds_double *)P, j0, j1, pi.x, pi.y, cx, cy);  // LDS broadcasts
                     else
-                        dense_range<REFINE>(reinterpret_cast<const double *>(gp), j0, j1, pi, cx, cy);
+                        dense_sum<REFINE, 8>(reinterpret_cast<const double *>(gp), j0, j1, pi.x, pi.y, cx, cy);
                     t.add(cx, cy);
                 }
                 red[tid] = t.total(lcpt);

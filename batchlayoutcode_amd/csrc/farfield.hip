@@ -284,7 +284,7 @@ __device__ void far_flush(const MlpLds &L, FarQueue &Q, int count, int lane, uin
 
 // Repulsion F(v) = sum over accepted cells of their far field + sum over the single points met
 // of (p - v)/|p - v|^2.  Opening test and monopole terms are FP64-grade (FP64 differences,
-// FP32-seeded reciprocal with an FP64 Newton step); sums in FP64.
+// reciprocals by one Newton step); sums in FP64.
 template <int MODE>
 __global__ __launch_bounds__(WG) void k_far_trav(const double2 *__restrict__ qpos, const int *__restrict__ qid,
                                                  int nq, const double2 *__restrict__ spos,
@@ -523,13 +523,8 @@ __global__ __launch_bounds__(WG) void k_far_exact(const double2 *__restrict__ qp
     const int k = blockIdx.x * WG + threadIdx.x;
     const double2 p = qpos[k < nq ? k : nq - 1];
     cdouble *cp = (cdouble *)pts;
-    double ax = 0.0, ay = 0.0;
-    int j = 0;
-    for (; j + 8 <= n; j += 8) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) pair_rep<true>(cp[2 * (j + u)], cp[2 * (j + u) + 1], p.x, p.y, ax, ay);
-    }
-    for (; j < n; ++j) pair_rep<true>(cp[2 * j], cp[2 * j + 1], p.x, p.y, ax, ay);
+    double ax, ay;
+    dense_sum<true, 8>(cp, 0, n, p.x, p.y, ax, ay);
     if (k < nq) out[qid ? qid[k] : k] = make_double2(-ax, -ay);  // pair_rep sums -d/|d|^2
 }
 
@@ -624,13 +619,8 @@ __global__ __launch_bounds__(JUDGE_S) void k_judge_exact(const double2 *__restri
     const int j0 = min(n, c * ch), j1 = min(n, j0 + ch);
     const double2 q = J->q[k < S ? k : 0];
     cdbl *cp = (cdbl *)pts;
-    double ax = 0.0, ay = 0.0;
-    int j = j0;
-    for (; j + 8 <= j1; j += 8) {
-#pragma unroll
-        for (int u = 0; u < 8; ++u) pair_rep<true>(cp[2 * (j + u)], cp[2 * (j + u) + 1], q.x, q.y, ax, ay);
-    }
-    for (; j < j1; ++j) pair_rep<true>(cp[2 * j], cp[2 * j + 1], q.x, q.y, ax, ay);
+    double ax, ay;
+    dense_sum<true, 8>(cp, j0, j1, q.x, q.y, ax, ay);
     if (k < S) J->part[c * JUDGE_S + k] = make_double2(ax, ay);
 }
 

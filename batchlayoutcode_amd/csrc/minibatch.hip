@@ -11,9 +11,9 @@
 // where N(i) is the set of column ids the reference's merge pointer meets (:758-762)
 // and A is the attraction law (W|d| d, W d, or log2(1+W|d|) d).
 //
-// FP32 mode (the fast path).  Per pair: the FP64 difference d = x_j - x_i, |d|^2 and
-// 1/|d|^2 in FP32 (v_rcp_f32), and the term -d/|d|^2 accumulated in FP64 (one FMA per
-// component with the FP64 difference).  The dense loop runs over all j; neighbours are not
+// Mixed and FP32 modes (the fast path).  Per pair: the FP64 difference d = x_j - x_i, |d|^2 and
+// 1/|d|^2 (mixed: FP64, one reciprocal for eight pairs; FP32: v_rcp_f32), and the term -d/|d|^2
+// accumulated in FP64 (one FMA per component with the FP64 difference).  The dense loop runs over all j; neighbours are not
 // branched on: a correction adds, in FP64, each neighbour's attraction and removes the
 // repulsion product the dense loop accumulated for it (the same operands, so it cancels).
 //   * k_pairs32 + k_move32 (default): two launches per batch step.  The pair kernel's
@@ -110,14 +110,8 @@ __global__ __launch_bounds__(WG) void k_pairs32(const double2 *__restrict__ pos,
     const int sub = (chunk + JS - 1) / JS;
     const int j0 = min(je, jb + js * sub);
     const int j1 = min(je, j0 + sub);
-    double ax = 0.0, ay = 0.0;
-    int u = j0;
-    for (; u + UNROLL <= j1; u += UNROLL) {
-#pragma unroll
-        for (int k = 0; k < UNROLL; ++k)
-            pair_rep<REFINE>(cpos[2 * (u + k)], cpos[2 * (u + k) + 1], px, py, ax, ay);
-    }
-    for (; u < j1; ++u) pair_rep<REFINE>(cpos[2 * u], cpos[2 * u + 1], px, py, ax, ay);
+    double ax, ay;
+    dense_sum<REFINE, UNROLL>(cpos, j0, j1, px, py, ax, ay);
     if constexpr (JS > 1) {
         red[tid] = make_double2(ax, ay);
         __syncthreads();

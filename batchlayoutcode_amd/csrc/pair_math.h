@@ -3,7 +3,7 @@
 // Reference semantics (sample/algorithms.cpp:758-768): a neighbour j of i contributes the
 // attraction A(d) with d = x_j - x_i; any other j with |d|^2 > 0 contributes -d/|d|^2.
 // The dense loops add -d/|d|^2 for every j (the self pair gives 0); correct_pair() then
-// removes, for each neighbour, exactly the product the dense loop added and adds A(d).
+// removes, for each neighbour, the product the dense loop added and adds A(d).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -13,9 +13,11 @@
 
 namespace bl {
 
-// |d|^2 floor: the self pair and coincident vertices give 0 * (1/kTiny) = 0, as the
-// reference's `dist > 0` test skips them.
+// |d|^2 floors: the self pair and coincident vertices give 0 * (1/floor) = 0, as the
+// reference's `dist > 0` test skips them.  The FP64 floor is below the last bit of |d|^2 for
+// |d| > 1e-22 (1e-30 moved the terms of a layout of extent 1e-7 by 1e-14).
 constexpr float kTiny = 1e-30f;
+constexpr double kTiny64 = 0x1p-200;
 
 // v + the value of the lane CTRL names (a DPP move; lanes without a source lane, or outside
 // ROW_MASK, add +0.0).
@@ -56,15 +58,19 @@ __device__ __forceinline__ void attract64(int law, double W, double dx, double d
     fy += dy * s;
 }
 
-// 1/|d|^2 for a pair with FP64 difference (dx, dy).  REFINE: |d|^2 in FP64, the FP32
-// reciprocal (v_rcp_f32) as seed and one FP64 Newton step (relative error ~1e-14).
-// Otherwise |d|^2 and the reciprocal in FP32 (relative error ~1e-7).
+// 1/x for x > 0: the hardware estimate (relative error about 2^-25) and one Newton step (about
+// 2^-50).
+__device__ __forceinline__ double recip(const double x) {
+    const double s = __builtin_amdgcn_rcp(x);
+    return fma(s, fma(-x, s, 1.0), s);
+}
+
+// 1/|d|^2 for a pair with FP64 difference (dx, dy).  REFINE: FP64 throughout.  Otherwise |d|^2 and
+// the reciprocal in FP32 (relative error ~1e-7).
 template <bool REFINE>
 __device__ __forceinline__ double inv_r2(const double dx, const double dy) {
     if constexpr (REFINE) {
-        const double r2 = fma(dy, dy, fma(dx, dx, (double)kTiny));
-        const double s = (double)__builtin_amdgcn_rcpf((float)r2);
-        return fma(s, fma(-r2, s, 1.0), s);
+        return recip(fma(dy, dy, fma(dx, dx, kTiny64)));
     } else {
         const float fx = (float)dx, fy = (float)dy;
         const float r2 = fmaf(fy, fy, fmaf(fx, fx, kTiny));
@@ -82,8 +88,85 @@ __device__ __forceinline__ void pair_rep(const double qx, const double qy, const
     ay = fma(-dy, inv, ay);
 }
 
-// Neighbour correction for one (i, j) pair: removes the dense loop's product (dx * inv with
-// the same operands) and adds the attraction.
+// 1/r[k] of N (a power of two) values from one reciprocal, that of their product: the product's
+// inverse times the other half's product is a half's inverse, down to single values.
+template <int N>
+__device__ __forceinline__ void recip_all(double *r) {
+    if constexpr (N == 1) {
+        r[0] = recip(r[0]);
+    } else {
+        double h[N / 2];
+#pragma unroll
+        for (int k = 0; k < N / 2; ++k) h[k] = r[2 * k] * r[2 * k + 1];
+        recip_all<N / 2>(h);
+#pragma unroll
+        for (int k = 0; k < N / 2; ++k) {
+            const double a = r[2 * k];
+            r[2 * k] = h[k] * r[2 * k + 1];
+            r[2 * k + 1] = h[k] * a;
+        }
+    }
+}
+
+// N dense repulsion pairs added in order.  What bounds the dense sum is its FP64 operations (a
+// reciprocal takes about four of them): 6 a pair (difference, |d|^2, the two sums) and the
+// reciprocal.  One of its own costs a pair 6 more (REFINE's former seed in FP32: two conversions, the FP32
+// reciprocal, the Newton step); shared by a group of N, 3 products and 6/N.  Measured: the all-pairs step's pair kernel on
+// the 250k random geometric graph 25.6 -> 20.6 us, on the R-MAT graph at -batch 1024 189 -> 162 us.
+// A product past the FP64 range (|d| beyond 1e19 in all of 8 pairs) makes the sum NaN (see
+// dense_sum).
+template <bool REFINE, int N>
+__device__ __forceinline__ void pair_rep_group(const double *qx, const double *qy, const double px, const double py,
+                                               double &ax, double &ay) {
+    if constexpr (REFINE) {
+        double dx[N], dy[N], r[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            dx[k] = qx[k] - px;
+            dy[k] = qy[k] - py;
+            r[k] = fma(dy[k], dy[k], fma(dx[k], dx[k], kTiny64));
+        }
+        recip_all<N>(r);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            ax = fma(-dx[k], r[k], ax);
+            ay = fma(-dy[k], r[k], ay);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < N; ++k) pair_rep<false>(qx[k], qy[k], px, py, ax, ay);
+    }
+}
+
+// The dense repulsion of position (px, py) against positions [j0, j1) of src (x, y interleaved),
+// U positions loaded at a time, in (ax, ay).  A sum that is not finite is formed again pair by
+// pair: a group's product may have left the FP64 range where no single |d|^2 does.
+template <bool REFINE, int U, class Src>
+__device__ __forceinline__ void dense_sum(Src src, const int j0, const int j1, const double px, const double py,
+                                          double &ax, double &ay) {
+    constexpr int N = 8;  // pairs that share a reciprocal
+    static_assert(U % N == 0, "whole groups");
+    ax = ay = 0.0;
+    int j = j0;
+    for (; j + U <= j1; j += U) {
+        double qx[U], qy[U];
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            qx[k] = src[2 * (j + k)];
+            qy[k] = src[2 * (j + k) + 1];
+        }
+#pragma unroll
+        for (int k = 0; k < U; k += N) pair_rep_group<REFINE, N>(qx + k, qy + k, px, py, ax, ay);
+    }
+    for (; j < j1; ++j) pair_rep<REFINE>(src[2 * j], src[2 * j + 1], px, py, ax, ay);
+    if (REFINE && !(isfinite(ax) && isfinite(ay))) {
+        ax = ay = 0.0;
+        for (j = j0; j < j1; ++j) pair_rep<REFINE>(src[2 * j], src[2 * j + 1], px, py, ax, ay);
+    }
+}
+
+// Neighbour correction for one (i, j) pair: removes the dense loop's product (dx * inv; with REFINE
+// to its last bits, of the order of the dense sum's own rounding) and adds the attraction.
 template <bool REFINE>
 __device__ __forceinline__ void correct_pair(int law, double W, double dx, double dy, double &cx, double &cy) {
     const double inv = inv_r2<REFINE>(dx, dy);
