@@ -41,10 +41,10 @@
 #include <string.h>
 
 #include <algorithm>
-#include <type_traits>
 #include <vector>
 
 #include "bh_common.h"
+#include "traverse.h"
 
 namespace bl {
 
@@ -754,32 +754,108 @@ struct Frame {
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Unit vector d/|d| added to (fx, fy).  REFINE (the default precision): FP64 difference, the
-// FP32 reciprocal square root refined by one FP64 Newton step (relative error ~1e-14) and an
-// FP64 sum.  Otherwise (BL_PREC_FP32) all in FP32.  Over hundreds of iterations the FP32
-// terms bias the layout: the 600-iteration energy on the 64x64 grid ends several percent
-// below the reference's, while the refined terms agree with it.
-template <bool REFINE>
-struct UnitSum {
-    typename std::conditional<REFINE, double, float>::type x = 0, y = 0;
-    __device__ __forceinline__ void add(double dx, double dy) {
-        if constexpr (REFINE) {
-            const double r2 = fma(dy, dy, dx * dx);
-            double q = (double)__builtin_amdgcn_rsqf((float)r2);
-            q = q * fma(-0.5 * r2 * q, q, 1.5);
-            x = fma(dx, q, x);
-            y = fma(dy, q, y);
-        } else {
-            const float fx = (float)dx, fy = (float)dy;
-            const float inv = __builtin_amdgcn_rsqf(fmaf(fy, fy, fx * fx));
-            x = fmaf(fx, inv, x);
-            y = fmaf(fy, inv, y);
+// Mixed mode (the default).  One wave per 64 Morton-consecutive vertices and one stack of nodes
+// (traverse.h).  The opening test D/|c - v| < theta (BarnesHut.h:71-72) is decided by the squares,
+// except within 2^-40 of equality, where the caller evaluates it as it stands for the whole node, so
+// the accepted set is the reference's.  Unit vectors d/|d| by the FP32 reciprocal square root refined
+// by one FP64 Newton step (relative error ~1e-14), sums in FP64: over hundreds of iterations FP32
+// terms bias the layout (the 600-iteration energy on the 64x64 grid ends several percent below the
+// reference's).  143 -> 97 us on the 250k random geometric graph, 253 -> 184 us on the R-MAT graph of
+// scale 20 (theta 1.2), with the sums of the C++ loop before it bit for bit.
+__global__ __launch_bounds__(WG) void k_rep(const double2 *__restrict__ qpos, const int *__restrict__ qid, int n,
+                                            const double2 *__restrict__ spos, const BHNode *__restrict__ nodes,
+                                            const int *__restrict__ misc, const double *__restrict__ frame,
+                                            double theta, double2 *__restrict__ rep, const int *__restrict__ status) {
+    if (*status) return;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int k = (xcd_tile(blockIdx.x, gridDim.x) * (WG / 64) + w) * 64 + lane;
+    const bool valid = k < n;
+    const uint64_t m0 = __ballot(valid);
+    if (m0 == 0) return;
+    const int root = misc[1];
+    if (root < 0) {  // single vertex: no other point, no force
+        if (valid) rep[qid[k]] = make_double2(0.0, 0.0);
+        return;
+    }
+    const double2 p = qpos[valid ? k : n - 1];
+    const double maxmin = frame[2], open = theta / maxmin;
+    const double open_lo = scalar(open * open * (1.0 - 0x1p-40)), open_hi = scalar(open * open * (1.0 + 0x1p-40));
+    double fx = 0.0, fy = 0.0;
+    __shared__ int save[WG / 64][3 * WAVE_STACK_SAVE];
+    WaveStack stk(lane, save[w], root, m0);
+    for (;;) {
+        int why, v, mlo, mhi, sp = scalar(stk.sp);
+        double dx, dy, r2, sv, t;
+        float q32;
+        __asm__ volatile(
+            BL_TRAV_POP
+            // BHNode: c in s[64:67], ch in s[68:71], depth in s75
+            "s_mul_i32 s82, s80, 48\n\t"
+            "s_mul_hi_u32 s83, s80, 48\n\t"
+            "s_add_u32 s82, s82, %[nodes0]\n\t"
+            "s_addc_u32 s83, s83, %[nodes1]\n\t"
+            "s_load_dwordx8 s[64:71], s[82:83], 0\n\t"
+            "s_load_dword s75, s[82:83], 32\n\t"
+            "s_waitcnt lgkmcnt(0)\n\t" BL_TRAV_DIST BL_TRAV_TEST("%[open_lo]")
+            "s_cbranch_scc0 Ltake%=\n\t"
+            "v_mul_f64 %[t], %[open_hi], %[r2]\n\t"
+            "v_cmp_lt_f64 vcc, s[90:91], %[t]\n\t"
+            "s_and_b64 vcc, vcc, s[88:89]\n\t"
+            "s_cbranch_scc1 Lnear%=\n"
+            "Ltake%=:\n\t"
+            BL_TRAV_TAKE(BL_TRAV_RSQRT BL_TRAV_ADD)
+            BL_TRAV_OPEN("s68", "s69", "s70", "s71", BL_TRAV_RSQRT BL_TRAV_ADD)
+            "Lnear%=:\n\t"
+            "s_mov_b32 %[why], 2\n"
+            "Lout%=:\n\t"
+            "s_mov_b32 %[v], s80\n\t"
+            "s_mov_b32 %[mlo], s84\n\t"
+            "s_mov_b32 %[mhi], s85"
+            : [node] "+v"(stk.node), [lo] "+v"(stk.lo), [hi] "+v"(stk.hi), [sp] "+s"(sp), [fx] "+v"(fx),
+              [fy] "+v"(fy), [why] "=&s"(why), [v] "=&s"(v), [mlo] "=&s"(mlo), [mhi] "=&s"(mhi), [dx] "=&v"(dx),
+              [dy] "=&v"(dy), [r2] "=&v"(r2), [s] "=&v"(sv), [t] "=&v"(t), [q] "=&v"(q32)
+            : [px] "v"(p.x), [py] "v"(p.y), [open_lo] "s"(open_lo), [open_hi] "s"(open_hi), [c15] "s"(1.5),
+              [nodes0] "s"((int)(uint64_t)nodes), [nodes1] "s"((int)((uint64_t)nodes >> 32)),
+              [spos0] "s"((int)(uint64_t)spos), [spos1] "s"((int)((uint64_t)spos >> 32))
+            : BL_TRAV_CLOBBERS);
+        stk.sp = sp;
+        why = scalar(why);
+        if (why == TRAV_FULL) {
+            stk.put_away();
+        } else if (why == TRAV_NEAR) {  // the test as it stands, for the whole node
+            const BHNode &nd = nodes[scalar(v)];
+            const uint64_t m = ((uint64_t)(unsigned)mhi << 32) | (unsigned)mlo;
+            const double ex = nd.c.x - p.x, ey = nd.c.y - p.y;
+            const double D = ldexp(maxmin, -nd.depth);
+            const uint64_t take = m & __ballot(D / sqrt(ex * ex + ey * ey) < theta);
+            auto add = [&](double x, double y) {
+                const double d2 = fma(y, y, x * x);
+                double q = (double)__builtin_amdgcn_rsqf((float)d2);
+                q = q * fma(-0.5 * d2 * q, q, 1.5);
+                fx = fma(x, q, fx);
+                fy = fma(y, q, fy);
+            };
+            if ((take >> lane) & 1ull) add(ex, ey);
+            const uint64_t rej = m & ~take;
+            if (rej) {
+                const int c[4] = {nd.ch.x, nd.ch.y, nd.ch.z, nd.ch.w};
+                for (int j = 3; j >= 0; --j) {
+                    if (c[j] > -2 || !((rej >> lane) & 1ull)) continue;
+                    const double2 l = spos[-c[j] - 2];
+                    if (l.x != p.x || l.y != p.y) add(l.x - p.x, l.y - p.y);
+                }
+                stk.push_children(nd.ch, rej);
+            }
+        } else if (!stk.more()) {
+            break;
         }
     }
-};
+    if (valid) rep[qid[k]] = make_double2(fx, fy);
+}
 
-// FP32 / mixed modes.  One wave per 64 Morton-consecutive vertices; shared stack of (node, mask).
-template <bool REFINE>
+// FP32 mode: unit vectors in FP32 and summed in FP32, in this order.  One wave per 64
+// Morton-consecutive vertices; shared stack of (node, mask).  The opening test runs in FP32 with a
+// guard band; the cases inside it are decided in FP64.
 __global__ __launch_bounds__(WG) void k_rep32(const double2 *__restrict__ qpos, const int *__restrict__ qid, int n,
                                               const double2 *__restrict__ spos,
                                               const BHNode *__restrict__ nodes, const int *__restrict__ misc,
@@ -795,7 +871,13 @@ __global__ __launch_bounds__(WG) void k_rep32(const double2 *__restrict__ qpos, 
     const double maxmin = frame[2];
     const float th2 = (float)(theta * theta);
     const float lo_band = 1.0f - 1.0f / 4096.0f, hi_band = 1.0f + 1.0f / 4096.0f;
-    UnitSum<REFINE> f;
+    float sx = 0.0f, sy = 0.0f;
+    auto add = [&](double dx, double dy) {
+        const float fx = (float)dx, fy = (float)dy;
+        const float inv = __builtin_amdgcn_rsqf(fmaf(fy, fy, fx * fx));
+        sx = fmaf(fx, inv, sx);
+        sy = fmaf(fy, inv, sy);
+    };
     const int root = misc[1];
     int sp = 0;
     uint64_t m0 = __ballot(valid);
@@ -827,7 +909,7 @@ __global__ __launch_bounds__(WG) void k_rep32(const double2 *__restrict__ qpos, 
         if (a < b * lo_band) acc = true;
         else if (a > b * hi_band) acc = false;
         else acc = D / sqrt(dx64 * dx64 + dy64 * dy64) < theta;  // exact FP64 test, :71-72
-        if (act && acc) f.add(dx64, dy64);
+        if (act && acc) add(dx64, dy64);
         const uint64_t rej = __ballot(act && !acc);
         if (rej) {
             const int c[4] = {nd.ch.x, nd.ch.y, nd.ch.z, nd.ch.w};
@@ -843,14 +925,14 @@ __global__ __launch_bounds__(WG) void k_rep32(const double2 *__restrict__ qpos, 
                     if ((rej >> lane) & 1ull) {  // leaf, :78-83
                         const double2 l = spos[-c[q] - 2];
                         const double lx = l.x - p.x, ly = l.y - p.y;
-                        if (lx * lx + ly * ly > 0.0) f.add(lx, ly);
+                        if (lx * lx + ly * ly > 0.0) add(lx, ly);
                     }
                 }
             }
             __builtin_amdgcn_wave_barrier();
         }
     }
-    if (valid) rep[qid[k]] = make_double2((double)f.x, (double)f.y);
+    if (valid) rep[qid[k]] = make_double2((double)sx, (double)sy);
 }
 
 // FP64 mode: the reference's depth-first order (quadrants 0..3, leaves in place) and its
@@ -2089,7 +2171,7 @@ int launch_rep(BHWork &w, int n, double theta, int precision, hipStream_t s) {
                            w.spos.as<double2>(), w.node_child.as<BHNode>(), w.misc.as<int>(), w.frame.as<double>(), theta,
                            w.rep.as<double2>(), w.misc.as<int>());
     else
-        hipLaunchKernelGGL(precision == BL_PREC_FP32 ? k_rep32<false> : k_rep32<true>, dim3(g), dim3(WG), 0, s,
+        hipLaunchKernelGGL(precision == BL_PREC_FP32 ? k_rep32 : k_rep, dim3(g), dim3(WG), 0, s,
                            w.spos.as<double2>(), w.idx_a.as<int>(), n, w.spos.as<double2>(), w.node_child.as<BHNode>(),
                            w.misc.as<int>(), w.frame.as<double>(), theta, w.rep.as<double2>(), w.misc.as<int>());
     BL_HIP(hipGetLastError());
@@ -2546,7 +2628,7 @@ int bh_forces_host(int32_t n, const double *xy, double theta, int32_t nq, const 
         hipLaunchKernelGGL(k_rep64, dim3(gq), dim3(WG), 0, sc.s, dq, qid, nq, w.spos.as<double2>(), w.node_child.as<BHNode>(),
                            w.misc.as<int>(), w.frame.as<double>(), theta, dout, w.misc.as<int>());
     else
-        hipLaunchKernelGGL(precision == BL_PREC_FP32 ? k_rep32<false> : k_rep32<true>, dim3(gq), dim3(WG), 0, sc.s, dq,
+        hipLaunchKernelGGL(precision == BL_PREC_FP32 ? k_rep32 : k_rep, dim3(gq), dim3(WG), 0, sc.s, dq,
                            qid, nq, w.spos.as<double2>(), w.node_child.as<BHNode>(), w.misc.as<int>(),
                            w.frame.as<double>(), theta, dout, w.misc.as<int>());
     BL_HIP(hipGetLastError());
