@@ -138,10 +138,38 @@ __device__ __forceinline__ void pair_rep_group(const double *qx, const double *q
     }
 }
 
+// The positions [j, j1) past the last whole group of N, added in order.  REFINE: one more group, filled
+// up with pairs of distance 0 and |d|^2 = 1 (a serial chain of reciprocals took 5 us of a batch step).
+template <bool REFINE, int N, class Src>
+__device__ __forceinline__ void dense_tail(Src src, const int j, const int j1, const double px, const double py,
+                                           double &ax, double &ay) {
+    if constexpr (REFINE) {
+        double dx[N], dy[N], r[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int q = min(j + k, j1 - 1);
+            const double qx = src[2 * q], qy = src[2 * q + 1];
+            const bool in = j + k < j1;
+            dx[k] = in ? qx - px : 0.0;
+            dy[k] = in ? qy - py : 0.0;
+            r[k] = in ? fma(dy[k], dy[k], fma(dx[k], dx[k], kTiny64)) : 1.0;
+        }
+        recip_all<N>(r);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            ax = fma(-dx[k], r[k], ax);
+            ay = fma(-dy[k], r[k], ay);
+        }
+    } else {
+        for (int k = j; k < j1; ++k) pair_rep<false>(src[2 * k], src[2 * k + 1], px, py, ax, ay);
+    }
+}
+
 // The dense repulsion of position (px, py) against positions [j0, j1) of src (x, y interleaved),
 // U positions loaded at a time, in (ax, ay).  A sum that is not finite is formed again pair by
 // pair: a group's product may have left the FP64 range where no single |d|^2 does.
-template <bool REFINE, int U, class Src>
+// PAD: the positions past the last whole group by dense_tail (for short ranges; otherwise one by one, in less code).
+template <bool REFINE, int U, bool PAD = false, class Src>
 __device__ __forceinline__ void dense_sum(Src src, const int j0, const int j1, const double px, const double py,
                                           double &ax, double &ay) {
     constexpr int N = 8;  // pairs that share a reciprocal
@@ -157,6 +185,10 @@ __device__ __forceinline__ void dense_sum(Src src, const int j0, const int j1, c
         }
 #pragma unroll
         for (int k = 0; k < U; k += N) pair_rep_group<REFINE, N>(qx + k, qy + k, px, py, ax, ay);
+    }
+    if constexpr (PAD) {
+        if (j < j1) dense_tail<REFINE, N>(src, j, j1, px, py, ax, ay);
+        j = j1;
     }
     for (; j < j1; ++j) pair_rep<REFINE>(src[2 * j], src[2 * j + 1], px, py, ax, ay);
     if (REFINE && !(isfinite(ax) && isfinite(ay))) {
