@@ -126,44 +126,91 @@ __global__ __launch_bounds__(WG) void k_pairs32(const double2 *__restrict__ pos,
     if (js == 0 && slot < bc) part[(size_t)slot * P + blockIdx.x] = make_double2(ax, ay);
 }
 
-// FP64 reference-order pair kernel.  grid = (ceil(n/512), rows); block x covers the
-// reference's j block [512x, 512x+512), one lane per batch vertex.
-__global__ __launch_bounds__(WG) void k_pairs64(const double2 *__restrict__ pos, int n, int b0, int bc,
-                                                double2 *__restrict__ part, int P, const int *__restrict__ erp,
-                                                const int *__restrict__ eci, const float *__restrict__ ew,
-                                                double W, int law) {
-    const int slot = (int)blockIdx.y * WG + threadIdx.x;
-    if (slot >= bc) return;
-    const int i = b0 + slot;
-    const int jb = (int)blockIdx.x * kBlockY;
-    const int je = min(n, jb + kBlockY);
-    const double vx = pos[i].x, vy = pos[i].y;
-    int lo = erp[i], hi = erp[i + 1];
-    const int kend = hi;
-    while (lo < hi) {  // first neighbour >= jb (the merge pointer's state at the block start)
-        const int m = (lo + hi) >> 1;
-        if (eci[m] < jb) lo = m + 1; else hi = m;
-    }
-    int k = lo;
-    int nb = k < kend ? eci[k] : -1;
-    double fx = 0.0, fy = 0.0;
-    for (int u = jb; u < je; ++u) {
-        const double2 q = pos[u];
-        const double dx = q.x - vx, dy = q.y - vy;
-        if (u == nb) {  // :758-762
-            attract64(law, ew ? W * (double)ew[k] : W, dx, dy, fx, fy);
-            ++k;
-            nb = k < kend ? eci[k] : -1;
-        } else {  // :764-768
-            const double dist = dx * dx + dy * dy;
-            if (dist > 0) {
-                const double inv = 1.0 / dist;
-                fx = fx - dx * inv;
-                fy = fy - dy * inv;
+// FP64 reference-order pair kernel.  grid = (ceil(n/512), rows of 16 batch vertices, in y and z);
+// block x covers the reference's j block [512x, 512x+512) for a row.
+//
+// A block's partial is a chain of 512 additions in j order, but the terms don't depend on the chain:
+// four waves form the terms of a tile of 64 positions (IEEE division, or the attraction at a
+// neighbour) in LDS while the fifth adds the tile before, a lane per vertex and component.  A pair
+// that adds nothing has the term 0, which leaves a sum that began with +0 as it is.  The neighbours
+// met in the block are bits in LDS, found once.  With one lane a vertex for both (division on the chain,
+// 20 workgroups for 10k vertices) a batch step of 10,007 vertices took 82 us, now 14 (18 with tiles of
+// 128); the chain is 2 of them.
+constexpr int SLOTS64 = 16, TILE64 = 64, ROWS64 = 32768;  // slots a row, positions a tile, rows in y
+
+__global__ __launch_bounds__(64 + WG) void k_pairs64(const double2 *__restrict__ pos, int n, int b0, int bc,
+                                                     double2 *__restrict__ part, int P, const int *__restrict__ erp,
+                                                     const int *__restrict__ eci, const float *__restrict__ ew,
+                                                     double W, int law) {
+    __shared__ double2 q[kBlockY];
+    __shared__ double2 term[2][TILE64][SLOTS64];
+    __shared__ unsigned met[SLOTS64][kBlockY / 32];  // bit u - jb: column u is a neighbour
+    __shared__ int first[SLOTS64];                   // the block's first neighbour entry
+    const int tid = threadIdx.x;
+    const int jb = (int)blockIdx.x * kBlockY, nj = min(n, jb + kBlockY) - jb;
+    const int s0 = ((int)blockIdx.z * ROWS64 + (int)blockIdx.y) * SLOTS64;
+    if (s0 >= bc) return;
+    for (int u = tid; u < kBlockY; u += 64 + WG) q[u] = pos[jb + min(u, nj - 1)];
+    for (int k = tid; k < SLOTS64 * (kBlockY / 32); k += 64 + WG) (&met[0][0])[k] = 0;
+    if (tid < SLOTS64) first[tid] = 0x7fffffff;
+    __syncthreads();
+    const int w = tid - 64;  // a producer's number
+    const int slot = w & (SLOTS64 - 1), jl = w >> 4;
+    const int i = b0 + min(s0 + (slot & (SLOTS64 - 1)), bc - 1);
+    double2 v = make_double2(0.0, 0.0);
+    if (w >= 0) {
+        v = pos[i];
+        const int kend = erp[i + 1];
+        int lo = erp[i], hi = kend;
+        while (hi - lo > 64) {  // first neighbour >= jb (the merge pointer's state at the block start): in [lo, hi]
+            const int m = (lo + hi) >> 1;
+            if (eci[m] < jb) lo = m + 1; else hi = m;
+        }
+        for (int e = lo + jl; e < kend; e += WG / SLOTS64) {
+            const int c = eci[e] - jb;
+            if (c >= nj) break;
+            if (c >= 0) {
+                atomicOr(&met[slot][c >> 5], 1u << (c & 31));
+                atomicMin(&first[slot], e);
             }
         }
     }
-    part[(size_t)slot * P + blockIdx.x] = make_double2(fx, fy);
+    __syncthreads();
+    const int tiles = (nj + TILE64 - 1) / TILE64;
+    double f = 0.0;
+    for (int t = 0; t <= tiles; ++t) {
+        if (w >= 0) {
+            if (t < tiles) {
+                unsigned near = 0;  // neighbours among this thread's positions: one copy of their code, after
+#pragma unroll
+                for (int k = 0; k < TILE64; k += WG / SLOTS64) {  // :764-768
+                    const int u = t * TILE64 + k + jl;
+                    const double2 p = q[u];
+                    const double dx = p.x - v.x, dy = p.y - v.y;
+                    const double dist = dx * dx + dy * dy;
+                    const double inv = 1.0 / dist;
+                    const bool in = u < nj && dist > 0;
+                    term[t & 1][k + jl][slot] = make_double2(in ? -(dx * inv) : 0.0, in ? -(dy * inv) : 0.0);
+                    near |= (met[slot][u >> 5] >> (u & 31) & 1) << (k / (WG / SLOTS64));
+                }
+                for (; near; near &= near - 1) {  // :758-762
+                    const int k = __ffs(near) - 1, u = t * TILE64 + k * (WG / SLOTS64) + jl;
+                    int e = first[slot] + __popc(met[slot][u >> 5] & ((1u << (u & 31)) - 1));
+                    for (int r = 0; r < u >> 5; ++r) e += __popc(met[slot][r]);
+                    double tx = 0.0, ty = 0.0;
+                    attract64(law, ew ? W * (double)ew[e] : W, q[u].x - v.x, q[u].y - v.y, tx, ty);
+                    term[t & 1][k * (WG / SLOTS64) + jl][slot] = make_double2(tx, ty);
+                }
+            }
+        } else if (t > 0) {
+            const double *col = &term[(t - 1) & 1][0][0].x + (tid & (2 * SLOTS64 - 1));
+#pragma unroll 16
+            for (int k = 0; k < TILE64; ++k) f += col[2 * SLOTS64 * k];
+        }
+        __syncthreads();
+    }
+    if (tid < 2 * SLOTS64 && s0 + tid / 2 < bc)
+        (&part[(size_t)(s0 + tid / 2) * P + blockIdx.x].x)[tid & 1] = f;
 }
 
 // FP32 path: one workgroup per batch vertex sums its G chunk partials and its correction
@@ -206,19 +253,18 @@ __global__ __launch_bounds__(WG) void k_move32(const double2 *__restrict__ part,
     }
 }
 
-// FP64 mode: prevCoordinates[i] += f per j block in block order (:771), then the move.
-__global__ __launch_bounds__(WG) void k_move64(const double2 *__restrict__ part, int P, double2 *__restrict__ pos,
+// FP64 mode: prevCoordinates[i] += f per j block in block order (:771), then the move.  A lane per
+// vertex and component, eight partials loaded at a time.
+__global__ __launch_bounds__(64) void k_move64(const double2 *__restrict__ part, int P, double2 *__restrict__ pos,
                                                int b0, int bc, const double *__restrict__ stepp,
                                                double *__restrict__ eterm) {
-    const int slot = (int)blockIdx.x * WG + threadIdx.x;
-    if (slot >= bc) return;
-    const double2 *row = part + (size_t)slot * P;
-    double sx = 0.0, sy = 0.0;
-    for (int p = 0; p < P; ++p) {
-        sx += row[p].x;
-        sy += row[p].y;
-    }
-    move_one(pos, b0 + slot, sx, sy, *stepp, eterm);
+    const int slot = (int)blockIdx.x * 32 + threadIdx.x / 2, c = threadIdx.x & 1;
+    const double *row = &part[(size_t)min(slot, bc - 1) * P].x + c;
+    double s = 0.0;
+#pragma unroll 8
+    for (int p = 0; p < P; ++p) s += row[2 * p];
+    const double other = __shfl_xor(s, 1);
+    if (slot < bc && c == 0) move_one(pos, b0 + slot, s, other, *stepp, eterm);
 }
 
 // STEP lives on the device so that one iteration's launches are the same every iteration (and
@@ -290,18 +336,47 @@ __global__ __launch_bounds__(64) void k_energy_final(double *out) {
     if (threadIdx.x == 0) out[0] = a;
 }
 
-// Sequential sum in vertex order, ENERGY += |F_i|^2 as the reference (FP64 mode).
-__global__ void k_energy_seq(const double *__restrict__ eterm, int n, double *out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Sequential sum in vertex order, ENERGY += |F_i|^2 as the reference (FP64 mode): one wave adds a
+// tile from LDS while the others load the next, so that the chain of additions is what takes the time
+// (10,007 terms: 50 us, 11 cycles a term; 362 with one thread loading each term).
+constexpr int SEQ_TILE = 1536;  // 8 loads a thread of three waves
+__global__ __launch_bounds__(256) void k_energy_seq(const double *__restrict__ eterm, int n, double *out) {
+    __shared__ double buf[2][SEQ_TILE];
+    const int w = (int)threadIdx.x - 64;
+    const int tiles = (n + SEQ_TILE - 1) / SEQ_TILE;
     double e = 0.0;
-    for (int i = 0; i < n; ++i) e += eterm[i];
-    *out = e;
+    for (int t = 0; t <= tiles; ++t) {
+        if (w >= 0) {
+#pragma unroll
+            for (int k = 0; k < SEQ_TILE / 192; ++k) {
+                const int i = t * SEQ_TILE + 192 * k + w;
+                buf[t & 1][192 * k + w] = i < n ? eterm[i] : 0.0;  // |F|^2 >= 0: adding 0 changes nothing
+            }
+        } else if (t > 0) {
+            const double *col = buf[(t - 1) & 1];
+            double a[16], b[16];  // read one group while the other is added
+#pragma unroll
+            for (int k = 0; k < 16; ++k) a[k] = col[k];
+            for (int g = 0; g < SEQ_TILE; g += 32) {
+#pragma unroll
+                for (int k = 0; k < 16; ++k) b[k] = col[g + 16 + k];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) e += a[k];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) a[k] = col[min(g + 32, SEQ_TILE - 16) + k];
+#pragma unroll
+                for (int k = 0; k < 16; ++k) e += b[k];
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = e;
 }
 
 // out: 4 + ENERGY_PARTS doubles (the sum in out[0])
 int launch_energy(const double *eterm, int n, double *out, int precision, hipStream_t s) {
     if (precision == BL_PREC_FP64)
-        hipLaunchKernelGGL(k_energy_seq, dim3(1), dim3(64), 0, s, eterm, n, out);
+        hipLaunchKernelGGL(k_energy_seq, dim3(1), dim3(256), 0, s, eterm, n, out);
     else {
         hipLaunchKernelGGL(k_energy_part, dim3(ENERGY_PARTS), dim3(256), 0, s, eterm, n, out);
         hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(64), 0, s, out);
@@ -413,11 +488,13 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
             const int bc = (n - b0) < B ? (n - b0) : B;
             if (fp64) {
                 prof.begin(0);
-                hipLaunchKernelGGL(k_pairs64, dim3(G, (bc + WG - 1) / WG), dim3(WG), 0, s, pos, n, b0, bc, part, P,
+                const int rows = (bc + SLOTS64 - 1) / SLOTS64;
+                hipLaunchKernelGGL(k_pairs64, dim3(G, std::min(rows, ROWS64), (rows + ROWS64 - 1) / ROWS64),
+                                   dim3(64 + WG), 0, s, pos, n, b0, bc, part, P,
                                    erp, eci, ew, p->weight, law);
                 prof.end();
                 prof.begin(1);
-                hipLaunchKernelGGL(k_move64, dim3((bc + WG - 1) / WG), dim3(WG), 0, s, part, P, pos, b0, bc, d_step,
+                hipLaunchKernelGGL(k_move64, dim3((bc + 31) / 32), dim3(64), 0, s, part, P, pos, b0, bc, d_step,
                                    eterm);
                 prof.end();
             } else {
