@@ -16,7 +16,8 @@
 // accumulated in FP64 (one FMA per component with the FP64 difference).  The dense loop runs over all j; neighbours are not
 // branched on: a correction adds, in FP64, each neighbour's attraction and removes the
 // repulsion product the dense loop accumulated for it (the same operands, so it cancels).
-//   * k_pairs32 + k_move32 (default): two launches per batch step.  The pair kernel's
+//   * k_step32 (small graphs): one launch per batch step, a workgroup per batch vertex.
+//   * k_pairs32 + k_move32: two launches per batch step.  The pair kernel's
 //     chunk workgroups write each batch vertex's chunk partials; its correction waves take
 //     the neighbour corrections in pieces of at most CORR_PIECE entries (a hub's
 //     correction is spread over many waves); k_move32 adds them in a fixed order and moves.
@@ -126,6 +127,51 @@ __global__ __launch_bounds__(WG) void k_pairs32(const double2 *__restrict__ pos,
     if (js == 0 && slot < bc) part[(size_t)slot * P + blockIdx.x] = make_double2(ax, ay);
 }
 
+// A whole batch step in one launch, a workgroup of NT threads per batch vertex: the dense sum (thread
+// t takes positions t, t + NT, ...), the corrections, the move.  No partial leaves the workgroup, so
+// the second launch and its loads go; every vertex's workgroup reads all positions itself.  The
+// positions are in two arrays: a step reads src, which holds every move before it, and writes dst,
+// which lacks the previous batch's (p0, pc) and gets them copied with this batch's.  What bounds a step
+// is the launch and two dependent loads (3.8 us); figures at one_launch.
+template <int NT, bool REFINE>
+__global__ __launch_bounds__(NT) void k_step32(const double2 *__restrict__ src, double2 *__restrict__ dst, int n,
+                                               int p0, int pc, int b0, const int *__restrict__ erp,
+                                               const int *__restrict__ eci, const float *__restrict__ ew, double W,
+                                               int law, const double *__restrict__ stepp, double step,
+                                               double *__restrict__ eterm) {
+    __shared__ double2 red[NT / 64];
+    const int tid = threadIdx.x;
+    const int i = b0 + (int)blockIdx.x;
+    const double2 pi = src[i];
+    const int e0 = erp[i], e1 = erp[i + 1];
+    const int jn = e0 + tid < e1 ? eci[e0 + tid] : 0;
+    double ax = 0.0, ay = 0.0;
+    strided_sum<REFINE, NT>(src, tid, n, pi.x, pi.y, ax, ay);
+    double cx = 0.0, cy = 0.0;
+    for (int e = e0 + tid; e < e1; e += NT) {
+        const double2 pj = src[e == e0 + tid ? jn : eci[e]];
+        correct_pair<REFINE>(law, ew ? W * (double)ew[e] : W, pj.x - pi.x, pj.y - pi.y, cx, cy);
+    }
+    ax = wave_sum(ax + cx);
+    ay = wave_sum(ay + cy);
+    if ((tid & 63) == 0) red[tid >> 6] = make_double2(ax, ay);
+    __syncthreads();
+    if (tid == 64)
+        for (int k = (int)blockIdx.x; k < pc; k += (int)gridDim.x) dst[p0 + k] = src[p0 + k];
+    if (tid == 0) {
+        double fx = red[0].x, fy = red[0].y;
+#pragma unroll
+        for (int w = 1; w < NT / 64; ++w) fx += red[w].x, fy += red[w].y;
+        dst[i] = moved(pi, fx, fy, stepp ? *stepp : step);
+        eterm[i] = fx * fx + fy * fy;
+    }
+}
+
+__global__ __launch_bounds__(WG) void k_copy(const double2 *__restrict__ src, double2 *__restrict__ dst, int n) {
+    const int i = (int)blockIdx.x * WG + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
 // FP64 reference-order pair kernel.  grid = (ceil(n/512), rows of 16 batch vertices, in y and z);
 // block x covers the reference's j block [512x, 512x+512) for a row.
 //
@@ -217,7 +263,8 @@ __global__ __launch_bounds__(64 + WG) void k_pairs64(const double2 *__restrict__
 // pieces (FP64, fixed order: strided per thread, then a fixed tree).
 __global__ __launch_bounds__(WG) void k_move32(const double2 *__restrict__ part, int P, int G,
                                                const int *__restrict__ cpre, double2 *__restrict__ pos, int b0,
-                                               int bc, const double *__restrict__ stepp, double *__restrict__ eterm) {
+                                               int bc, const double *__restrict__ stepp, double step,
+                                               double *__restrict__ eterm) {
     __shared__ double2 red[WG / 64];
     const int slot = (int)blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -248,7 +295,7 @@ __global__ __launch_bounds__(WG) void k_move32(const double2 *__restrict__ part,
     if (tid == 0) {
         const double fx = (red[0].x + red[1].x) + (red[2].x + red[3].x);
         const double fy = (red[0].y + red[1].y) + (red[2].y + red[3].y);
-        pos[i] = moved(x0, fx, fy, *stepp);
+        pos[i] = moved(x0, fx, fy, stepp ? *stepp : step);
         eterm[i] = fx * fx + fy * fy;
     }
 }
@@ -256,7 +303,7 @@ __global__ __launch_bounds__(WG) void k_move32(const double2 *__restrict__ part,
 // FP64 mode: prevCoordinates[i] += f per j block in block order (:771), then the move.  A lane per
 // vertex and component, eight partials loaded at a time.
 __global__ __launch_bounds__(64) void k_move64(const double2 *__restrict__ part, int P, double2 *__restrict__ pos,
-                                               int b0, int bc, const double *__restrict__ stepp,
+                                               int b0, int bc, const double *__restrict__ stepp, double step,
                                                double *__restrict__ eterm) {
     const int slot = (int)blockIdx.x * 32 + threadIdx.x / 2, c = threadIdx.x & 1;
     const double *row = &part[(size_t)min(slot, bc - 1) * P].x + c;
@@ -264,12 +311,12 @@ __global__ __launch_bounds__(64) void k_move64(const double2 *__restrict__ part,
 #pragma unroll 8
     for (int p = 0; p < P; ++p) s += row[2 * p];
     const double other = __shfl_xor(s, 1);
-    if (slot < bc && c == 0) move_one(pos, b0 + slot, s, other, *stepp, eterm);
+    if (slot < bc && c == 0) move_one(pos, b0 + slot, s, other, stepp ? *stepp : step, eterm);
 }
 
-// STEP lives on the device so that one iteration's launches are the same every iteration (and
-// can be replayed as a captured graph): set once, then multiplied after each iteration with the
-// host's FP64 operation.
+// STEP for a captured graph lives on the device so that one iteration's launches are the same every
+// iteration: set once, then multiplied after each iteration with the host's FP64 operation.
+// Otherwise it is an argument of the launches.
 __global__ void k_step_set(double *stepp, double v) {
     if (threadIdx.x == 0) *stepp = v;
 }
@@ -415,6 +462,25 @@ static int static_scratch(int device, unsigned char **out) {
 
 static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 
+// One launch a step (k_step32) or two (k_pairs32, k_move32).  A step of one launch takes 3.8 us and
+// each workgroup's pass over all positions, one of two 6.6 us and its pairs at the whole chip's rate.
+// us a step, two launches / one, by n (random geometric graphs):
+//   -batch    1,000        4,000        10,000       20,000        40,000
+//     64      6.6 / 3.8    6.5 / 3.9    6.8 / 5.2    7.1 / 6.0     7.1 / 7.9
+//    256      8.4 / 5.3    7.2 / 5.0    6.8 / 6.2    7.6 / 6.9     8.8 / 8.8
+//  1,024     14.9 / 12.2   9.9 / 7.8   11.0 / 9.5   13.7 / 13.7   20.7 / 24.6
+// Threads a vertex: 1,024 where 256 would each take many positions and a CU has one vertex (10,000 at
+// -batch 256: 6.2 us against 6.3, 20,000: 6.9 against 7.7; 4,000: 5.0 both); with more vertices a CU
+// 256 (10,000 at -batch 1,024: 9.5 against 15.9).
+constexpr int STEP_ONE_MAX = 20480, STEP_ONE_BATCH = 1024, STEP_WIDE = 8192;
+static bool one_launch(int n, int bmax) {
+    if (const char *e = getenv("BL_STEP_LAUNCHES"))  // tests
+        if (atoi(e) == 2) return false;
+    return n <= STEP_ONE_MAX && bmax <= STEP_ONE_BATCH;
+}
+// The second array never makes a layout too large for the static workspace.
+static_assert(4096 + 24u * (STEP_ONE_MAX + 64) <= BL_STATIC_SCRATCH_BYTES, "two arrays exceed the workspace");
+
 int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double decay, double step0, int iters,
                   bool converged, bl_stats *st, bool static_ws) {
     const int n = g->n;
@@ -451,6 +517,8 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         P = G + g->corr_max_pieces;
         part_elems = (size_t)bmax * P;
     }
+    const bool one = !fp64 && one_launch(n, bmax);
+    const size_t a_elems = one ? (size_t)n : part_elems;  // the second position array in the partials' place
     double2 *part;
     double *eterm, *energy;
     if (static_ws) {
@@ -458,7 +526,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         // earlier in the same step, so the contents of the previous call do not matter
         static_assert(sizeof(double) * (4 + ENERGY_PARTS) <= 4096, "energy shares exceed their part");
         const size_t off_part = 4096;
-        const size_t off_eterm = off_part + round256(sizeof(double2) * part_elems);
+        const size_t off_eterm = off_part + round256(sizeof(double2) * std::max(a_elems, part_elems));
         const size_t need = off_eterm + round256(sizeof(double) * (size_t)n);
         if (need > BL_STATIC_SCRATCH_BYTES) return BL_E_SCRATCH;
         unsigned char *ws = nullptr;
@@ -468,7 +536,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         part = reinterpret_cast<double2 *>(ws + off_part);
         eterm = reinterpret_cast<double *>(ws + off_eterm);
     } else {
-        if (g->part.ensure(sizeof(double2) * part_elems)) return BL_E_NOMEM;
+        if (g->part.ensure(sizeof(double2) * a_elems)) return BL_E_NOMEM;
         if (g->eterm.ensure(sizeof(double) * (size_t)n)) return BL_E_NOMEM;
         if (g->energy.ensure(sizeof(double) * (4 + ENERGY_PARTS))) return BL_E_NOMEM;
         part = g->part.as<double2>();
@@ -479,14 +547,45 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
     Prof prof;
     prof.on = p->profile != 0;
     prof.s = s;
-    double *d_step = energy + 1;  // energy[0] is the sum, energy[4 ..] its shares
-    hipLaunchKernelGGL(k_step_set, dim3(1), dim3(64), 0, s, d_step, step0);
+    const char *genv = getenv("BL_GRAPH");
+    const bool want_graph = !prof.on && !static_ws && (converged || iters >= 2) && genv && !strcmp(genv, "1");
+    double STEP = step0;
+    // energy[0] is the sum, energy[1] STEP for a captured graph (else a launch's argument), energy[4 ..]
+    // the sum's shares
+    double *const d_step = want_graph ? energy + 1 : nullptr;
+    if (want_graph) hipLaunchKernelGGL(k_step_set, dim3(1), dim3(64), 0, s, d_step, step0);
+    // One launch a step: the array that the next step reads, and the batch that the other one lacks.
+    // The steps' number is known (or made even, each iteration) so that the last one writes pos.
+    double2 *const both[2] = {pos, part};
+    const bool even_out = converged || want_graph;
+    int cur = even_out ? 0 : (int)((int64_t)iters * nb & 1), p0 = 0, pc = 0;
+    if (one && (converged || iters > 0))
+        hipLaunchKernelGGL(k_copy, dim3((n + WG - 1) / WG), dim3(WG), 0, s, pos, part, n);
     // One iteration's launches: every batch step (pairs, then the move), the energy, STEP *= decay.
-    auto emit_iteration = [&]() -> int {
+    auto emit_iteration = [&](bool energy_seen) -> int {
         for (int b = 0; b < nb; ++b) {
             const int b0 = b * B;
             const int bc = (n - b0) < B ? (n - b0) : B;
-            if (fp64) {
+            if (one) {
+                hipEvent_t e0 = nullptr, e1 = nullptr;
+                if (prof.on) prof.ext(0, &e0, &e1);
+                const auto go = [&](auto kernel, int threads) {
+                    if (prof.on)  // the dispatch records its own start and end
+                        hipExtLaunchKernelGGL(kernel, dim3(bc), dim3(threads), 0, s, e0, e1, 0, both[cur],
+                                              both[cur ^ 1], n, p0, nb > 1 ? pc : 0, b0, erp, eci, ew, p->weight, law,
+                                              d_step, STEP, eterm);
+                    else
+                        hipLaunchKernelGGL(kernel, dim3(bc), dim3(threads), 0, s, both[cur], both[cur ^ 1], n, p0,
+                                           nb > 1 ? pc : 0, b0, erp, eci, ew, p->weight, law, d_step, STEP, eterm);
+                };
+                const bool wide = n > STEP_WIDE && bmax <= 256;
+                if (p->precision == BL_PREC_FP32)
+                    wide ? go(k_step32<1024, false>, 1024) : go(k_step32<256, false>, 256);
+                else
+                    wide ? go(k_step32<1024, true>, 1024) : go(k_step32<256, true>, 256);
+                cur ^= 1;
+                p0 = b0, pc = bc;
+            } else if (fp64) {
                 prof.begin(0);
                 const int rows = (bc + SLOTS64 - 1) / SLOTS64;
                 hipLaunchKernelGGL(k_pairs64, dim3(G, std::min(rows, ROWS64), (rows + ROWS64 - 1) / ROWS64),
@@ -494,7 +593,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
                                    erp, eci, ew, p->weight, law);
                 prof.end();
                 prof.begin(1);
-                hipLaunchKernelGGL(k_move64, dim3((bc + 31) / 32), dim3(64), 0, s, part, P, pos, b0, bc, d_step,
+                hipLaunchKernelGGL(k_move64, dim3((bc + 31) / 32), dim3(64), 0, s, part, P, pos, b0, bc, d_step, STEP,
                                    eterm);
                 prof.end();
             } else {
@@ -513,7 +612,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
                                               chunk, G, part, P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc);
                     prof.ext(1, &e0, &e1);
                     hipExtLaunchKernelGGL(k_move32, dim3(bc), dim3(WG), 0, s, e0, e1, 0, part, P, G, cpre, pos, b0, bc,
-                                          d_step, eterm);
+                                          d_step, STEP, eterm);
                 } else {
                     if (p->precision == BL_PREC_FP32)
                         hipLaunchKernelGGL((k_pairs32<4, false>), grid, dim3(WG), 0, s, pos, n, b0, bc, chunk, G, part,
@@ -522,14 +621,21 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
                         hipLaunchKernelGGL((k_pairs32<4, true>), grid, dim3(WG), 0, s, pos, n, b0, bc, chunk, G, part,
                                            P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc);
                     hipLaunchKernelGGL(k_move32, dim3(bc), dim3(WG), 0, s, part, P, G, cpre, pos, b0, bc, d_step,
-                                       eterm);
+                                       STEP, eterm);
                 }
             }
         }
-        prof.begin(2);
-        const int rc = launch_energy(eterm, n, energy, p->precision, s);
-        prof.end();
-        hipLaunchKernelGGL(k_step_decay, dim3(1), dim3(64), 0, s, d_step, decay);
+        if (one && even_out && cur) {  // the last step wrote the other array: its batch is what pos lacks
+            hipLaunchKernelGGL(k_copy, dim3((pc + WG - 1) / WG), dim3(WG), 0, s, part + p0, pos + p0, pc);
+            cur = pc = 0;
+        }
+        int rc = BL_OK;
+        if (energy_seen) {
+            prof.begin(2);
+            rc = launch_energy(eterm, n, energy, p->precision, s);
+            prof.end();
+        }
+        if (want_graph) hipLaunchKernelGGL(k_step_decay, dim3(1), dim3(64), 0, s, d_step, decay);
         return rc;
     };
     // BL_GRAPH=1 (and no per-launch timing): one iteration is captured once as a graph and
@@ -544,10 +650,8 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
             if (e) (void)hipGraphExecDestroy(e);
         }
     } ex;
-    const char *genv = getenv("BL_GRAPH");
-    const bool want_graph = !prof.on && !static_ws && (converged || iters >= 2) && genv && !strcmp(genv, "1");
     if (want_graph && hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) {
-        const int rc = emit_iteration();
+        const int rc = emit_iteration(true);
         hipGraph_t gr = nullptr;
         const hipError_t ee = hipStreamEndCapture(s, &gr);
         if (rc == BL_OK && ee == hipSuccess && gr) {
@@ -556,7 +660,6 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         if (gr) (void)hipGraphDestroy(gr);
         (void)hipGetLastError();  // a failed capture leaves the launches to the loop below
     }
-    double STEP = step0;
     double E = 0.0, E0 = 1.79769313486231570815e+308;
     int loop = 0;
     for (;;) {
@@ -569,7 +672,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         if (ex.e) {
             BL_HIP(hipGraphLaunch(ex.e, s));
         } else {
-            const int rc = emit_iteration();
+            const int rc = emit_iteration(converged || want_graph || loop == iters - 1);
             if (rc) return rc;
             prof.flush();
         }

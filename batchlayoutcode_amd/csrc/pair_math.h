@@ -197,6 +197,52 @@ __device__ __forceinline__ void dense_sum(Src src, const int j0, const int j1, c
     }
 }
 
+// The dense repulsion of (px, py) against positions j0, j0 + D, ... below n, added to (ax, ay): groups of 8
+// as dense_sum, the last one filled up as dense_tail.
+template <bool REFINE, int D>
+__device__ __forceinline__ void strided_sum(const double2 *__restrict__ src, const int j0, const int n, const double px,
+                                            const double py, double &ax, double &ay) {
+    constexpr int N = 8;
+    double sx = 0.0, sy = 0.0;
+    int j = j0;
+    for (; j + (N - 1) * D < n; j += N * D) {
+        double qx[N], qy[N];
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const double2 q = src[j + k * D];
+            qx[k] = q.x, qy[k] = q.y;
+        }
+        pair_rep_group<REFINE, N>(qx, qy, px, py, sx, sy);
+    }
+    if constexpr (REFINE) {
+        if (j < n) {
+            double dx[N], dy[N], r[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                const bool in = j + k * D < n;
+                const double2 q = src[in ? j + k * D : j];
+                dx[k] = in ? q.x - px : 0.0;
+                dy[k] = in ? q.y - py : 0.0;
+                r[k] = in ? fma(dy[k], dy[k], fma(dx[k], dx[k], kTiny64)) : 1.0;
+            }
+            recip_all<N>(r);
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                sx = fma(-dx[k], r[k], sx);
+                sy = fma(-dy[k], r[k], sy);
+            }
+        }
+        if (!(isfinite(sx) && isfinite(sy))) {
+            sx = sy = 0.0;
+            for (j = j0; j < n; j += D) pair_rep<true>(src[j].x, src[j].y, px, py, sx, sy);
+        }
+    } else {
+        for (; j < n; j += D) pair_rep<false>(src[j].x, src[j].y, px, py, sx, sy);
+    }
+    ax += sx;
+    ay += sy;
+}
+
 // Neighbour correction for one (i, j) pair: removes the dense loop's product (dx * inv; with REFINE
 // to its last bits, of the order of the dense sum's own rounding) and adds the attraction.
 template <bool REFINE>

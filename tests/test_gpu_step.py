@@ -1,0 +1,48 @@
+"""The one-launch batch step of small graphs: against the oracle to 1e-4 of the diameter after one iteration
+(as the two-launch step), and through its two position arrays (odd and even numbers of steps, a batch that
+holds the whole graph, a last batch of one, the static workspace, a stop by convergence) bit for bit the
+same as iteration by iteration."""
+import numpy as np
+import pytest
+import torch
+
+from batchlayoutcode_amd import graphs
+from conftest import diameter
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,batch", [(2, 1), (255, 64), (257, 256), (2049, 1024), (2600, 100), (8193, 256), (20480, 1000),
+                                     (20481, 1000)])
+def test_one_launch_a_step(bl, oracle, n, batch, monkeypatch):
+    rng = np.random.default_rng(n)
+    e = np.concatenate([rng.integers(0, n, (3 * n, 2)), np.stack([np.full(n, n // 2), np.arange(n)], 1)])
+    rp, ci = graphs.csr_from_edges(n, e[e[:, 0] != e[:, 1]])
+    w = rng.uniform(0.5, 2.0, len(ci)).astype(np.float32)
+    x0 = rng.random((n, 2))
+    for law, prec in ((2, bl.PREC_MIXED), (3, bl.PREC_MIXED), (8, bl.PREC_FP32)):
+        kw = dict(algo=law, batch=batch, weight=1.5, precision=prec)
+        with bl.Graph(rp, ci, w) as g:
+            print(f"[case] n {n} batch {batch} law {law}", flush=True)
+            one, st1 = g.run(x0, iters=1, **kw)
+            x, step = one, 0.999 if law == 2 else 0.99
+            for _ in range(2):
+                x, st = g.run(x, iters=1, step0=step, **kw)
+                step *= 0.999 if law == 2 else 0.99
+            xy, st3 = g.run(x0, iters=3, **kw)
+            assert np.array_equal(xy, x) and st3.energy == st.energy
+            d = torch.from_numpy(x0).cuda()
+            torch.cuda.synchronize()
+            sts = g.run_device_static(d.data_ptr(), iters=3, **kw)
+            assert np.array_equal(d.cpu().numpy(), xy) and sts.energy == st3.energy
+            if law == 2:  # the law that has the convergence option
+                conv, stc = g.run(x0, converged=1, engt=0.5, **kw)
+                fixed, stf = g.run(x0, iters=int(stc.iters_done), **kw)
+                assert np.array_equal(conv, fixed) and stc.energy == stf.energy
+            monkeypatch.setenv("BL_STEP_LAUNCHES", "2")
+            two, st2 = g.run(x0, iters=1, **kw)
+            monkeypatch.delenv("BL_STEP_LAUNCHES")
+        ref, e_ref, _ = oracle.minibatch(rp, ci, x0, 1, batch, law=law, weight=1.5, w_edge=w)
+        for out, st in ((one, st1), (two, st2)):
+            assert np.abs(out - ref).max() <= 1e-4 * diameter(ref)
+            assert abs(st.energy - e_ref) <= 1e-4 * e_ref
