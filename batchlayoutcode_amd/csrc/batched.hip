@@ -136,11 +136,6 @@ struct PairTree {
     }
 };
 
-__device__ __forceinline__ double2 load_through(const double2 *p) {
-    return make_double2(__hip_atomic_load(&p->x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                        __hip_atomic_load(&p->y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-}
-
 // The subtree of chunks [c0, c0 + cpt) of `sub` positions (whole groups of 8) for position p.
 template <bool REFINE, class Src>
 __device__ __forceinline__ double2 chunk_sums(Src src, int n, int c0, int cpt, int sub, double2 p) {

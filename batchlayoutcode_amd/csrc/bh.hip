@@ -209,7 +209,7 @@ __global__ __launch_bounds__(WG) void k_scan_top(int *__restrict__ bsum, int nb)
 }
 
 __global__ __launch_bounds__(WG) void k_scan_apply(const int *__restrict__ in, int n, const int *__restrict__ bsum,
-                                                   int *__restrict__ out) {
+                                                   int *__restrict__ out, int *__restrict__ list) {
     __shared__ int lds[WG];
     const int base = blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;  // contiguous per thread
     int v[SCAN_ITEMS];
@@ -224,6 +224,7 @@ __global__ __launch_bounds__(WG) void k_scan_apply(const int *__restrict__ in, i
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; ++k) {
         if (base + k < n) out[base + k] = run;
+        if (v[k]) list[run] = base + k;
         run += v[k];
     }
 }
@@ -246,7 +247,7 @@ __device__ __forceinline__ int4 scan_item4(const int4 *src, int q, int i, int n)
 }
 
 __global__ __launch_bounds__(1024) void k_scan_single(const int *__restrict__ in, int n, int *__restrict__ out,
-                                                      int *__restrict__ total) {
+                                                      int *__restrict__ list, int *__restrict__ total) {
     __shared__ int wsum[SCAN_SINGLE_TILES][16];  // [tile][wave]
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int4 *src = reinterpret_cast<const int4 *>(in) + t;
@@ -285,6 +286,10 @@ __global__ __launch_bounds__(1024) void k_scan_single(const int *__restrict__ in
             if (i + 1 < n) out[i + 1] = r1;
             if (i + 2 < n) out[i + 2] = r2;
         }
+        if (v[q].x) list[r0] = i;
+        if (v[q].y) list[r1] = i + 1;
+        if (v[q].z) list[r2] = i + 2;
+        if (v[q].w) list[r3] = i + 3;
         carry += tile;
     }
     if (t == 0) *total = carry;
@@ -502,62 +507,13 @@ __global__ __launch_bounds__(WG) void k_sort_ties(uint64_t *__restrict__ keys, i
 
 // ---------------------------------------------------------------------------------------
 // 5. tree
-__device__ __forceinline__ int digit_at(uint64_t k, int d) { return (int)((k >> (62 - 2 * d)) & 3u); }
-__device__ __forceinline__ uint64_t prefix_of(uint64_t k, int d) { return d == 0 ? 0ull : (k >> (64 - 2 * d)); }
-
-// first index in [lo, hi) whose 2d-bit prefix equals pfx (keys sorted)
-__device__ __forceinline__ int first_with_prefix(const uint64_t *keys, int lo, int hi, int d, uint64_t pfx) {
-    while (lo < hi) {
-        const int m = (lo + hi) >> 1;
-        if (prefix_of(keys[m], d) < pfx) lo = m + 1; else hi = m;
-    }
-    return lo;
-}
-// last index in [lo, hi) whose prefix equals pfx, given keys[lo] has it
-__device__ __forceinline__ int last_with_prefix(const uint64_t *keys, int lo, int hi, int d, uint64_t pfx) {
-    while (hi - lo > 1) {
-        const int m = (lo + hi) >> 1;
-        if (prefix_of(keys[m], d) <= pfx) lo = m; else hi = m;
-    }
-    return lo;
-}
-// first index in [0, i] whose 2d-bit prefix equals pfx, given keys[i] has it: probes leftwards
-// at distances 1, 3, 7, ... from i (a node's points are contiguous and most nodes are small),
-// then a binary search over the last interval
-__device__ __forceinline__ int gallop_first(const uint64_t *keys, int i, int d, uint64_t pfx) {
-    int hi = i, step = 1, lo = i - 1;
-    while (lo >= 0 && prefix_of(keys[lo], d) == pfx) {
-        hi = lo;
-        step <<= 1;
-        lo = hi - step;
-    }
-    return first_with_prefix(keys, lo < 0 ? 0 : lo + 1, hi, d, pfx);
-}
-// last index in [j, n) whose prefix equals pfx, given keys[j] has it (the mirror image)
-__device__ __forceinline__ int gallop_last(const uint64_t *keys, int j, int n, int d, uint64_t pfx) {
-    int lo = j, step = 1, hi = j + 1;
-    while (hi < n && prefix_of(keys[hi], d) == pfx) {
-        lo = hi;
-        step <<= 1;
-        hi = lo + step;
-    }
-    return last_with_prefix(keys, lo, hi < n ? hi : n, d, pfx);
-}
-// first index in [lo, hi) whose digit d is >= q (lower_bound of BarnesHut.h:143-146)
-__device__ __forceinline__ int lower_digit(const uint64_t *keys, int lo, int hi, int d, int q) {
-    while (lo < hi) {
-        const int m = (lo + hi) >> 1;
-        if (digit_at(keys[m], d) < q) lo = m + 1; else hi = m;
-    }
-    return lo;
-}
-// the node whose points are [s, e] (inclusive, e > s): the boundary where its first
-// quadrant ends
-__device__ __forceinline__ int rep_of_range(const uint64_t *keys, int s, int e) {
-    const int d = __clzll((long long)(keys[s] ^ keys[e])) >> 1;
-    const int q0 = digit_at(keys[s], d);
-    return lower_digit(keys, s, e + 1, d, q0 + 1) - 1;
-}
+// A cell of level d is a range of keys; its quadrants' bounds are keys too, so every search is for the
+// first key at or above a bound: one comparison a probe.
+__device__ __forceinline__ int level_of(uint64_t a, uint64_t b) { return __clzll((long long)(a ^ b)) >> 1; }  // a != b
+__device__ __forceinline__ uint64_t cell_low(uint64_t k, int d) { return d == 0 ? 0ull : k >> (64 - 2 * d) << (64 - 2 * d); }
+__device__ __forceinline__ uint64_t cell_high(uint64_t k, int d) { return d == 0 ? ~0ull : k | ((1ull << (64 - 2 * d)) - 1); }
+// the low end of quadrant v of the cell of level d < 32 that begins at low
+__device__ __forceinline__ uint64_t quadrant_low(uint64_t low, int d, int v) { return low + ((uint64_t)v << (62 - 2 * d)); }
 
 // boundary i (between Morton ranks i and i+1) is a node representative when it ends the
 // first quadrant of the cell where k_i and k_i+1 split
@@ -571,80 +527,169 @@ __global__ __launch_bounds__(WG) void k_tree_bounds(const uint64_t *__restrict__
         isrep[i] = 0;
         return;
     }
-    const int d = __clzll((long long)(a ^ b)) >> 1;
-    const uint64_t pfx = prefix_of(a, d);
-    const int L = d == 0 ? 0 : gallop_first(keys, i, d, pfx);
-    isrep[i] = digit_at(keys[L], d) == digit_at(a, d) ? 1 : 0;
+    // a's quadrant is the cell's first when no key of the cell lies below it: probes leftwards at
+    // distances 1, 3, 7, ... (the quadrant's keys are contiguous and most are few), then a binary search
+    // for the key before the quadrant
+    const int d = level_of(a, b);
+    const uint64_t cell = cell_low(a, d), quad = cell_low(a, d + 1);
+    int hi = i, lo = i - 1;  // keys[hi] >= quad; keys[lo] < quad or lo < 0 in the end
+    uint64_t k = lo >= 0 ? keys[lo] : 0ull;
+    for (int step = 2; lo >= 0 && k >= quad; step <<= 1) {
+        hi = lo;
+        lo = hi - step;
+        k = keys[max(lo, 0)];
+    }
+    bool first = quad == cell || lo < 0 || k < cell;  // not yet known to hold a key of the cell below
+    if (quad != cell && first) {
+        lo = max(lo, -1);
+        while (hi - lo > 1) {
+            const int m = (lo + hi) >> 1;
+            k = keys[m];
+            if (k >= quad) {
+                hi = m;
+            } else {
+                lo = m;
+                if (k >= cell) break;
+            }
+        }
+        first = lo < 0 || keys[lo] < cell;
+    }
+    isrep[i] = first ? 1 : 0;
 }
 
-// root = the node spanning all points; also the node count (scan total)
-__global__ void k_tree_root(const uint64_t *__restrict__ keys, int n, const int *__restrict__ nodeid,
-                            const int *__restrict__ scan_total, int *__restrict__ misc) {
-    if (threadIdx.x != 0 || blockIdx.x != 0 || misc[0]) return;
-    misc[1] = nodeid[rep_of_range(keys, 0, n - 1)];
-    misc[2] = *scan_total;
-}
-
-__global__ __launch_bounds__(WG) void k_tree_nodes(const uint64_t *__restrict__ keys, int n,
-                                                   const int *__restrict__ isrep, const int *__restrict__ nodeid,
-                                                   BHNode *__restrict__ nodes, int *__restrict__ npts,
-                                                   int *__restrict__ node_lo, int *__restrict__ misc,
-                                                   const int *__restrict__ status) {
-    const int i = xcd_tile(blockIdx.x, gridDim.x) * WG + threadIdx.x;
-    if (*status) return;
-    if (i >= n - 1 || !isrep[i]) return;
-    const int v = nodeid[i];
-    const uint64_t a = keys[i];
-    const int d = __clzll((long long)(a ^ keys[i + 1])) >> 1;
-    const uint64_t pfx = prefix_of(a, d);
-    const int L = d == 0 ? 0 : gallop_first(keys, i, d, pfx);
-    const int R = d == 0 ? n - 1 : gallop_last(keys, i + 1, n, d, pfx);
-    int bnd[5];
-    bnd[0] = L;
-    bnd[4] = R + 1;
-    for (int q = 1; q < 4; ++q) bnd[q] = lower_digit(keys, L, R + 1, d, q);
-    int ch[4];
-    int nint = 0;
-    for (int q = 0; q < 4; ++q) {
-        const int s = bnd[q], e = bnd[q + 1];
-        if (e - s == 0) {
-            ch[q] = -1;
-        } else if (e - s == 1) {
-            ch[q] = -(s + 2);
-        } else {
-            const int c = nodeid[rep_of_range(keys, s, e - 1)];
-            ch[q] = c;
-            nodes[c].parent = v;
-            ++nint;
+// N searches in step (lower_bound of BarnesHut.h:143-146): lo[q] = the first index in [lo[q], hi[q])
+// whose key is at least bound[q], or hi[q].
+template <int N>
+__device__ __forceinline__ void lower_bounds(const uint64_t *keys, int *lo, int *hi, const uint64_t *bound) {
+    for (;;) {
+        bool more = false;
+        uint64_t k[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const bool on = lo[q] < hi[q];
+            more = more || on;
+            k[q] = keys[on ? (lo[q] + hi[q]) >> 1 : 0];
+        }
+        if (!more) break;
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const int m = (lo[q] + hi[q]) >> 1;
+            const bool on = lo[q] < hi[q], below = k[q] < bound[q];
+            lo[q] = on && below ? m + 1 : lo[q];
+            hi[q] = on && !below ? m : hi[q];
         }
     }
+}
+
+// The range [L, R] of ranks around boundary i with keys in [low, high], all distinct: probes on both
+// sides at distances 1, 3, 7, ..., then the search of the last intervals.
+__device__ __forceinline__ void gallop_both(const uint64_t *keys, int i, int n, uint64_t low, uint64_t high, int &L,
+                                            int &R) {
+    int a = i - 1, b = i, x = i + 1, y = i + 2;  // [b, x] is inside; a and y are probed
+    bool left = true, right = true;
+    for (int step = 2; left || right; step <<= 1) {
+        const uint64_t ka = keys[max(a, 0)], ky = keys[min(y, n - 1)];
+        left = left && a >= 0 && ka >= low;
+        right = right && y < n && ky <= high;
+        if (left) b = a, a = b - step;
+        if (right) x = y, y = x + step;
+    }
+    int lo[2] = {max(a, -1) + 1, x + 1}, hi[2] = {b, min(y, n)};
+    const int end = hi[1];
+    const uint64_t bound[2] = {low, high};  // not high + 1, which is 0 for the last cell
+    lower_bounds<2>(keys, lo, hi, bound);
+    L = lo[0];
+    R = lo[1] < end && keys[lo[1]] == high ? lo[1] : lo[1] - 1;
+}
+
+// One node a thread, by the list of the representative boundaries (misc: status, the root, the number of
+// nodes).  What bounds it is the operations of each wave's longest searches (neither a window of the keys
+// in LDS nor seven probes a round is faster).  The two ends of the range, then the three inner quadrant
+// bounds, then the representatives of the four quadrants are searched in step: 34 -> 25 us on the 250k
+// random geometric graph, 98 -> 90 on the 1.66M-vertex mesh.
+__global__ __launch_bounds__(WG) void k_tree_nodes(const uint64_t *__restrict__ keys, int n,
+                                                   const int *__restrict__ list, const int *__restrict__ nodeid,
+                                                   const int *__restrict__ scan_total, BHNode *__restrict__ nodes,
+                                                   int *__restrict__ npts, int *__restrict__ node_lo,
+                                                   int *__restrict__ misc, const int *__restrict__ status) {
+    const int v = xcd_tile(blockIdx.x, gridDim.x) * WG + threadIdx.x;
+    if (*status || v >= *scan_total) return;
+    const int i = list[v];
+    const uint64_t a = keys[i];
+    const int d = level_of(a, keys[i + 1]);
+    const uint64_t low = cell_low(a, d);
+    int L = 0, R = n - 1;
+    if (d != 0) gallop_both(keys, i, n, low, cell_high(a, d), L, R);
+    int bnd[5] = {L, L, L, L, R + 1};
+    {
+        int hi[3] = {R + 1, R + 1, R + 1};
+        const uint64_t bound[3] = {quadrant_low(low, d, 1), quadrant_low(low, d, 2), quadrant_low(low, d, 3)};
+        lower_bounds<3>(keys, bnd + 1, hi, bound);
+    }
+    // the representative of each quadrant of more than one point: the boundary where its first
+    // quadrant ends
+    int lo[4], hi[4], ch[4], nint = 0;
+    uint64_t bound[4];
+    {
+        uint64_t first[4], last[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            lo[q] = bnd[q], hi[q] = bnd[q + 1] - bnd[q] > 1 ? bnd[q + 1] : bnd[q];
+            first[q] = keys[min(bnd[q], n - 1)], last[q] = keys[max(bnd[q + 1] - 1, 0)];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            bound[q] = hi[q] > lo[q] ? cell_high(first[q], level_of(first[q], last[q]) + 1) + 1 : 0ull;
+    }
+    lower_bounds<4>(keys, lo, hi, bound);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int m = bnd[q + 1] - bnd[q];
+        ch[q] = m == 0 ? -1 : m == 1 ? -(bnd[q] + 2) : lo[q] - 1;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool in = ch[q] >= 0;
+        const int c = nodeid[in ? ch[q] : 0];  // the loads together
+        ch[q] = in ? c : ch[q];
+        nint += in ? 1 : 0;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (ch[q] >= 0) nodes[ch[q]].parent = v;
     nodes[v].ch = make_int4(ch[0], ch[1], ch[2], ch[3]);
     nodes[v].depth = d;
     nodes[v].nint = nint;
     nodes[v].cnt = 0;
     npts[v] = R - L + 1;
     node_lo[v] = L;
-    if (v == misc[1]) nodes[v].parent = -1;
+    if (L == 0 && R == n - 1) {  // spans all points
+        nodes[v].parent = -1;
+        misc[1] = v;
+        misc[2] = *scan_total;
+    }
 }
 
-// 6. centroids, bottom-up; the last child to finish computes its parent.  WT: stored with
-// agent-scope stores, which the L2 writes through to memory
-template <bool WT = false>
-__device__ __forceinline__ void centroid_of(BHNode *nodes, const double2 *spos, int v) {
-    const int4 ch = nodes[v].ch;
+// 6. centroids, bottom-up
+// The positions of the children ch of a node, c of an internal child (of leaf or empty ones any
+// position): unconditional agent-scope loads, all four in flight together.
+__device__ __forceinline__ void child_points(const BHNode *nodes, const double2 *spos, const int4 ch, double2 *p) {
+    const int c[4] = {ch.x, ch.y, ch.z, ch.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        p[q] = load_through(c[q] >= 0 ? &nodes[c[q]].c : &spos[c[q] <= -2 ? -c[q] - 2 : 0]);
+    }
+}
+
+// The unweighted mean of the non-empty quadrants, in the reference's order.
+__device__ __forceinline__ double2 mean_of(const int4 ch, const double2 *p) {
     const int c[4] = {ch.x, ch.y, ch.z, ch.w};
     double sx = 0.0, sy = 0.0, count = 0.0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        if (c[q] >= 0) {
-            const double2 cc = nodes[c[q]].c;
-            sx += cc.x;
-            sy += cc.y;
-            count++;
-        } else if (c[q] <= -2) {
-            const double2 p = spos[-c[q] - 2];
-            sx += p.x;
-            sy += p.y;
+        if (c[q] != -1) {
+            sx += p[q].x;
+            sy += p[q].y;
             count++;
         }
     }
@@ -652,96 +697,110 @@ __device__ __forceinline__ void centroid_of(BHNode *nodes, const double2 *spos, 
         sx /= count;
         sy /= count;
     }
-    if (WT) {
-        __hip_atomic_store(&nodes[v].c.x, sx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&nodes[v].c.y, sy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-        nodes[v].c = make_double2(sx, sy);
-    }
+    return make_double2(sx, sy);
 }
 
-// Centroids bottom-up in two launches that keep the agent-scope handoffs to the top of the
-// tree.  A "small" node holds at most SMALL_CELL points.  k_centroid_small: one thread per
-// small subtree (a small node whose parent is not small) computes its nodes in post-order,
-// with no synchronisation.  k_centroid_top: the large nodes, from those without large
-// children upwards; the last large child to arrive at a parent computes it; small children
-// were done by the previous launch.  Every centroid is formed by centroid_of from its
-// children, so the order of the operations is the reference's.
+// Centroids in two launches that keep the agent-scope handoffs to the top of the tree.  A "small" node
+// holds at most SMALL_CELL points, so all nodes below it are among the SMALL_CELL - 2 node ids on either
+// side of its own (ids follow the Morton order of the points).  k_centroid_small: one thread per node of
+// WG ids and the SMALL_CELL on either side, children and leaf positions loaded at once, then a round
+// per level of the subtrees in LDS; the nodes on the sides are formed by two workgroups and stored
+// by their own: 46 -> 12 us on the 250k random geometric graph, 60 -> 19 on the R-MAT graph of scale 20,
+// against one thread that walked each subtree in memory.  k_centroid_top: the large nodes, from those without large children upwards; the
+// last large child to arrive at a parent computes it; small children were done by the previous
+// launch.  Every centroid is formed by mean_of from its children, so the order of the
+// operations is the reference's.
 constexpr int SMALL_CELL = 32;
+constexpr int CS_T = WG + 2 * SMALL_CELL;
 
-// The first internal child of node u in quadrant order (-1: none).
-__device__ __forceinline__ int first_internal(const BHNode *nodes, int u) {
-    const int4 ch = nodes[u].ch;
-    return ch.x >= 0 ? ch.x : ch.y >= 0 ? ch.y : ch.z >= 0 ? ch.z : ch.w;  // ch.w: itself, or < 0
-}
-
-// The internal sibling after child u of node p in quadrant order (-1: none).
-__device__ __forceinline__ int next_internal(const BHNode *nodes, int p, int u) {
-    const int4 ch = nodes[p].ch;
+__global__ __launch_bounds__(CS_T) void k_centroid_small(BHNode *__restrict__ nodes, const double2 *__restrict__ spos,
+                                                         const int *__restrict__ npts, const int *__restrict__ misc) {
+    constexpr int NEVER = 1 << 30, SKIP = -1;  // not formed yet; a subtree that leaves the workgroup's nodes
+    __shared__ double2 cen[CS_T];
+    __shared__ int done[CS_T];  // the round that formed the node
+    const int tid = threadIdx.x, count = misc[2];
+    if (misc[0] || (int)blockIdx.x * WG >= count) return;
+    const int base = (int)blockIdx.x * WG - SMALL_CELL, v = base + tid;
+    bool todo = v >= 0 && v < count && npts[v] <= SMALL_CELL;
+    int4 ch = make_int4(-1, -1, -1, -1);
+    if (todo) ch = nodes[v].ch;
     const int c[4] = {ch.x, ch.y, ch.z, ch.w};
-    int nx = -1;
-    bool past = false;
+    double2 p[4];
+    bool leaves = false;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        if (past && nx < 0 && c[q] >= 0) nx = c[q];
-        past = past || c[q] == u;
+        p[q] = spos[c[q] <= -2 ? -c[q] - 2 : 0];
+        leaves = leaves || (c[q] >= 0 && (unsigned)(c[q] - base) >= (unsigned)CS_T);
     }
-    return nx;
-}
-
-// One thread per small subtree: its internal nodes in post-order (children in quadrant order)
-// without a stack, by the parent links (no LDS, so the mostly idle workgroups of the node-id
-// grid do not hold back occupancy).
-__global__ __launch_bounds__(WG) void k_centroid_small(BHNode *__restrict__ nodes, const double2 *__restrict__ spos,
-                                                       const int *__restrict__ npts, const int *__restrict__ misc) {
-    const int r = blockIdx.x * WG + threadIdx.x;
-    if (misc[0] || r >= misc[2]) return;
-    const int par = nodes[r].parent;
-    if (npts[r] > SMALL_CELL || (par >= 0 && npts[par] <= SMALL_CELL)) return;
-    int u = r;
-    for (int d; (d = first_internal(nodes, u)) >= 0;) u = d;
-    for (;;) {
-        centroid_of(nodes, spos, u);  // its internal children are done
-        if (u == r) break;
-        const int p = nodes[u].parent;
-        const int nx = next_internal(nodes, p, u);
-        if (nx < 0) {
-            u = p;
-            continue;
+    done[tid] = leaves || !todo ? SKIP : NEVER;
+    todo = todo && !leaves;
+    __syncthreads();
+    for (int round = 1; __syncthreads_or(todo) && round < 2 * SMALL_CELL; ++round) {
+        if (!todo) continue;
+        bool ready = true, skip = false;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (c[q] < 0) continue;
+            const int d = *(volatile int *)&done[c[q] - base];
+            skip = skip || d == SKIP;
+            ready = ready && d < round;
         }
-        u = nx;
-        for (int d; (d = first_internal(nodes, u)) >= 0;) u = d;
+        if (skip) {
+            done[tid] = SKIP;
+            todo = false;
+        } else if (ready) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c[q] >= 0) p[q] = cen[c[q] - base];
+            const double2 m = mean_of(ch, p);
+            cen[tid] = m;
+            done[tid] = round;
+            todo = false;
+            if (tid >= SMALL_CELL && tid < SMALL_CELL + WG) nodes[v].c = m;
+        }
     }
 }
 
 __device__ __forceinline__ int large_children(const BHNode *nodes, const int *npts, int v) {
     const int4 ch = nodes[v].ch;
     const int c[4] = {ch.x, ch.y, ch.z, ch.w};
-    int k = 0;
+    int m[4], k = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) k += (c[q] >= 0 && npts[c[q]] > SMALL_CELL) ? 1 : 0;
+    for (int q = 0; q < 4; ++q) m[q] = npts[max(c[q], 0)];  // the loads together
+#pragma unroll
+    for (int q = 0; q < 4; ++q) k += c[q] >= 0 && m[q] > SMALL_CELL ? 1 : 0;
     return k;
 }
 
 // The large nodes climb: a node's centroid is stored with agent-scope stores (written through
 // the XCD's L2 to memory), and once they have completed a relaxed counter at the parent counts
-// the arrival; the last child to arrive acquires (invalidating its own L2's stale lines) and
-// computes the parent from memory.  An acq_rel counter would write the whole L2 back at every
-// step.
+// the arrival; the last child to arrive computes the parent, from memory by agent-scope loads (an
+// acquire would drop the L2's lines at every step, an acq_rel counter write them back).  What the
+// launch doesn't change (the parent, its children and their counts) is loaded before the hand-off.  39 -> 18
+// us on the 250k random geometric graph, 74 -> 24 on the R-MAT graph.
 __global__ __launch_bounds__(WG) void k_centroid_top(BHNode *__restrict__ nodes, const double2 *__restrict__ spos,
                                                      const int *__restrict__ npts, const int *__restrict__ misc) {
     int v = blockIdx.x * WG + threadIdx.x;
     if (misc[0] || v >= misc[2]) return;
     if (npts[v] <= SMALL_CELL || large_children(nodes, npts, v) != 0) return;
+    int4 ch = nodes[v].ch;
     for (;;) {
-        centroid_of<true>(nodes, spos, v);
+        double2 p[4];
+        child_points(nodes, spos, ch, p);
         const int u = nodes[v].parent;
+        int need = 0;
+        int4 chu = ch;
+        if (u >= 0) {
+            need = large_children(nodes, npts, u);
+            chu = nodes[u].ch;
+        }
+        store_through(&nodes[v].c, mean_of(ch, p));
         if (u < 0) break;
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         const int old = __hip_atomic_fetch_add(&nodes[u].cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (old != large_children(nodes, npts, u) - 1) break;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (old != need - 1) break;
         v = u;
+        ch = chu;
     }
 }
 
@@ -2068,16 +2127,16 @@ struct TreeBufs {
 // Exclusive scan of in[0, n) into out, the total at bsum[nb].  `in` must hold at least
 // SCAN_SINGLE_MAX ints whatever n is (k_scan_single reads all its tiles; ensure_bh sizes the
 // boundary-flag buffer so).
-int scan_excl(const int *in, int n, int *out, int *bsum, hipStream_t s) {
+int scan_excl(const int *in, int n, int *out, int *list, int *bsum, hipStream_t s) {
     const int nb = (n + SCAN_TILE - 1) / SCAN_TILE;
     if (n <= SCAN_SINGLE_MAX) {  // one launch instead of three
-        hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(1024), 0, s, in, n, out, bsum + nb);
+        hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(1024), 0, s, in, n, out, list, bsum + nb);
         BL_HIP(hipGetLastError());
         return BL_OK;
     }
     hipLaunchKernelGGL(k_scan_sums, dim3(nb), dim3(WG), 0, s, in, n, bsum);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(WG), 0, s, bsum, nb);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(WG), 0, s, in, n, bsum, out);
+    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(WG), 0, s, in, n, bsum, out, list);
     BL_HIP(hipGetLastError());
     return BL_OK;
 }
@@ -2143,16 +2202,16 @@ int build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t *
         int *isrep = w.isrep.as<int>(), *nodeid = w.nodeid.as<int>();
         BHNode *nodes = w.node_child.as<BHNode>();
         hipLaunchKernelGGL(k_tree_bounds, dim3(g1), dim3(WG), 0, s, ka, n, isrep, misc);
-        rc = scan_excl(isrep, n - 1, nodeid, bsum, s);
+        int *list = w.idx_b.as<int>();  // free after the sort
+        rc = scan_excl(isrep, n - 1, nodeid, list, bsum, s);
         if (rc) return rc;
         const int nsb = (n - 1 + SCAN_TILE - 1) / SCAN_TILE;
-        hipLaunchKernelGGL(k_tree_root, dim3(1), dim3(64), 0, s, ka, n, nodeid, bsum + nsb, misc);
         int *npts = w.node_cnt.as<int>();
-        hipLaunchKernelGGL(k_tree_nodes, dim3(g1), dim3(WG), 0, s, ka, n, isrep, nodeid, nodes, npts,
-                           w.node_lo.as<int>(), misc, misc);
+        hipLaunchKernelGGL(k_tree_nodes, dim3(g1), dim3(WG), 0, s, ka, n, list, nodeid, bsum + nsb, nodes,
+                           npts, w.node_lo.as<int>(), misc, misc);
         // n-1 boundaries give at most n-1 nodes; threads beyond the node count (misc[2]) exit
         if (centroids) {
-            hipLaunchKernelGGL(k_centroid_small, dim3(g1), dim3(WG), 0, s, nodes, spos, npts, misc);
+            hipLaunchKernelGGL(k_centroid_small, dim3(g1), dim3(CS_T), 0, s, nodes, spos, npts, misc);
             hipLaunchKernelGGL(k_centroid_top, dim3(g1), dim3(WG), 0, s, nodes, spos, npts, misc);
         }
     } else {

@@ -57,24 +57,26 @@ __device__ FarCell far_summary(int4 ch, const double2 *spos, const FarCell *cell
     const int c[4] = {ch.x, ch.y, ch.z, ch.w};
     double m = 0.0, sx = 0.0, sy = 0.0;
     double km[4], kx[4], ky[4], kxx[4], kxy[4], kyy[4];
+    // every child's record and position loaded, whatever it is, so that the loads are in flight together
+    FarCell k[4];
+    double2 p[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        km[q] = 0.0;
-        kx[q] = ky[q] = kxx[q] = kxy[q] = kyy[q] = 0.0;
-        if (c[q] >= 0) {
-            const FarCell k = cells[c[q]];
-            km[q] = k.m;
-            kx[q] = k.cx;
-            ky[q] = k.cy;
-            kxx[q] = k.mxx;
-            kxy[q] = k.mxy;
-            kyy[q] = k.myy;
-        } else if (c[q] <= -2) {
-            const double2 p = spos[-c[q] - 2];
-            km[q] = 1.0;
-            kx[q] = p.x;
-            ky[q] = p.y;
-        }
+        const FarCell *cell = cells + max(c[q], 0);
+        k[q].cx = load_through(&cell->cx), k[q].cy = load_through(&cell->cy);
+        k[q].mxx = load_through(&cell->mxx), k[q].mxy = load_through(&cell->mxy), k[q].myy = load_through(&cell->myy);
+        k[q].m = load_through(&cell->m);
+        p[q] = spos[c[q] <= -2 ? -c[q] - 2 : 0];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const bool in = c[q] >= 0, leaf = c[q] <= -2;
+        km[q] = in ? (double)k[q].m : leaf ? 1.0 : 0.0;
+        kx[q] = in ? k[q].cx : leaf ? p[q].x : 0.0;
+        ky[q] = in ? k[q].cy : leaf ? p[q].y : 0.0;
+        kxx[q] = in ? k[q].mxx : 0.0;
+        kxy[q] = in ? k[q].mxy : 0.0;
+        kyy[q] = in ? k[q].myy : 0.0;
         m += km[q];
         sx += km[q] * kx[q];
         sy += km[q] * ky[q];
@@ -116,13 +118,11 @@ __device__ __forceinline__ void store_cell_through(FarCell *cells, int v, const 
 // than FAR_SMALL points (nlc).  The larger nodes climb, from those
 // without large children: a node's summary is stored with agent-scope stores (written through
 // to memory) and, once they have completed, a relaxed counter at the parent (BHNode.cnt, zeroed
-// by the tree build) counts the arrival; the last child to arrive acquires (invalidating its own
-// L2's stale lines) and forms the parent from its children by far_summary.  An acq_rel counter
-// would write the whole L2 back at every step.  What does not change in the launch (the
-// parent, its children and its nlc) is loaded before the hand-off, so a step waits for the
-// children's summaries, the stores and the counter only (k_far_top 145 -> 137 us on the
-// 1.66M-vertex Delaunay graph's layout at FAR_SMALL 32; the climb's nine levels cost about
-// 15 us each).
+// by the tree build) counts the arrival; the last child to arrive forms the parent from its children by
+// far_summary, which loads them from memory by agent-scope loads, all at once.  What does not change
+// in the launch (the parent, its children and its nlc) is loaded before the hand-off.  A step took
+// about 12 us when it acquired (which drops the L2's lines) and loaded child after child: k_far_top
+// 112 -> 49 us on the 1.66M-vertex Delaunay graph.
 constexpr int FAR_SMALL = 64;  // Delaunay graph, per iteration: 16: 251 us, 32: 204, 64: 179, 128: 191
 
 __global__ __launch_bounds__(WG) void k_far_direct(const BHNode *__restrict__ nodes, const double2 *__restrict__ spos,
@@ -191,7 +191,6 @@ __global__ __launch_bounds__(WG) void k_far_top(BHNode *nodes, const double2 *__
         __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
         const int old = __hip_atomic_fetch_add(&nodes[u].cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (old != need - 1) break;
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         v = u;
         ch = chu;
     }
