@@ -6,6 +6,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <mutex>
 #include <new>
@@ -467,15 +468,18 @@ extern "C" int bl_run_batched(int32_t count, const int32_t *voff, const int64_t 
         if (voff[k + 1] <= voff[k] || voff[k + 1] - voff[k] > BL_BATCHED_MAX_N || eoff[k + 1] < eoff[k])
             return BL_E_ARG;
     if (eoff[count] > INT32_MAX || (eoff[count] > 0 && !colids)) return BL_E_ARG;
-    for (int32_t k = 0; k < count; ++k) {  // per-graph CSR validation
-        const int32_t n = voff[k + 1] - voff[k];
-        if (n <= 0 || n > BL_BATCHED_MAX_N) return BL_E_ARG;
-        if (rowptr[voff[k]] != eoff[k] || rowptr[voff[k + 1]] != eoff[k + 1]) return BL_E_GRAPH;
-        for (int32_t i = voff[k]; i < voff[k + 1]; ++i)
-            if (rowptr[i + 1] < rowptr[i]) return BL_E_GRAPH;
-        for (int64_t e = eoff[k]; e < eoff[k + 1]; ++e)
-            if (colids[e] < 0 || colids[e] >= n) return BL_E_GRAPH;
-    }
+    std::atomic<bool> bad{false};
+    auto check = [&](int k0, int k1) {  // per-graph CSR validation
+        for (int k = k0; k < k1 && !bad; ++k) {
+            const int32_t n = voff[k + 1] - voff[k];
+            bool ok = rowptr[voff[k]] == eoff[k] && rowptr[voff[k + 1]] == eoff[k + 1];
+            for (int32_t i = voff[k]; i < voff[k + 1]; ++i) ok &= rowptr[i + 1] >= rowptr[i];
+            for (int64_t e = eoff[k]; e < eoff[k + 1]; ++e) ok &= (uint32_t)colids[e] < (uint32_t)n;
+            if (!ok) bad = true;
+        }
+    };
+    for_ranges(count, check, (int)eoff[count]);
+    if (bad) return BL_E_GRAPH;
     rc = check_device_once();
     if (rc) return rc;
     return run_batched(count, voff, eoff, rowptr, colids, xy_inout, p, energies, finish_ms, st);
