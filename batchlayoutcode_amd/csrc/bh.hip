@@ -2538,10 +2538,12 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
                                g->bh.misc.as<int>());
         }
         prof.end();
-        prof.begin(2);
-        rc = launch_energy(g->eterm.as<double>(), n, g->energy.as<double>(), p->precision, s);
-        prof.end();
-        if (rc) return rc;
+        if (it == iters - 1) {  // only the last iteration's energy is returned
+            prof.begin(2);
+            rc = launch_energy(g->eterm.as<double>(), n, g->energy.as<double>(), p->precision, s);
+            prof.end();
+            if (rc) return rc;
+        }
         prof.flush();
         STEP = STEP * 0.999;  // :1070
     }
