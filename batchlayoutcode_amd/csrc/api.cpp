@@ -216,6 +216,7 @@ static int validate_params(const bl_params *p) {
 static int run_on_device(bl_graph *g, double *d_xy, const bl_params *p, bl_stats *st) {
     bl_stats local;
     memset(&local, 0, sizeof(local));
+    local.nonfinite = -1;  // not counted
     int rc = BL_OK;
     switch (p->algo) {
         case BL_ALGO_CACHE:
@@ -258,7 +259,7 @@ static int run_on_device(bl_graph *g, double *d_xy, const bl_params *p, bl_stats
         default:
             rc = BL_E_ARG;
     }
-    if (rc == BL_OK) {  // the non-finite guard
+    if (rc == BL_OK && local.nonfinite < 0) {  // the non-finite guard of a run without iterations
         if (g->guard.ensure(64)) {
             rc = BL_E_NOMEM;
         } else {
@@ -267,6 +268,7 @@ static int run_on_device(bl_graph *g, double *d_xy, const bl_params *p, bl_stats
             local.nonfinite = nf;
         }
     }
+    local.nonfinite = std::max<decltype(local.nonfinite)>(0, local.nonfinite);
     local.status = rc;
     if (st) *st = local;
     return rc;

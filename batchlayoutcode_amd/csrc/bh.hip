@@ -49,7 +49,6 @@
 namespace bl {
 
 // out: 4 + 256 doubles, the sum in out[0] (minibatch.hip)
-int launch_energy(const double *eterm, int n, double *out, int precision, hipStream_t s);
 
 namespace {
 
@@ -2364,7 +2363,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     const int n = g->n;
     hipStream_t s = g->stream;
     double2 *pos = reinterpret_cast<double2 *>(d_xy);
-    if (g->eterm.ensure(sizeof(double) * (size_t)n) || g->energy.ensure(sizeof(double) * (4 + 256)) ||
+    if (g->eterm.ensure(sizeof(double) * (size_t)n) || g->energy.ensure(sizeof(EnergyOut)) ||
         g->scratch.ensure(sizeof(double2) * (size_t)n))
         return BL_E_NOMEM;
     int rc = ensure_bh(g->bh, n);
@@ -2540,7 +2539,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         prof.end();
         if (it == iters - 1) {  // only the last iteration's energy is returned
             prof.begin(2);
-            rc = launch_energy(g->eterm.as<double>(), n, g->energy.as<double>(), p->precision, s);
+            rc = launch_energy(g->eterm.as<double>(), pos, n, g->energy.as<EnergyOut>(), p->precision, s);
             prof.end();
             if (rc) return rc;
         }
@@ -2561,10 +2560,10 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         if (rc) return rc;
     }
     int status = 0;
-    double E = 1.79769313486231570815e+308;  // ENERGY starts at DBL_MAX (:1024)
+    EnergySeen seen{1.79769313486231570815e+308, 0.0, -1, 0};  // ENERGY starts at DBL_MAX (:1024)
     if (iters > 0) {
         BL_HIP(hipMemcpyAsync(&status, g->bh.misc.as<int>(), sizeof(int), hipMemcpyDeviceToHost, s));
-        BL_HIP(hipMemcpyAsync(&E, g->energy.as<double>(), sizeof(double), hipMemcpyDeviceToHost, s));
+        BL_HIP(hipMemcpyAsync(&seen, g->energy.p, sizeof(seen), hipMemcpyDeviceToHost, s));
     }
     int gerr = 0, werr = 0, waited = 0;
     if (g->bh.gwalk_used) BL_HIP(hipMemcpyAsync(&gerr, gwalk_err(g->bh), sizeof(int), hipMemcpyDeviceToHost, s));
@@ -2584,7 +2583,8 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         st->walk_lag = walk == BL_WALK_LAG ? lag_d : walk == BL_WALK_WIDE ? wide_d : 0;
         st->far_judge_err[0] = judge_err[0];
         st->far_judge_err[1] = judge_err[1];
-        st->energy = E;
+        st->energy = seen.energy;
+        st->nonfinite = seen.nonfinite;
         st->iters_done = iters;
         st->step_final = STEP;
     }

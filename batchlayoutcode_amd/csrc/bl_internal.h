@@ -268,6 +268,17 @@ inline void effective_neighbors(const int32_t *rowptr, const int32_t *colids, co
 }
 
 // minibatch.hip
+// What a run's end shows the host, in the graph's energy buffer (or the static workspace).
+constexpr int ENERGY_PARTS = 256;
+struct EnergySeen {
+    double energy, step;  // STEP of a captured graph
+    int nonfinite, pad;
+};
+struct EnergyOut : EnergySeen {
+    double share[ENERGY_PARTS];
+    int bad_share[ENERGY_PARTS];
+};
+int launch_energy(const double *eterm, const double2 *pos, int n, EnergyOut *out, int precision, hipStream_t s);
 // The number of the n positions that are not finite, counted on the device into *d_count (one
 // int of device memory) and returned in *h_count (waits for the stream).
 int count_nonfinite(const double2 *pos, int n, int *d_count, hipStream_t s, int *h_count);

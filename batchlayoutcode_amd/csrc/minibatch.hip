@@ -353,34 +353,56 @@ int count_nonfinite(const double2 *pos, int n, int *d_count, hipStream_t s, int 
 }
 
 // ---- energy reductions (shared with the Barnes-Hut path) -------------------------------
-// Fixed-order tree sum of |F_i|^2 (FP32 mode).
-// Energy sum_i |F_i|^2 in two fixed-order stages: ENERGY_PARTS workgroups each add a
-// contiguous share (threads strided, then a wave and workgroup reduction), then one wave adds
-// the shares in order.  Deterministic; out[0] = the sum, out[4 ..] = the shares.
-constexpr int ENERGY_PARTS = 256;
-
-__global__ __launch_bounds__(256) void k_energy_part(const double *__restrict__ eterm, int n, double *out) {
+// Energy sum_i |F_i|^2 (not FP64 mode's) and the number of positions that are not finite, in two
+// fixed-order stages: ENERGY_PARTS workgroups each add a contiguous share (threads strided, then a
+// wave and workgroup reduction), then one wave adds the shares in order.  Deterministic.  One copy
+// and one wait bring both to the host (EnergyOut); a count of its own took two more launches, a copy and
+// a wait, about 20 us of a run.
+__global__ __launch_bounds__(256) void k_energy_part(const double *__restrict__ eterm, const double2 *__restrict__ pos,
+                                                     int n, EnergyOut *out) {
     __shared__ double red[4];
+    __shared__ int bad[4];
     const int ch = (n + ENERGY_PARTS - 1) / ENERGY_PARTS;
     const int i0 = blockIdx.x * ch, i1 = min(n, i0 + ch);
     double a = 0.0, b = 0.0;
+    int k = 0;
+    auto count = [&](int i) {
+        const double2 p = pos[i];
+        k += isfinite(p.x) && isfinite(p.y) ? 0 : 1;
+    };
     int i = i0 + (int)threadIdx.x;
     for (; i + 256 < i1; i += 512) {
         a += eterm[i];
         b += eterm[i + 256];
+        count(i);
+        count(i + 256);
     }
-    if (i < i1) a += eterm[i];
+    if (i < i1) {
+        a += eterm[i];
+        count(i);
+    }
     a = wave_sum(a + b);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
+#pragma unroll
+    for (int off = 32; off; off >>= 1) k += __shfl_xor(k, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a, bad[threadIdx.x >> 6] = k;
     __syncthreads();
-    if (threadIdx.x == 0) out[4 + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (threadIdx.x == 0) {
+        out->share[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+        out->bad_share[blockIdx.x] = bad[0] + bad[1] + bad[2] + bad[3];
+    }
 }
 
-__global__ __launch_bounds__(64) void k_energy_final(double *out) {
+__global__ __launch_bounds__(64) void k_energy_final(EnergyOut *out) {
     double a = 0.0;
-    for (int k = threadIdx.x; k < ENERGY_PARTS; k += 64) a += out[4 + k];
+    int bad = 0;
+    for (int k = threadIdx.x; k < ENERGY_PARTS; k += 64) a += out->share[k], bad += out->bad_share[k];
     a = wave_sum(a);
-    if (threadIdx.x == 0) out[0] = a;
+#pragma unroll
+    for (int off = 32; off; off >>= 1) bad += __shfl_xor(bad, off, 64);
+    if (threadIdx.x == 0) {
+        out->energy = a;
+        out->nonfinite = bad;
+    }
 }
 
 // Sequential sum in vertex order, ENERGY += |F_i|^2 as the reference (FP64 mode): one wave adds a
@@ -420,14 +442,11 @@ __global__ __launch_bounds__(256) void k_energy_seq(const double *__restrict__ e
     if (threadIdx.x == 0) *out = e;
 }
 
-// out: 4 + ENERGY_PARTS doubles (the sum in out[0])
-int launch_energy(const double *eterm, int n, double *out, int precision, hipStream_t s) {
+int launch_energy(const double *eterm, const double2 *pos, int n, EnergyOut *out, int precision, hipStream_t s) {
+    hipLaunchKernelGGL(k_energy_part, dim3(ENERGY_PARTS), dim3(256), 0, s, eterm, pos, n, out);
+    hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(64), 0, s, out);
     if (precision == BL_PREC_FP64)
-        hipLaunchKernelGGL(k_energy_seq, dim3(1), dim3(256), 0, s, eterm, n, out);
-    else {
-        hipLaunchKernelGGL(k_energy_part, dim3(ENERGY_PARTS), dim3(256), 0, s, eterm, n, out);
-        hipLaunchKernelGGL(k_energy_final, dim3(1), dim3(64), 0, s, out);
-    }
+        hipLaunchKernelGGL(k_energy_seq, dim3(1), dim3(256), 0, s, eterm, n, &out->energy);
     BL_HIP(hipGetLastError());
     return BL_OK;
 }
@@ -520,11 +539,12 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
     const bool one = !fp64 && one_launch(n, bmax);
     const size_t a_elems = one ? (size_t)n : part_elems;  // the second position array in the partials' place
     double2 *part;
-    double *eterm, *energy;
+    double *eterm;
+    EnergyOut *energy;
     if (static_ws) {
         // [energy shares | partial forces | energy terms]; every word a step reads is written
         // earlier in the same step, so the contents of the previous call do not matter
-        static_assert(sizeof(double) * (4 + ENERGY_PARTS) <= 4096, "energy shares exceed their part");
+        static_assert(sizeof(EnergyOut) <= 4096, "energy shares exceed their part");
         const size_t off_part = 4096;
         const size_t off_eterm = off_part + round256(sizeof(double2) * std::max(a_elems, part_elems));
         const size_t need = off_eterm + round256(sizeof(double) * (size_t)n);
@@ -532,16 +552,16 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         unsigned char *ws = nullptr;
         const int rc = static_scratch(g->device, &ws);
         if (rc) return rc;
-        energy = reinterpret_cast<double *>(ws);
+        energy = reinterpret_cast<EnergyOut *>(ws);
         part = reinterpret_cast<double2 *>(ws + off_part);
         eterm = reinterpret_cast<double *>(ws + off_eterm);
     } else {
         if (g->part.ensure(sizeof(double2) * a_elems)) return BL_E_NOMEM;
         if (g->eterm.ensure(sizeof(double) * (size_t)n)) return BL_E_NOMEM;
-        if (g->energy.ensure(sizeof(double) * (4 + ENERGY_PARTS))) return BL_E_NOMEM;
+        if (g->energy.ensure(sizeof(EnergyOut))) return BL_E_NOMEM;
         part = g->part.as<double2>();
         eterm = g->eterm.as<double>();
-        energy = g->energy.as<double>();
+        energy = g->energy.as<EnergyOut>();
     }
 
     Prof prof;
@@ -550,9 +570,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
     const char *genv = getenv("BL_GRAPH");
     const bool want_graph = !prof.on && !static_ws && (converged || iters >= 2) && genv && !strcmp(genv, "1");
     double STEP = step0;
-    // energy[0] is the sum, energy[1] STEP for a captured graph (else a launch's argument), energy[4 ..]
-    // the sum's shares
-    double *const d_step = want_graph ? energy + 1 : nullptr;
+    double *const d_step = want_graph ? &energy->step : nullptr;  // else a launch's argument
     if (want_graph) hipLaunchKernelGGL(k_step_set, dim3(1), dim3(64), 0, s, d_step, step0);
     // One launch a step: the array that the next step reads, and the batch that the other one lacks.
     // The steps' number is known (or made even, each iteration) so that the last one writes pos.
@@ -632,7 +650,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         int rc = BL_OK;
         if (energy_seen) {
             prof.begin(2);
-            rc = launch_energy(eterm, n, energy, p->precision, s);
+            rc = launch_energy(eterm, pos, n, energy, p->precision, s);
             prof.end();
         }
         if (want_graph) hipLaunchKernelGGL(k_step_decay, dim3(1), dim3(64), 0, s, d_step, decay);
@@ -660,6 +678,7 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         if (gr) (void)hipGraphDestroy(gr);
         (void)hipGetLastError();  // a failed capture leaves the launches to the loop below
     }
+    EnergySeen seen;
     double E = 0.0, E0 = 1.79769313486231570815e+308;
     int loop = 0;
     for (;;) {
@@ -679,23 +698,25 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         STEP = STEP * decay;  // the host's copy (the device multiplies its own the same way)
         ++loop;
         if (converged) {
-            BL_HIP(hipMemcpyAsync(&E, energy, sizeof(double), hipMemcpyDeviceToHost, s));
+            BL_HIP(hipMemcpyAsync(&seen, energy, sizeof(seen), hipMemcpyDeviceToHost, s));
             BL_HIP(hipStreamSynchronize(s));
+            E = seen.energy;
         }
     }
     BL_HIP(hipGetLastError());
-    if (!converged && loop > 0) {
-        BL_HIP(hipMemcpyAsync(&E, energy, sizeof(double), hipMemcpyDeviceToHost, s));
-    }
+    if (!converged && loop > 0) BL_HIP(hipMemcpyAsync(&seen, energy, sizeof(seen), hipMemcpyDeviceToHost, s));
     BL_HIP(hipStreamSynchronize(s));
+    if (loop > 0) E = seen.energy;
     prof.report(st);
     if (st) {
         st->energy = loop > 0 ? E : (law == LAW_FR ? 0.0 : 1.79769313486231570815e+308);
         st->iters_done = loop;
         st->step_final = STEP;
-        if (static_ws) {  // the guard's counter in the energy block's spare word
+        if (loop > 0) {
+            st->nonfinite = seen.nonfinite;
+        } else if (static_ws) {  // nothing ran: counted here, in the energy block
             int nf = 0;
-            const int rc = count_nonfinite(pos, n, reinterpret_cast<int *>(energy + 3), s, &nf);
+            const int rc = count_nonfinite(pos, n, &energy->nonfinite, s, &nf);
             if (rc) return rc;
             st->nonfinite = nf;
         }
