@@ -1784,11 +1784,21 @@ __global__ __launch_bounds__(2 * WROW_T) void k_walk_row(const int *__restrict__
 constexpr int GW_T = 1024;
 constexpr int GW_G = 24;  // 8..32 measured on the R-MAT walk: 24 is fastest
 constexpr int GW_K = 4;  // entries per thread loaded a batch ahead
-// Measured times (us): a level of the walk by levels, on its own launch (5 to 25 with its size;
-// 5 where it decides) and in a run of small levels; a step of the lagged walk of 256 and of 512
-// vertices; a batch of the row walk.  The other walks take 4 us a batch or more, and there are never
-// more levels than batches.
-constexpr double LEVEL_US = 5.0, LEVEL_RUN_US = 2.3, LAG_US = 0.5, LAG512_US = 0.7, ROW_US = 2.2;
+// The times in us of an iteration's walk, by which the level walk is chosen where the row or the lagged
+// walk could run.  Measured (level / other walk, -batch 64 and 256):
+//   random geometric graph  4,000: 62 / 166 lagged, 52 / 48 row    30,000: 101 / 987, 94 / 475 lagged
+//   triangulation           3,400: 48 / 118 lagged, 39 / 35 row    48,000: 65 / 284, 65 / 514 lagged
+//   grid in row order       4,000: 86 / 55, 16 / 37 lagged         60,000: 347 / 492, 76 / 140 lagged
+// A level that is a launch takes 4 us, one in a run 1.2 and more with its vertices.  The lagged walk takes
+// 0.5 us a step (0.7 with 512 threads) only where the ids follow the edges, which makes many small levels;
+// without such an order, 1 to 4.
+inline double level_us(int n, int big, int small) {
+    return 6.0 + 4.0 * big + (1.2 + 8e-4 * n / (big + small + 1)) * small;
+}
+inline double row_us(int batches) { return 10.0 + 2.2 * batches; }
+inline double lag_us(int steps, int threads, bool ordered) {
+    return 22.0 + (!ordered ? 2.0 : threads == 512 ? 0.7 : 0.5) * steps;
+}
 constexpr int GW_MIN_ENTRIES = 4096;  // mean CSR entries per batch from which it is used
 
 struct GridWalk {
@@ -2410,13 +2420,12 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     bool use_level = p->precision != BL_PREC_FP64 && iters > 0 && !wenv && !getenv("BL_LAG_D") && !getenv("BL_LAG_H") &&
                      !getenv("BL_WIDE_D") && !getenv("BL_WIDE_H") && !(lenv && !strcmp(lenv, "0")) &&
                      level_walk_plan(g, p->batch, use_lag ? lag_d : 0);
-    // The lagged walk stays on graphs whose ids follow the edges: a 1000 x 1000 grid in row order at
-    // -batch 256 has 1,001 levels and 3,907 steps, 2.26 against 1.98 ms (at -batch 64: 2.27 against
-    // 7.84); without such an order 24 levels against 976 steps, 0.12 against 0.53 ms (250k random
-    // geometric graph).
+    // The lagged walk stays on graphs whose ids follow the edges with large batches (a 1000 x 1000 grid in
+    // row order at -batch 256: 1.98 ms against 2.26; at -batch 64 7.84 against 2.27), the row walk on
+    // those of few batches.
     if (use_level && (use_lag || use_row) && !lenv)
-        use_level = LEVEL_US * g->lev_big + LEVEL_RUN_US * g->lev_small <
-                    (!use_lag ? ROW_US * nbt : (lag_w == 512 ? LAG512_US : LAG_US) * lag_steps);
+        use_level = level_us(n, g->lev_big, g->lev_small) <
+                    (use_lag ? lag_us(lag_steps, lag_w, g->lev_small > 0) : row_us(nbt));
     if (!use_level) {
         if (use_wide) use_wide = wide_walk_fits(g, p->batch);
         if (use_wide) {
