@@ -514,8 +514,36 @@ __device__ __forceinline__ uint64_t cell_high(uint64_t k, int d) { return d == 0
 // the low end of quadrant v of the cell of level d < 32 that begins at low
 __device__ __forceinline__ uint64_t quadrant_low(uint64_t low, int d, int v) { return low + ((uint64_t)v << (62 - 2 * d)); }
 
-// boundary i (between Morton ranks i and i+1) is a node representative when it ends the
-// first quadrant of the cell where k_i and k_i+1 split
+// Boundary i (between Morton ranks i and i+1, keys a != b) is a node representative when it ends the
+// first quadrant of the cell where a and b split: when no key of the cell lies below a's quadrant.
+// Probes leftwards at distances 1, 3, 7, ... (the quadrant's keys are contiguous and most are few), then
+// a binary search for the key before the quadrant.
+__device__ __forceinline__ bool ends_first_quadrant(const uint64_t *keys, int i, uint64_t a, uint64_t b) {
+    const int d = level_of(a, b);
+    const uint64_t cell = cell_low(a, d), quad = cell_low(a, d + 1);
+    int hi = i, lo = i - 1;  // keys[hi] >= quad; keys[lo] < quad or lo < 0 in the end
+    uint64_t k = lo >= 0 ? keys[lo] : 0ull;
+    for (int step = 2; lo >= 0 && k >= quad; step <<= 1) {
+        hi = lo;
+        lo = hi - step;
+        k = keys[max(lo, 0)];
+    }
+    if (quad == cell) return true;
+    if (lo >= 0 && k >= cell) return false;
+    lo = max(lo, -1);
+    while (hi - lo > 1) {
+        const int m = (lo + hi) >> 1;
+        k = keys[m];
+        if (k >= quad) {
+            hi = m;
+        } else {
+            lo = m;
+            if (k >= cell) break;
+        }
+    }
+    return lo < 0 || keys[lo] < cell;
+}
+
 __global__ __launch_bounds__(WG) void k_tree_bounds(const uint64_t *__restrict__ keys, int n, int *__restrict__ isrep,
                                                     int *__restrict__ status) {
     const int i = xcd_tile(blockIdx.x, gridDim.x) * WG + threadIdx.x;
@@ -526,34 +554,203 @@ __global__ __launch_bounds__(WG) void k_tree_bounds(const uint64_t *__restrict__
         isrep[i] = 0;
         return;
     }
-    // a's quadrant is the cell's first when no key of the cell lies below it: probes leftwards at
-    // distances 1, 3, 7, ... (the quadrant's keys are contiguous and most are few), then a binary search
-    // for the key before the quadrant
-    const int d = level_of(a, b);
-    const uint64_t cell = cell_low(a, d), quad = cell_low(a, d + 1);
-    int hi = i, lo = i - 1;  // keys[hi] >= quad; keys[lo] < quad or lo < 0 in the end
-    uint64_t k = lo >= 0 ? keys[lo] : 0ull;
-    for (int step = 2; lo >= 0 && k >= quad; step <<= 1) {
-        hi = lo;
-        lo = hi - step;
-        k = keys[max(lo, 0)];
+    isrep[i] = ends_first_quadrant(keys, i, a, b) ? 1 : 0;
+}
+
+// Steps 1 to 5 as far as the node ids, for up to TREE_SMALL points: one workgroup, one launch instead of
+// 24 (3 of the frame and the keys, 18 of the sort, ties, boundaries, scan), which take 3 us each however
+// few the points.  Keys and ids stay in registers, element w * 64 R + 64 r + lane in round r of a wave's
+// lane; a pass of the LSD sort (8 bits) ranks them by ballots as k_sort_scatter,
+// counts digits per wave in LDS and exchanges them there.  Elements past n are keys of all ones, behind
+// every point by the sort's stability.  The tree of 300 points 102 -> 44 us, of 2,000 120 -> 57, of 4,000
+// 129 -> 76, of 8,100 135 -> 109 (one CU's operations).
+constexpr int TS_T = 1024, TS_W = TS_T / 64, TREE_SMALL = 8 * TS_T;
+constexpr size_t tree_small_lds(int rounds) { return (size_t)TS_T * rounds * 12 + 4 * TS_W * 256; }
+
+template <int R>
+__global__ __launch_bounds__(TS_T) void k_tree_small(const double2 *__restrict__ pos, int n, double *__restrict__ frame,
+                                                     uint64_t *__restrict__ keys, int *__restrict__ ids,
+                                                     double2 *__restrict__ spos, int *__restrict__ nodeid,
+                                                     int *__restrict__ list, int *__restrict__ total,
+                                                     int *__restrict__ misc, uint32_t *__restrict__ xs,
+                                                     uint32_t *__restrict__ ys) {
+    extern __shared__ __align__(16) uint64_t sk[];
+    int *sv = reinterpret_cast<int *>(sk + TS_T * R);
+    int *wrun = sv + TS_T * R;  // [wave][digit]
+    __shared__ double4 box[TS_W];
+    __shared__ int wsum[TS_W];
+    __shared__ int dup;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int e0 = w * 64 * R + lane;
+    double2 p[R];
+    double4 a = make_double4(INFINITY, -INFINITY, INFINITY, -INFINITY);  // minx maxx miny maxy
+#pragma unroll
+    for (int r = 0; r < R; ++r) p[r] = pos[min(e0 + 64 * r, n - 1)];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        a.x = fmin(a.x, p[r].x);
+        a.y = fmax(a.y, p[r].x);
+        a.z = fmin(a.z, p[r].y);
+        a.w = fmax(a.w, p[r].y);
     }
-    bool first = quad == cell || lo < 0 || k < cell;  // not yet known to hold a key of the cell below
-    if (quad != cell && first) {
-        lo = max(lo, -1);
-        while (hi - lo > 1) {
-            const int m = (lo + hi) >> 1;
-            k = keys[m];
-            if (k >= quad) {
-                hi = m;
-            } else {
-                lo = m;
-                if (k >= cell) break;
+    for (int off = 32; off; off >>= 1) {
+        a.x = fmin(a.x, __shfl_xor(a.x, off, 64));
+        a.y = fmax(a.y, __shfl_xor(a.y, off, 64));
+        a.z = fmin(a.z, __shfl_xor(a.z, off, 64));
+        a.w = fmax(a.w, __shfl_xor(a.w, off, 64));
+    }
+    if (lane == 0) box[w] = a;
+    if (tid == 0) dup = 0;
+    __syncthreads();
+    a = box[0];
+    for (int q = 1; q < TS_W; ++q) {
+        const double4 b = box[q];
+        a.x = fmin(a.x, b.x);
+        a.y = fmax(a.y, b.y);
+        a.z = fmin(a.z, b.z);
+        a.w = fmax(a.w, b.w);
+    }
+    const double dy = a.w - a.z, dx = a.y - a.x, mm = (dy < dx) ? dx : dy;
+    if (tid == 0) {
+        frame[0] = a.x;
+        frame[1] = a.z;
+        frame[2] = mm;
+    }
+    uint64_t k[R];
+    int v[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int e = e0 + 64 * r;
+        const uint32_t sx = scale32(p[r].x, a.x, mm), sy = scale32(p[r].y, a.z, mm);
+        k[r] = e < n ? (spread(sy) << 1) | spread(sx) : ~0ull;
+        v[r] = e;
+        if (xs && e < n) {
+            xs[e] = sx;
+            ys[e] = sy;
+        }
+    }
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    for (int shift = SORT_SKIP; shift < 64; shift += 8) {
+#pragma unroll
+        for (int q = 0; q < TS_W * 256; q += TS_T) wrun[q + tid] = 0;
+        __syncthreads();
+        int rk[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int d = (int)((k[r] >> shift) & 255u);
+            uint64_t peers = ~0ull;
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const bool bit = (d >> b) & 1;
+                const uint64_t bal = __ballot(bit);
+                peers &= bit ? bal : ~bal;
+            }
+            const int below = __popcll(peers & lt);
+            // every lane reads before the leaders write: one wave's LDS operations complete in order
+            const int before = wrun[w * 256 + d];
+            rk[r] = before + below;
+            if (below == 0) wrun[w * 256 + d] = before + __popcll(peers);
+        }
+        __syncthreads();
+        // thread t < 256 = digit: where each wave's keys of it begin
+        int tot = 0, x = 0;
+        if (tid < 256) {
+#pragma unroll
+            for (int q = 0; q < TS_W; ++q) tot += wrun[q * 256 + tid];
+            x = tot;
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const int y = __shfl_up(x, off, 64);
+                if (lane >= off) x += y;
+            }
+            if (lane == 63) wsum[w] = x;
+        }
+        __syncthreads();
+        if (tid < 256) {
+            int at = x - tot;
+            for (int q = 0; q < w; ++q) at += wsum[q];
+#pragma unroll
+            for (int q = 0; q < TS_W; ++q) {
+                const int c = wrun[q * 256 + tid];
+                wrun[q * 256 + tid] = at;
+                at += c;
             }
         }
-        first = lo < 0 || keys[lo] < cell;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int l = wrun[w * 256 + (int)((k[r] >> shift) & 255u)] + rk[r];
+            sk[l] = k[r];
+            sv[l] = v[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            k[r] = sk[e0 + 64 * r];
+            v[r] = sv[e0 + 64 * r];
+        }
     }
-    isrep[i] = first ? 1 : 0;
+    // runs of keys equal above the skipped bits, in full-key order (k_sort_ties)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = e0 + 64 * r;
+        const uint64_t h = k[r] >> SORT_SKIP;
+        if (i + 1 >= n || (sk[i + 1] >> SORT_SKIP) != h || (i > 0 && (sk[i - 1] >> SORT_SKIP) == h)) continue;
+        int end = i + 2;
+        while (end < n && (sk[end] >> SORT_SKIP) == h) ++end;
+        for (int x = i + 1; x < end; ++x) {
+            const uint64_t kx = sk[x];
+            const int vx = sv[x];
+            int b = x - 1;
+            for (; b >= i && sk[b] > kx; --b) {
+                sk[b + 1] = sk[b];
+                sv[b + 1] = sv[b];
+            }
+            sk[b + 1] = kx;
+            sv[b + 1] = vx;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int e = e0 + 64 * r;
+        if (e < n) {
+            const int id = sv[e];
+            keys[e] = sk[e];
+            ids[e] = id;
+            spos[e] = pos[id];
+        }
+    }
+    // the representative boundaries, numbered: R consecutive ones a thread
+    unsigned rep = 0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int i = tid * R + q;
+        if (i < n - 1) {
+            const uint64_t ka = sk[i], kb = sk[i + 1];
+            if (ka == kb) dup = 1;
+            else rep |= (ends_first_quadrant(sk, i, ka, kb) ? 1u : 0u) << q;
+        }
+    }
+    int x = __popc(rep);
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
+    }
+    __syncthreads();  // wsum has been read; dup is set
+    if (lane == 63) wsum[w] = x;
+    __syncthreads();
+    int run = x - __popc(rep);
+    for (int q = 0; q < w; ++q) run += wsum[q];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int i = tid * R + q;
+        if (i < n - 1) nodeid[i] = run;
+        if (rep >> q & 1) list[run++] = i;
+    }
+    if (tid == TS_T - 1) *total = run;
+    if (tid < 4) misc[tid] = tid == 0 && dup ? ST_DUPKEY : 0;
 }
 
 // N searches in step (lower_bound of BarnesHut.h:143-146): lo[q] = the first index in [lo[q], hi[q])
@@ -2166,30 +2363,24 @@ int ensure_bh(BHWork &w, int n) {
     return BL_OK;
 }
 
-// Builds the tree of the positions d_pos (device, n points) into w; returns BL_OK and
-// leaves the status word in misc[0] (checked by the caller when it needs it).  centroids: the
-// unweighted centroids of algo 4's traversal (the far-field modes summarise cells themselves).
-int build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t *d_xs, uint32_t *d_ys,
-               bool centroids = true) {
-    int rc = ensure_bh(w, n);
-    if (rc) return rc;
+// Steps 1 to 4: the points in Morton order (keys_a, idx_a, spos), for any n.
+int sort_points(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t *d_xs, uint32_t *d_ys) {
     int *misc = w.misc.as<int>();
     double *frame = w.frame.as<double>();
     double4 *fpart = reinterpret_cast<double4 *>(frame + 8);
+    const int g1 = (n + WG - 1) / WG;
     BL_HIP(hipMemsetAsync(misc, 0, 16, s));
     const int gf = std::min(1024, (n + WG - 1) / WG);
     hipLaunchKernelGGL(k_frame_partial, dim3(gf), dim3(WG), 0, s, d_pos, n, fpart);
     hipLaunchKernelGGL(k_frame_final, dim3(1), dim3(WG), 0, s, fpart, gf, frame);
     uint64_t *ka = w.keys_a.as<uint64_t>(), *kb = w.keys_b.as<uint64_t>();
     int *ia = w.idx_a.as<int>(), *ib = w.idx_b.as<int>();
-    const int g1 = (n + WG - 1) / WG;
     hipLaunchKernelGGL(k_keys, dim3(g1), dim3(WG), 0, s, d_pos, n, frame, ka, ia, d_xs, d_ys);
     const int rounds = SORT_ROUNDS;
     const int nblk = (n + WG * rounds - 1) / (WG * rounds);
     double2 *spos = w.spos.as<double2>();
     int *hist = w.hist.as<int>();
     int *dtot = w.scan_tmp.as<int>();
-    int *bsum = misc + 64;
     for (int pass = SORT_SKIP / 8; pass < 8; ++pass) {
         const int shift = 8 * pass;
         hipLaunchKernelGGL(k_sort_hist, dim3(nblk), dim3(WG), 0, s, ka, n, shift, nblk, rounds, hist);
@@ -2207,14 +2398,47 @@ int build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t *
     // the keys' top 48 bits; runs of keys equal in those bits are put in full-key order here
     static_assert((8 - SORT_SKIP / 8) % 2 == 0, "an even number of passes ends in keys_a");
     if (n >= 2) hipLaunchKernelGGL(k_sort_ties, dim3(g1), dim3(WG), 0, s, ka, ia, spos, n);
-    if (n >= 2) {
-        int *isrep = w.isrep.as<int>(), *nodeid = w.nodeid.as<int>();
-        BHNode *nodes = w.node_child.as<BHNode>();
-        hipLaunchKernelGGL(k_tree_bounds, dim3(g1), dim3(WG), 0, s, ka, n, isrep, misc);
-        int *list = w.idx_b.as<int>();  // free after the sort
-        rc = scan_excl(isrep, n - 1, nodeid, list, bsum, s);
+    BL_HIP(hipGetLastError());
+    return BL_OK;
+}
+
+// Builds the tree of the positions d_pos (device, n points) into w; returns BL_OK and
+// leaves the status word in misc[0] (checked by the caller when it needs it).  centroids: the
+// unweighted centroids of algo 4's traversal (the far-field modes summarise cells themselves).
+int build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t *d_xs, uint32_t *d_ys,
+               bool centroids = true) {
+    int rc = ensure_bh(w, n);
+    if (rc) return rc;
+    int *misc = w.misc.as<int>();
+    double *frame = w.frame.as<double>();
+    const int g1 = (n + WG - 1) / WG;
+    uint64_t *ka = w.keys_a.as<uint64_t>();
+    int *ia = w.idx_a.as<int>();
+    double2 *spos = w.spos.as<double2>();
+    int *bsum = misc + 64, *nodeid = w.nodeid.as<int>();
+    int *list = w.idx_b.as<int>();  // free after the sort
+    const int nsb = (n - 1 + SCAN_TILE - 1) / SCAN_TILE;
+    const char *tenv = getenv("BL_TREE_SMALL");  // 0: the general path (tests)
+    const bool small = n <= TREE_SMALL && !(tenv && !strcmp(tenv, "0"));
+    if (small) {
+        const int rounds = n <= 2 * TS_T ? 2 : n <= 4 * TS_T ? 4 : 8;
+        const auto kernel = rounds == 2 ? k_tree_small<2> : rounds == 4 ? k_tree_small<4> : k_tree_small<8>;
+        BL_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)tree_small_lds(rounds)));
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(TS_T), tree_small_lds(rounds), s, d_pos, n, frame, ka, ia, spos,
+                           nodeid, list, bsum + nsb, misc, d_xs, d_ys);
+    } else {
+        rc = sort_points(w, d_pos, n, s, d_xs, d_ys);
         if (rc) return rc;
-        const int nsb = (n - 1 + SCAN_TILE - 1) / SCAN_TILE;
+    }
+    if (n >= 2) {
+        int *isrep = w.isrep.as<int>();
+        BHNode *nodes = w.node_child.as<BHNode>();
+        if (!small) {
+            hipLaunchKernelGGL(k_tree_bounds, dim3(g1), dim3(WG), 0, s, ka, n, isrep, misc);
+            rc = scan_excl(isrep, n - 1, nodeid, list, bsum, s);
+            if (rc) return rc;
+        }
         int *npts = w.node_cnt.as<int>();
         hipLaunchKernelGGL(k_tree_nodes, dim3(g1), dim3(WG), 0, s, ka, n, list, nodeid, bsum + nsb, nodes,
                            npts, w.node_lo.as<int>(), misc, misc);
