@@ -1009,7 +1009,7 @@ struct Frame {
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Mixed mode (the default).  One wave per 64 Morton-consecutive vertices and one stack of nodes
+// Mixed mode (the default).  One wave per `per` (wave_points) Morton-consecutive vertices and one stack of nodes
 // (traverse.h).  The opening test D/|c - v| < theta (BarnesHut.h:71-72) is decided by the squares,
 // except within 2^-40 of equality, where the caller evaluates it as it stands for the whole node, so
 // the accepted set is the reference's.  Unit vectors d/|d| by the FP32 reciprocal square root refined
@@ -1020,11 +1020,11 @@ __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlan
 __global__ __launch_bounds__(WG) void k_rep(const double2 *__restrict__ qpos, const int *__restrict__ qid, int n,
                                             const double2 *__restrict__ spos, const BHNode *__restrict__ nodes,
                                             const int *__restrict__ misc, const double *__restrict__ frame,
-                                            double theta, double2 *__restrict__ rep, const int *__restrict__ status) {
+                                            double theta, double2 *__restrict__ rep, const int *__restrict__ status, int per) {
     if (*status) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int k = (xcd_tile(blockIdx.x, gridDim.x) * (WG / 64) + w) * 64 + lane;
-    const bool valid = k < n;
+    const int k = (xcd_tile(blockIdx.x, gridDim.x) * (WG / 64) + w) * per + lane;
+    const bool valid = lane < per && k < n;
     const uint64_t m0 = __ballot(valid);
     if (m0 == 0) return;
     const int root = misc[1];
@@ -1115,13 +1115,13 @@ __global__ __launch_bounds__(WG) void k_rep32(const double2 *__restrict__ qpos, 
                                               const double2 *__restrict__ spos,
                                               const BHNode *__restrict__ nodes, const int *__restrict__ misc,
                                               const double *__restrict__ frame, double theta,
-                                              double2 *__restrict__ rep, const int *__restrict__ status) {
+                                              double2 *__restrict__ rep, const int *__restrict__ status, int per) {
     __shared__ int stk_node[WG / 64][STACK];
     __shared__ uint64_t stk_mask[WG / 64][STACK];
     if (*status) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int k = (xcd_tile(blockIdx.x, gridDim.x) * (WG / 64) + w) * 64 + lane;
-    const bool valid = k < n;
+    const int k = (xcd_tile(blockIdx.x, gridDim.x) * (WG / 64) + w) * per + lane;
+    const bool valid = lane < per && k < n;
     const double2 p = qpos[valid ? k : n - 1];
     const double maxmin = frame[2];
     const float th2 = (float)(theta * theta);
@@ -2456,8 +2456,8 @@ int build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t *
 }
 
 int launch_rep(BHWork &w, int n, double theta, int precision, hipStream_t s) {
-    const int waves = (n + 63) / 64;
-    const int g = (waves + WG / 64 - 1) / (WG / 64);
+    const int per = precision == BL_PREC_FP64 ? 64 : wave_points(n);
+    const int g = (n + per * (WG / 64) - 1) / (per * (WG / 64));
     if (precision == BL_PREC_FP64)
         hipLaunchKernelGGL(k_rep64, dim3(g), dim3(WG), 0, s, w.spos.as<double2>(), w.idx_a.as<int>(), n,
                            w.spos.as<double2>(), w.node_child.as<BHNode>(), w.misc.as<int>(), w.frame.as<double>(), theta,
@@ -2465,7 +2465,7 @@ int launch_rep(BHWork &w, int n, double theta, int precision, hipStream_t s) {
     else
         hipLaunchKernelGGL(precision == BL_PREC_FP32 ? k_rep32 : k_rep, dim3(g), dim3(WG), 0, s,
                            w.spos.as<double2>(), w.idx_a.as<int>(), n, w.spos.as<double2>(), w.node_child.as<BHNode>(),
-                           w.misc.as<int>(), w.frame.as<double>(), theta, w.rep.as<double2>(), w.misc.as<int>());
+                           w.misc.as<int>(), w.frame.as<double>(), theta, w.rep.as<double2>(), w.misc.as<int>(), per);
     BL_HIP(hipGetLastError());
     return BL_OK;
 }
@@ -2915,8 +2915,8 @@ int bh_forces_host(int32_t n, const double *xy, double theta, int32_t nq, const 
     std::vector<int> ids(nq);
     for (int k = 0; k < nq; ++k) ids[k] = k;
     BL_HIP(hipMemcpyAsync(qid, ids.data(), 4 * (size_t)nq, hipMemcpyHostToDevice, sc.s));
-    const int waves = (nq + 63) / 64;
-    const int gq = (waves + WG / 64 - 1) / (WG / 64);
+    const int per = precision == BL_PREC_FP64 ? 64 : wave_points(nq);
+    const int gq = (nq + per * (WG / 64) - 1) / (per * (WG / 64));
     BHWork &w = sc.w;
     if (precision == BL_PREC_FP64)
         hipLaunchKernelGGL(k_rep64, dim3(gq), dim3(WG), 0, sc.s, dq, qid, nq, w.spos.as<double2>(), w.node_child.as<BHNode>(),
@@ -2924,7 +2924,7 @@ int bh_forces_host(int32_t n, const double *xy, double theta, int32_t nq, const 
     else
         hipLaunchKernelGGL(precision == BL_PREC_FP32 ? k_rep32 : k_rep, dim3(gq), dim3(WG), 0, sc.s, dq,
                            qid, nq, w.spos.as<double2>(), w.node_child.as<BHNode>(), w.misc.as<int>(),
-                           w.frame.as<double>(), theta, dout, w.misc.as<int>());
+                           w.frame.as<double>(), theta, dout, w.misc.as<int>(), per);
     BL_HIP(hipGetLastError());
     int status = 0;
     BL_HIP(hipMemcpyAsync(&status, w.misc.p, sizeof(int), hipMemcpyDeviceToHost, sc.s));

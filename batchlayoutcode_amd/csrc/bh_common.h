@@ -2,6 +2,8 @@
 // farfield.hip reads it).
 #pragma once
 
+#include <stdlib.h>
+
 #include "bl_internal.h"
 
 namespace bl {
@@ -49,6 +51,24 @@ __device__ __forceinline__ void store_through(double2 *p, double2 v) {
 }
 __device__ __forceinline__ void store_through(int *p, int v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Points a wave of a traversal takes: 64 where that makes enough waves for the chip (4 on each of its 1,024
+// SIMDs), else as few as 8.  A wave visits the nodes that any of its points needs, so fewer points make it
+// shorter, and the waves that then run side by side cost nothing while SIMDs are idle.  Traversal in us
+// with 64 / 32 / 16 / 8 points a wave (random geometric graph; algo 4 at theta 1.2, far field at theta 0.4):
+//   1,000: 54 / 45 / 34 / 26, 85 / 76 / 62 / 56           40,000: 76 / 61 / 53 / 50, 190 / 186 / 171 / 172
+//  10,000: 69 / 52 / 40 / 37, 151 / 126 / 105 / 110      120,000: 92 / 77 / 88 / 109, 242 / 233 / 315 / 468
+// 200,000: 102 / 107 / 125 / 168, 275 / 345 / 474 / 722
+// A point's sums don't depend on it: it meets its own nodes in the same order.
+inline int wave_points(int n) {
+    if (const char *e = getenv("BL_WAVE_POINTS")) {  // tests
+        const int per = atoi(e);
+        if (per == 8 || per == 16 || per == 32 || per == 64) return per;
+    }
+    int per = 8;
+    while (per < 64 && n > 4096 * per) per <<= 1;
+    return per;
 }
 
 // Agent-scope loads: what store_through stored, once its completion is known, without an acquire.

@@ -365,7 +365,7 @@ __global__ __launch_bounds__(WG) void k_far_trav(const double2 *__restrict__ qpo
                                                  const int *__restrict__ misc, const double *__restrict__ frame,
                                                  double theta, const float *__restrict__ model,
                                                  double2 *__restrict__ out, unsigned long long *ncells,
-                                                 const int *use_model, int *model_iters) {
+                                                 const int *use_model, int *model_iters, int per) {
     // learned mode: the model and the per-wave queues in dynamic LDS (LEARNED_LDS bytes)
     extern __shared__ __align__(16) unsigned char dyn[];
     MlpLds *L = reinterpret_cast<MlpLds *>(dyn);
@@ -382,8 +382,8 @@ __global__ __launch_bounds__(WG) void k_far_trav(const double2 *__restrict__ qpo
         __syncthreads();
     }
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int k = (xcd_tile(blockIdx.x, gridDim.x) * (WG / 64) + w) * 64 + lane;
-    const bool valid = k < nq && qid[k] >= 0;  // a negative id: an idle lane (the judge's sample)
+    const int k = (xcd_tile(blockIdx.x, gridDim.x) * (WG / 64) + w) * per + lane;
+    const bool valid = lane < per && k < nq && qid[k] >= 0;  // a negative id: an idle lane (the judge's sample)
     const double2 p = qpos[valid ? k : nq - 1];
     double fx = 0.0, fy = 0.0;
     const int root = misc[1];
@@ -581,21 +581,22 @@ __global__ __launch_bounds__(WG) void k_far_exact(const double2 *__restrict__ qp
 int launch_trav(BHWork &w, const double2 *qpos, const int *qid, int nq, double theta, int mode, const float *model,
                 double2 *out, hipStream_t s, unsigned long long *ncells = nullptr, const int *use_model = nullptr,
                 int *model_iters = nullptr) {
-    const int g64 = ((nq + 63) / 64 + WG / 64 - 1) / (WG / 64);
+    const int per = mode == FAR_LEARNED ? 64 : wave_points(nq);  // the model's batches take a wave's 64 lanes
+    const int g = (nq + per * (WG / 64) - 1) / (per * (WG / 64));
     const BHNode *nodes = w.node_child.as<BHNode>();
     const FarCell *cells = w.far_cells.as<FarCell>();
     const int *misc = w.misc.as<int>();
     const double2 *spos = w.spos.as<double2>();
     const double *frame = w.frame.as<double>();
     if (mode == FAR_MONO)
-        hipLaunchKernelGGL(k_far_trav<TRAV_MONO>, dim3(g64), dim3(WG), 0, s, qpos, qid, nq, spos, nodes, cells, misc,
-                           frame, theta, model, out, ncells, use_model, model_iters);
+        hipLaunchKernelGGL(k_far_trav<TRAV_MONO>, dim3(g), dim3(WG), 0, s, qpos, qid, nq, spos, nodes, cells, misc,
+                           frame, theta, model, out, ncells, use_model, model_iters, per);
     else if (mode == FAR_QUAD)
-        hipLaunchKernelGGL(k_far_trav<TRAV_QUAD>, dim3(g64), dim3(WG), 0, s, qpos, qid, nq, spos, nodes, cells, misc,
-                           frame, theta, model, out, ncells, use_model, model_iters);
+        hipLaunchKernelGGL(k_far_trav<TRAV_QUAD>, dim3(g), dim3(WG), 0, s, qpos, qid, nq, spos, nodes, cells, misc,
+                           frame, theta, model, out, ncells, use_model, model_iters, per);
     else if (mode == FAR_LEARNED && model)
-        hipLaunchKernelGGL(k_far_trav<TRAV_LEARNED>, dim3(g64), dim3(WG), LEARNED_LDS, s, qpos, qid, nq, spos, nodes, cells,
-                           misc, frame, theta, model, out, ncells, use_model, model_iters);
+        hipLaunchKernelGGL(k_far_trav<TRAV_LEARNED>, dim3(g), dim3(WG), LEARNED_LDS, s, qpos, qid, nq, spos, nodes, cells,
+                           misc, frame, theta, model, out, ncells, use_model, model_iters, per);
     else
         return BL_E_ARG;
     BL_HIP(hipGetLastError());
