@@ -8,8 +8,8 @@
 // Results.txt row.  Layouts run on the GPU through libbatchlayout.so.
 //
 // Build-only flags use a prefix the reference never parses:
-//   --gpu-precision mixed|fp32|fp64   pair arithmetic (default mixed: FP64 with an FP32-seeded
-//                               reciprocal; fp32: FP32 |d|^2 and reciprocal; fp64: the
+//   --gpu-precision mixed|fp32|fp64   pair arithmetic (default mixed: FP64, one reciprocal
+//                               for eight pairs; fp32: FP32 |d|^2 and reciprocal; fp64: the
 //                               reference's FP64 operation order)
 // Algorithms 0, 1, 5 and 7 (sequential / naive / greedy / algebraic baselines of the
 // reference) are not provided by this build; they exit with status 1 and a message.

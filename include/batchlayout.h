@@ -60,8 +60,8 @@ extern "C" {
 #define BL_ALGO_FAR_QUAD 43  /* monopoles corrected by the analytic second-order multipole term */
 
 /* ---- precision of the pair arithmetic -------------------------------------------- */
-#define BL_PREC_MIXED 0      /* default: FP64 differences and sums; 1/|d|^2 seeded by the FP32
-                                reciprocal and refined by one FP64 Newton step (FP64-grade terms) */
+#define BL_PREC_MIXED 0      /* default: FP64 differences and sums; 1/|d|^2 in FP64, one reciprocal
+                                (hardware estimate and a Newton step) for eight pairs */
 #define BL_PREC_FP64 1       /* reference-grade path: the reference's FP64 operations in its order */
 #define BL_PREC_FP32 2       /* fastest: |d|^2 and 1/|d|^2 in FP32, FP64 differences and sums */
 
