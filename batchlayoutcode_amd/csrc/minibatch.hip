@@ -646,6 +646,9 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
         if (one && even_out && cur) {  // the last step wrote the other array: its batch is what pos lacks
             hipLaunchKernelGGL(k_copy, dim3((pc + WG - 1) / WG), dim3(WG), 0, s, part + p0, pos + p0, pc);
             cur = pc = 0;
+        } else if (one && want_graph) {  // a replay begins with both arrays complete, as the captured iteration
+            hipLaunchKernelGGL(k_copy, dim3((pc + WG - 1) / WG), dim3(WG), 0, s, pos + p0, part + p0, pc);
+            pc = 0;
         }
         int rc = BL_OK;
         if (energy_seen) {

@@ -1,7 +1,7 @@
 """The one-launch batch step of small graphs: against the oracle to 1e-4 of the diameter after one iteration
 (as the two-launch step), and through its two position arrays (odd and even numbers of steps, a batch that
-holds the whole graph, a last batch of one, the static workspace, a stop by convergence) bit for bit the
-same as iteration by iteration."""
+holds the whole graph, a last batch of one, the static workspace, a stop by convergence, replays of a
+captured iteration) bit for bit the same as iteration by iteration."""
 import numpy as np
 import pytest
 import torch
@@ -39,6 +39,10 @@ def test_one_launch_a_step(bl, oracle, n, batch, monkeypatch):
                 conv, stc = g.run(x0, converged=1, engt=0.5, **kw)
                 fixed, stf = g.run(x0, iters=int(stc.iters_done), **kw)
                 assert np.array_equal(conv, fixed) and stc.energy == stf.energy
+            monkeypatch.setenv("BL_GRAPH", "1")  # one iteration captured, three replays of it
+            xg, stg = g.run(x0, iters=3, **kw)
+            monkeypatch.delenv("BL_GRAPH")
+            assert np.array_equal(xg, xy) and stg.energy == st3.energy
             monkeypatch.setenv("BL_STEP_LAUNCHES", "2")
             two, st2 = g.run(x0, iters=1, **kw)
             monkeypatch.delenv("BL_STEP_LAUNCHES")
