@@ -184,7 +184,7 @@ extern "C" int bl_graph_destroy(bl_graph *g) {
     for (DevBuf *b : all) b->release();
     g->lev_early.release();
     g->lev_late.release();
-    g->lev_start.release();
+    for (DevBuf *b : {&g->lev_start, &g->lev_blk, &g->lev_shape, &g->lev_moved, &g->lev_ticket}) b->release();
     g->bh.release();
     if (g->stream) (void)hipStreamDestroy(g->stream);
     delete g;

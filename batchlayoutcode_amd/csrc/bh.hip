@@ -1983,14 +1983,14 @@ constexpr int GW_G = 24;  // 8..32 measured on the R-MAT walk: 24 is fastest
 constexpr int GW_K = 4;  // entries per thread loaded a batch ahead
 // The times in us of an iteration's walk, by which the level walk is chosen where the row or the lagged
 // walk could run.  Measured (level / other walk, -batch 64 and 256):
-//   random geometric graph  4,000: 62 / 166 lagged, 52 / 48 row    30,000: 101 / 987, 94 / 475 lagged
-//   triangulation           3,400: 48 / 118 lagged, 39 / 35 row    48,000: 65 / 284, 65 / 514 lagged
-//   grid in row order       4,000: 86 / 55, 16 / 37 lagged         60,000: 347 / 492, 76 / 140 lagged
-// A level that is a launch takes 4 us, one in a run 1.2 and more with its vertices.  The lagged walk takes
-// 0.5 us a step (0.7 with 512 threads) only where the ids follow the edges, which makes many small levels;
-// without such an order, 1 to 4.
+//   random geometric graph  4,000: 37 / 169 lagged, 31 / 47 row    30,000: 60 / 939, 58 / 454 lagged
+//   triangulation           3,400: 30 / 119 lagged, 26 / 36 row    25,000: 39 / 200, 38 / 279 lagged
+//   grid in row order       4,000: 85 / 56, 13 / 36 lagged         30,000: 228 / 259, 16 / 80 lagged
+// A launch of levels takes 4 us and 1.9 a level, a level in a run 1.2 and more with its vertices.  The lagged
+// walk takes 0.5 us a step (0.7 with 512 threads) only where the ids follow the edges, which makes many small
+// levels; without such an order, 1 to 4.
 inline double level_us(int n, int big, int small) {
-    return 6.0 + 4.0 * big + (1.2 + 8e-4 * n / (big + small + 1)) * small;
+    return 6.0 + (big ? 4.0 + 1.9 * big : 0.0) + (1.2 + 8e-4 * n / (big + small + 1)) * small;
 }
 inline double row_us(int batches) { return 10.0 + 2.2 * batches; }
 inline double lag_us(int steps, int threads, bool ordered) {
@@ -2645,7 +2645,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
                      !getenv("BL_WIDE_D") && !getenv("BL_WIDE_H") && !(lenv && !strcmp(lenv, "0")) &&
                      level_walk_plan(g, p->batch, use_lag ? lag_d : 0);
     // The lagged walk stays on graphs whose ids follow the edges with large batches (a 1000 x 1000 grid in
-    // row order at -batch 256: 1.98 ms against 2.26; at -batch 64 7.84 against 2.27), the row walk on
+    // row order at -batch 256: 1.99 ms against 2.19; at -batch 64 7.85 against 2.17), the row walk on
     // those of few batches.
     if (use_level && (use_lag || use_row) && !lenv)
         use_level = level_us(n, g->lev_big, g->lev_small) <
@@ -2718,7 +2718,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         if (rc) return rc;
         if (use_level) {
             prof.begin(5);
-            rc = launch_level_late(g, pos, p, s);
+            rc = launch_level_late(g, pos, p, it, s);
             prof.end();
             if (rc) return rc;
         } else if (p->precision != BL_PREC_FP64 && !use_grid && use_row) {
@@ -2792,17 +2792,18 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         rc = far_judge_read(g->bh, &model_iters, judge_err, s);
         if (rc) return rc;
     }
-    int status = 0;
+    int misc[BH_LEVEL_ERR + 1] = {};  // the status word and the level walk's
     EnergySeen seen{1.79769313486231570815e+308, 0.0, -1, 0};  // ENERGY starts at DBL_MAX (:1024)
     if (iters > 0) {
-        BL_HIP(hipMemcpyAsync(&status, g->bh.misc.as<int>(), sizeof(int), hipMemcpyDeviceToHost, s));
+        BL_HIP(hipMemcpyAsync(misc, g->bh.misc.as<int>(), sizeof(misc), hipMemcpyDeviceToHost, s));
         BL_HIP(hipMemcpyAsync(&seen, g->energy.p, sizeof(seen), hipMemcpyDeviceToHost, s));
     }
     int gerr = 0, werr = 0, waited = 0;
     if (g->bh.gwalk_used) BL_HIP(hipMemcpyAsync(&gerr, gwalk_err(g->bh), sizeof(int), hipMemcpyDeviceToHost, s));
     if (walk == BL_WALK_WIDE && !use_level && (rc = wide_walk_read(g, &werr, &waited, s))) return rc;
     BL_HIP(hipStreamSynchronize(s));
-    if (status & ST_DUPKEY) return BL_E_DUPKEY;
+    if (misc[0] & ST_DUPKEY) return BL_E_DUPKEY;
+    if (use_level && g->lev_big && misc[BH_LEVEL_ERR]) return BL_E_DEVICE;  // a wait for a position timed out
     if (gerr) return BL_E_DEVICE;  // a grid barrier timed out (the walk stopped early)
     if (werr) {  // a wait of the wide walk timed out: its chunk counts are incomplete
         (void)wide_walk_reset(g);

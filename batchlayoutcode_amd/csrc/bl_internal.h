@@ -61,10 +61,10 @@ struct LevelLists {
         for (DevBuf *b : {&head, &vid, &ids, &w, &row, &rids, &rw}) b->release();
     }
 };
-// One launch: levels [l0, l1) of slices from vertex slot v0 and entry block e0, or one level (l1 ==
-// l0): nn waves of rows of 4 lanes, nw of 8, then from row r0 nr rows of a wave and nh of a workgroup.
+// One launch: levels [l0, l1) of slices from vertex slot v0 and entry block e0 by one workgroup, or
+// `blocks` workgroups (> 0) of `levels` consecutive levels, each workgroup's level listed from b0.
 struct LevelLaunch {
-    int32_t l0, l1, v0, nn, nw, r0, nr, nh;
+    int32_t l0, l1, v0, b0, blocks, levels;
     uint32_t e0;
 };
 
@@ -122,7 +122,7 @@ struct bl_graph {
             lev_late_hubs = 0;
     bool lev_ok = false;
     bl::LevelLists lev_early, lev_late;
-    bl::DevBuf lev_start;
+    bl::DevBuf lev_start, lev_blk, lev_shape, lev_moved, lev_ticket;
     std::vector<bl::LevelLaunch> lev_launch;
     // the neighbours the reference's merge pointer actually meets (algorithms.cpp:758-762),
     // as a CSR of strictly increasing column ids per row (+ their weights)

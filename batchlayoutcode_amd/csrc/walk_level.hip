@@ -13,26 +13,30 @@
 //
 //   f_i = (sum over early, in list order) - rep'_i,    rep'_i = rep_i - sum over late
 //
-// What bounds a small level is its launch and its chain of dependent loads, about 5 us together, not
-// its arithmetic; a large one is bound by its random 16-byte reads and writes (25 us for 200k
-// vertices).  So a level's rows are laid out for two round trips, the vertices with their entries
-// and then every position these name:
+// Consecutive levels are one launch (k_level_flow).  Nothing but the new positions orders them: before the
+// walk every vertex's entry of `moved` is marked as not there, a move stores its vertex's, and whoever
+// needs it reads it until it has come.  So a level costs one store and one load through memory, about
+// 2.4 us, where a launch of its own cost 5 (two dependent loads past caches that a launch leaves empty, the
+// dispatch, the write-back), and the next levels' rows are loaded while they wait.  Workgroups take their
+// level and place in it by a ticket in level order: what a workgroup waits for was given to one that
+// started before it, so some workgroup can always go on.  Eight counters, one for each residue of the
+// workgroup's number (workgroups start in order on each XCD): with a single one the tickets themselves took
+// 13 ns each, 215 us on the triangulation.  A wait ends at a deadline, and the run with an error.
 //   - rows of up to 4 entries take 4 lanes each, rows of up to 8 take 8, at an address that the lane's
 //     number gives: a lane forms the factors of one entry, and the lanes' products are added one after
 //     another by DPP moves;
-//   - rows of up to LV_WAVE entries one a wave, longer ones (hubs) one a workgroup, the row's header
-//     first.
-// One lane an entry also keeps the code short: with one lane a row, eight terms unrolled, a level
-// waited longer for its instructions (cold after every launch) than for its data (10 us against 5
-// for the small levels of the triangulation).
-// A level of more than LV_RUN vertices, or with a row beyond 8 entries, is one launch.  Runs of
-// smaller levels are one launch of one workgroup, which takes the levels one after another with a
-// barrier between them and loads a level's vertices and entries two levels ahead.
+//   - rows of up to LV_WAVE entries one a wave, longer ones (hubs) one a workgroup.
+// What bounds the walk: on R-MAT the hand-off of 188 levels; on the triangulation random 16-byte reads and
+// writes (1.66M moves in 195 us).  k_level_flow against a launch a level: R-MAT scale 20 at -batch 1024
+// 989 -> 462 us, 250k random geometric graph 111 -> 65, triangulation 215 -> 195.
+// Runs of levels of at most LV_RUN vertices without rows beyond 8 entries are one launch of one
+// workgroup, which takes the levels one after another with a barrier between them (1.2 to 3 us each) and
+// loads a level's vertices and entries two levels ahead.
 //
 // Walk per iteration, with the late sums, before and after: triangulation of 1.66M points at -batch
-// 256 2.65 -> 0.28 ms (lagged walk), 250k random geometric graph 0.54 -> 0.13 ms (lagged walk),
-// R-MAT scale 20 at -batch 1024 2.07 -> 1.09 ms (wide walk), a 1000 x 1000 grid in row order at
-// -batch 64 7.84 -> 2.29 ms (lagged walk) and at -batch 1024 5.20 -> 0.15 ms (entry-split walk).
+// 256 2.65 -> 0.28 ms (lagged walk), 250k random geometric graph 0.54 -> 0.08 ms (lagged walk),
+// R-MAT scale 20 at -batch 1024 2.07 -> 0.56 ms (wide walk), a 1000 x 1000 grid in row order at
+// -batch 64 7.84 -> 2.17 ms (lagged walk) and at -batch 1024 5.20 -> 0.08 ms (entry-split walk).
 //
 // Graphs for which the lagged walk (walk_lag.hip) is chosen keep its sums bit for bit: the
 // early neighbours at least D groups back ("settled") are summed first, the repulsion is
@@ -56,11 +60,22 @@ constexpr int LV_T = 512;         // threads of a level's workgroups: 8 slices o
 constexpr int LV_WAVES = LV_T / 64;
 constexpr int LV_RUN = 2048;      // largest level of a run: 2 slices per wave of 1024 threads
 constexpr int LV_RUNS = 8;        // shortest run: a level in it takes 2-3 us, after about 15 us to start
+constexpr int LV_TICKETS = 8, LV_LINE = 32;  // ticket counters of a launch, ints between them
+constexpr int LV_TICKET_INTS = LV_TICKETS * LV_LINE;
 constexpr int LV_MAXLEVELS = 1 << 16;
 constexpr int LV_LATE = 32;       // longest row of a slice of the late lists
 constexpr int LV_WINDOW = 4096;   // where rows are longer, these lists are sorted by length within such windows
 constexpr unsigned LV_PAD = 0x7fffffffu, LV_RECENT = 0x80000000u;
 constexpr int64_t LV_SHORT = (int64_t)1 << 62;  // host: marks a short row's place
+
+// A level in k_level_flow, its workgroups [first, end) from the last: nn waves of rows of 4 lanes (16 a
+// wave), then nw of rows of 8 (8 a wave), from vertex slot v0 and entry block e0 (64 entries each),
+// then nr rows from row r0, one a wave, then hubs, one a workgroup.
+struct LevelShape {
+    int v0, nn, nw, r0, nr;
+    unsigned e0;
+    int first, end;
+};
 
 struct LevelArgs {
     const int2 *head;      // late slices: first entry, columns
@@ -74,24 +89,88 @@ struct LevelArgs {
     const int *lstart;     // the run kernel: first slice of each level in its run
     double W, step;
     double2 *pos, *rep;
+    double2 *moved;        // new positions, LV_NONE until they are there
     double *eterm;
     const int *status;
+    const int *blk;        // k_level_flow: each workgroup's level
+    const LevelShape *shape;
+    int *ticket, *err;
+    long long ticks;       // the longest wait for a position
 };
 
-// One launch of a level: nn waves of rows of 4 lanes (16 a wave), then nw of rows of 8 (8 a wave),
-// from vertex slot v0 and entry block e0 (64 entries each), then nr rows from row r0, one a wave,
-// then hubs, one a workgroup.
-struct LevelShape {
-    int v0, nn, nw, r0, nr;
-    unsigned e0;
-};
+// "Not moved yet": all ones, a NaN that no stored position is.
+constexpr unsigned long long LV_NONE = ~0ull;
+__device__ __forceinline__ bool is_none(double x) { return (unsigned long long)__double_as_longlong(x) == LV_NONE; }
+
+// Positions between workgroups: 16 bytes an access, past the XCD's L2 on both sides.  One lane's access to an
+// aligned address is one request, so a coordinate is seen whole, and each is looked at by itself.  As two
+// 8-byte accesses (load_through, store_through) the walk took 657 us on R-MAT against 462, for twice
+// the requests of the waves that wait.
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+template <int N>
+__device__ __forceinline__ void load_moved(const LevelArgs &a, const int *j, double2 *p) {
+    f64x2 v[N];
+    if constexpr (N == 1) {
+        __asm__ volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)"
+                         : "=&v"(v[0])
+                         : "v"(a.moved + j[0])
+                         : "memory");
+    } else {
+        static_assert(N == 8, "one or eight positions");
+        __asm__ volatile(
+            "global_load_dwordx4 %0, %8, off sc1\n\tglobal_load_dwordx4 %1, %9, off sc1\n\t"
+            "global_load_dwordx4 %2, %10, off sc1\n\tglobal_load_dwordx4 %3, %11, off sc1\n\t"
+            "global_load_dwordx4 %4, %12, off sc1\n\tglobal_load_dwordx4 %5, %13, off sc1\n\t"
+            "global_load_dwordx4 %6, %14, off sc1\n\tglobal_load_dwordx4 %7, %15, off sc1\n\ts_waitcnt vmcnt(0)"
+            : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
+            : "v"(a.moved + j[0]), "v"(a.moved + j[1]), "v"(a.moved + j[2]), "v"(a.moved + j[3]), "v"(a.moved + j[4]),
+              "v"(a.moved + j[5]), "v"(a.moved + j[6]), "v"(a.moved + j[7])
+            : "memory");
+    }
+#pragma unroll
+    for (int g = 0; g < N; ++g) p[g] = make_double2(v[g].x, v[g].y);
+}
+__device__ __forceinline__ void store_moved(double2 *p, double2 q) {
+    f64x2 v = {q.x, q.y};
+    // two wait states before the registers of a 16-byte store may be written again
+    __asm__ volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+}
 
 // x_i += (F/|F|) * STEP (:1062-1066), the unit vector F * rsqrt2(|F|^2): the lagged walk's operations.
+// FLOW: published for the workgroups of the same launch, else for later launches if there are any that
+// read it (a.moved).
+template <bool FLOW>
 __device__ __forceinline__ void move_vertex(const LevelArgs &a, int i, double2 v, double2 f) {
     const double m2 = f.x * f.x + f.y * f.y;
     const double r = rsqrt2(m2) * a.step;
-    a.pos[i] = make_double2(fma(f.x, r, v.x), fma(f.y, r, v.y));
+    const double2 q = make_double2(fma(f.x, r, v.x), fma(f.y, r, v.y));
+    const double2 m = make_double2(is_none(q.x) ? NAN : q.x, is_none(q.y) ? NAN : q.y);
+    if constexpr (FLOW) store_moved(a.moved + i, m);
+    else if (a.moved) a.moved[i] = m;
+    a.pos[i] = q;
     a.eterm[i] = m2;
+}
+
+// The new positions of the early neighbours j[g] (of which only those with need[g] must be there), each
+// read until it has come.  False: given up, at the deadline or because another wave did.
+template <int N>
+__device__ __forceinline__ bool moved_pos(const LevelArgs &a, const int *j, const bool *need, double2 *p) {
+    load_moved<N>(a, j, p);
+    long long t0 = 0;
+    for (int k = 0;; ++k) {
+        bool wait = false;
+#pragma unroll
+        for (int g = 0; g < N; ++g) wait = wait || (need[g] && (is_none(p[g].x) || is_none(p[g].y)));
+        if (!__any(wait)) return true;
+        if (k == 0) t0 = wall_clock64();
+        if ((k & 15) == 15 || a.ticks < 0) {
+            const bool late = wall_clock64() - t0 > a.ticks;
+            if (late) store_through(a.err, 1);
+            if (late || load_through(a.err)) return false;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        if (wait) load_moved<N>(a, j, p);
+    }
 }
 
 // The late term: |d| by the IEEE square root where the graph keeps the lagged walk's sums.
@@ -162,7 +241,7 @@ __device__ __forceinline__ double lane_before(double v) {
 // of a row forms entry k's factors and adds its product to the sum of the lanes before it, in the
 // k-th of N steps; the repulsion is subtracted before the first recent entry, else at the end.
 template <bool HAS_W, int N>
-__device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t block, int bad) {
+__device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t block) {
     const int lane = threadIdx.x & 63, k = lane & (N - 1);
     const int id = a.vid[vs + lane / N], i = max(id, 0);
     const size_t e = block * 64 + lane;
@@ -170,7 +249,9 @@ __device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t bl
     const double Wk = HAS_W ? a.W * (double)a.w[e] : a.W;
     const bool real = c != LV_PAD;
     const double2 v = a.pos[i], r = a.rep[i];
-    const double2 pj = a.pos[real ? (int)(c & LV_PAD) : i];
+    const int j = real ? (int)(c & LV_PAD) : i;
+    double2 pj;
+    if (!moved_pos<1>(a, &j, &real, &pj)) return;
     double dx, dy, sc;
     attr_factors(pj, v, Wk, dx, dy, sc);
     const unsigned rec = (unsigned)(__ballot(c >= LV_RECENT) >> (lane - k)) & ((1u << N) - 1);
@@ -185,31 +266,39 @@ __device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t bl
         const double sx = fma(dx, sc, px), sy = fma(dy, sc, py);
         if (k == g) f = make_double2(real ? sx : px, real ? sy : py);
     }
-    if (k != N - 1 || id < 0 || bad) return;
+    if (k != N - 1 || id < 0) return;
     if (rec == 0) f = make_double2(f.x - r.x, f.y - r.y);
-    move_vertex(a, i, v, f);
+    move_vertex<true>(a, i, v, f);
 }
 
 // This thread's share of a row's sum: entries t, t + T, ..., eight loads in flight.
-template <bool HAS_W, int T>
-__device__ __forceinline__ double2 row_share(const LevelArgs &a, int4 row, int t, double2 v) {
+// LATE: their iteration-start positions, else the new ones (bad: given up).
+template <bool HAS_W, bool LATE, int T>
+__device__ __forceinline__ double2 row_share(const LevelArgs &a, int4 row, int t, double2 v, int &bad) {
     constexpr int N = 8;
     double2 f = make_double2(0.0, 0.0);
     for (int e = row.y + t; e < row.z; e += N * T) {
-        unsigned c[N];
+        int c[N];
+        bool on[N];
         double2 p[N];
         float w[N];
 #pragma unroll
         for (int g = 0; g < N; ++g) {
             const int k = min(e + g * T, row.z - 1);
-            c[g] = a.rids[k] & LV_PAD;
+            on[g] = e + g * T < row.z;
+            c[g] = (int)(a.rids[k] & LV_PAD);
             w[g] = HAS_W ? a.rw[k] : 0.0f;
         }
+        if constexpr (LATE) {
 #pragma unroll
-        for (int g = 0; g < N; ++g) p[g] = a.pos[c[g]];
+            for (int g = 0; g < N; ++g) p[g] = a.pos[c[g]];
+        } else if (!moved_pos<N>(a, c, on, p)) {
+            bad = 1;
+            break;
+        }
 #pragma unroll
         for (int g = 0; g < N; ++g)
-            add_if(e + g * T < row.z, p[g], v, HAS_W ? a.W * (double)w[g] : a.W, f);
+            add_if(on[g], p[g], v, HAS_W ? a.W * (double)w[g] : a.W, f);
     }
     return f;
 }
@@ -222,11 +311,14 @@ __device__ __forceinline__ double lane_of(double v, int l) {
 // The total force of a row of at most 64 entries with its sums in list order, in every lane: lane
 // k forms the factors of entry k, then the products are added one after another.
 template <bool HAS_W>
-__device__ __forceinline__ double2 row_in_order(const LevelArgs &a, int4 row, int lane, double2 v, double2 r) {
+__device__ __forceinline__ double2 row_in_order(const LevelArgs &a, int4 row, int lane, double2 v, double2 r, int &bad) {
     const int cnt = row.z - row.y, k = row.y + min(lane, cnt - 1);
     const unsigned c = a.rids[k];
     const double Wk = HAS_W ? a.W * (double)a.rw[k] : a.W;
-    const double2 pj = a.pos[c & LV_PAD];
+    const int j = (int)(c & LV_PAD);
+    const bool real = true;
+    double2 pj;
+    if (!moved_pos<1>(a, &j, &real, &pj)) bad = 1;
     double dx, dy, sc;
     attr_factors(pj, v, Wk, dx, dy, sc);
     const uint64_t rec = __ballot(c >= LV_RECENT && lane < cnt);
@@ -248,7 +340,7 @@ __device__ __forceinline__ void finish_row(const LevelArgs &a, bool one, int i, 
     if constexpr (LATE)
         a.rep[i] = make_double2(r.x - f.x, r.y - f.y);
     else
-        move_vertex(a, i, v, make_double2(f.x - r.x, f.y - r.y));
+        move_vertex<true>(a, i, v, make_double2(f.x - r.x, f.y - r.y));
 }
 
 // Rows by workgroup b past the slices' workgroups: nr rows from row r0 one a wave, then hubs (a
@@ -264,11 +356,12 @@ __device__ __forceinline__ void long_rows(const LevelArgs &a, int b, int r0, int
         const int4 row = a.row[r0 + k];  // wave-uniform
         const double2 v = a.pos[row.x], r = a.rep[row.x];
         if constexpr (SEQ) {
-            const double2 f = row_in_order<HAS_W>(a, row, lane, v, r);
-            if (lane == 0 && !bad) move_vertex(a, row.x, v, f);
+            const double2 f = row_in_order<HAS_W>(a, row, lane, v, r, bad);
+            if (lane == 0 && !bad) move_vertex<true>(a, row.x, v, f);
             return;
         }
-        double2 f = row_share<HAS_W, 64>(a, row, lane, v);
+        double2 f = row_share<HAS_W, LATE, 64>(a, row, lane, v, bad);
+        bad = __any(bad);
         f.x = wave_sum(f.x);
         f.y = wave_sum(f.y);
         finish_row<LATE>(a, lane == 0, row.x, v, r, f, bad);
@@ -276,38 +369,66 @@ __device__ __forceinline__ void long_rows(const LevelArgs &a, int b, int r0, int
     }
     const int4 row = a.row[r0 + nr + b - rb];
     const double2 v = a.pos[row.x], r = a.rep[row.x];
-    double2 f = row_share<HAS_W, LV_T>(a, row, (int)threadIdx.x, v);
+    double2 f = row_share<HAS_W, LATE, LV_T>(a, row, (int)threadIdx.x, v, bad);
     f.x = wave_sum(f.x);
     f.y = wave_sum(f.y);
     if (lane == 0) red[wave] = f;
-    __syncthreads();
+    bad = __syncthreads_or(bad);
     f = red[0];
 #pragma unroll
     for (int k = 1; k < LV_WAVES; ++k) f = add2(f, red[k]);
     finish_row<LATE>(a, threadIdx.x == 0, row.x, v, r, f, bad);
 }
 
-// One level (SEQ: every row's sum in list order).  The status word is looked at last, so that no
-// load waits for it.
+// Consecutive levels (SEQ: every row's sum in list order), the longest rows of each first.
 template <bool HAS_W, bool SEQ>
-__global__ __launch_bounds__(LV_T) void k_level(LevelArgs a, LevelShape q) {
+__global__ __launch_bounds__(LV_T) void k_level_flow(LevelArgs a) {
+    __shared__ int tk;
+    if (threadIdx.x == 0) tk = (int)blockIdx.x;
+    if (threadIdx.x == 0 && a.ticket) {  // nullptr: a single level, nothing to wait for
+        const int x = (int)blockIdx.x % LV_TICKETS;
+        tk = x + LV_TICKETS * __hip_atomic_fetch_add(a.ticket + LV_LINE * x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     const int bad = *a.status;
-    const int nsb = (q.nn + q.nw + LV_WAVES - 1) / LV_WAVES;
-    if ((int)blockIdx.x < nsb) {
-        const int k = __builtin_amdgcn_readfirstlane((int)blockIdx.x * LV_WAVES + ((int)threadIdx.x >> 6));
+    __syncthreads();
+    if (bad) return;
+    const int t = __builtin_amdgcn_readfirstlane(tk);
+    const LevelShape q = a.shape[a.blk[t]];
+    const int b = q.end - 1 - t, nsb = (q.nn + q.nw + LV_WAVES - 1) / LV_WAVES;
+    if (b < nsb) {
+        const int k = __builtin_amdgcn_readfirstlane(b * LV_WAVES + ((int)threadIdx.x >> 6));
         constexpr int RN = 64 / LV_NARROW, RW = 64 / LV_WIDE;  // rows a wave
         if (k < q.nn)
-            short_rows<HAS_W, LV_NARROW>(a, q.v0 + RN * k, (size_t)q.e0 + k, bad);
+            short_rows<HAS_W, LV_NARROW>(a, q.v0 + RN * k, (size_t)q.e0 + k);
         else if (k < q.nn + q.nw)
-            short_rows<HAS_W, LV_WIDE>(a, q.v0 + RN * q.nn + RW * (k - q.nn), (size_t)q.e0 + k, bad);
+            short_rows<HAS_W, LV_WIDE>(a, q.v0 + RN * q.nn + RW * (k - q.nn), (size_t)q.e0 + k);
         return;
     }
-    long_rows<HAS_W, false, SEQ>(a, (int)blockIdx.x - nsb, q.r0, q.nr, bad);
+    long_rows<HAS_W, false, SEQ>(a, b - nsb, q.r0, q.nr, 0);
+}
+
+// What k_level_late leaves for an iteration's k_level_flow: no vertex has moved, no workgroup has a ticket.
+struct LevelClear {
+    int late;     // k_level_late's workgroups for the late sums; the others clear
+    int n, nt;    // vertices and ints of tickets (0, 0 where no launch reads them)
+    int *ticket;
+    int first;    // the run's first iteration
+};
+__device__ __forceinline__ void clear_moved(const LevelArgs &a, const LevelClear &q) {
+    const double none = __longlong_as_double((long long)LV_NONE);
+    const int i = ((int)blockIdx.x - q.late) * LV_T + (int)threadIdx.x;
+    if (i < q.n) a.moved[i] = make_double2(none, none);
+    for (int k = i; k < q.nt; k += ((int)gridDim.x - q.late) * LV_T) q.ticket[k] = 0;
+    if (q.first && i == 0) *a.err = 0;
 }
 
 // The late sums of all vertices, folded into the repulsion: ns slices, then the rows.
 template <bool HAS_W, bool IEEE>
-__global__ __launch_bounds__(LV_T) void k_level_late(LevelArgs a, int ns, int nr) {
+__global__ __launch_bounds__(LV_T) void k_level_late(LevelArgs a, int ns, int nr, LevelClear q) {
+    if ((int)blockIdx.x >= q.late) {
+        clear_moved(a, q);
+        return;
+    }
     const int bad = *a.status;
     const int nsb = (ns + LV_WAVES - 1) / LV_WAVES;
     if ((int)blockIdx.x < nsb) {
@@ -404,7 +525,7 @@ __global__ __launch_bounds__(1024) void k_level_run(LevelArgs a, int l0, int l1,
         entries(l + 2, nxt);
 #pragma unroll
         for (int j = 0; j < PER; ++j)
-            if (ido[j] >= 0) move_vertex(a, ido[j], vo[j], f[j]);
+            if (ido[j] >= 0) move_vertex<false>(a, ido[j], vo[j], f[j]);
         __syncthreads();
     }
 }
@@ -502,6 +623,10 @@ __global__ __launch_bounds__(256) void k_level_fill(int n, int B, int D, const i
 }  // namespace
 
 namespace {
+int level_blocks(int slices, int rows, int hubs) {
+    return (slices + LV_WAVES - 1) / LV_WAVES + (rows + LV_WAVES - 1) / LV_WAVES + hubs;
+}
+
 bool build_plan(bl_graph *g, int B, int D) {
     const int n = g->n;
     if ((int)g->h_rowptr.size() != n + 1 || (int64_t)g->h_colids.size() != g->nnz) return false;
@@ -578,16 +703,20 @@ bool build_plan(bl_graph *g, int B, int D) {
     std::vector<int32_t> start;  // of each level of the runs, its first slice in its run, and the run's end
     auto count = [&](int l, int c) { return first[(size_t)l * K + c + 1] - first[(size_t)l * K + c]; };
     auto small = [&](int l) { return count(l, 0) + count(l, 1) <= LV_RUN && count(l, 2) + count(l, 3) == 0; };
+    std::vector<LevelShape> shape;
+    std::vector<int32_t> blk;  // of each workgroup of k_level_flow, its level
     g->lev_launch.clear();
     g->lev_big = g->lev_small = 0;
     for (int l = 0; l < nl;) {
         int e = l;
         while (e < nl && small(e)) ++e;
-        LevelLaunch q{};
-        q.v0 = (int)E.L.vid.size();
-        q.e0 = (uint32_t)(E.nid / 64);
+        const int v0 = (int)E.L.vid.size();
+        const uint32_t e0 = (uint32_t)(E.nid / 64);
         const int32_t *vs = order.data() + first[(size_t)l * K];
         if (e - l >= LV_RUNS) {
+            LevelLaunch q{};
+            q.v0 = v0;
+            q.e0 = e0;
             q.l0 = (int)start.size();
             q.l1 = q.l0 + e - l;
             int at = 0;  // slices of the run
@@ -599,18 +728,32 @@ bool build_plan(bl_graph *g, int B, int D) {
             }
             start.push_back(at);
             g->lev_small += q.l1 - q.l0;
+            g->lev_launch.push_back(q);
         } else {
+            LevelShape q{};
+            q.v0 = v0;
+            q.e0 = e0;
             q.nn = E.short_rows(vs, count(l, 0), LV_NARROW);
             q.nw = E.short_rows(vs + count(l, 0), count(l, 1), LV_WIDE);
             vs += count(l, 0) + count(l, 1);
             q.r0 = (int)E.L.row.size();
             q.nr = count(l, 2);
-            q.nh = count(l, 3);
-            for (int t = 0; t < q.nr + q.nh; ++t) E.row(vs[t], ec[vs[t]]);
+            const int nh = count(l, 3);
+            for (int t = 0; t < q.nr + nh; ++t) E.row(vs[t], ec[vs[t]]);
+            if (g->lev_launch.empty() || g->lev_launch.back().l1 > g->lev_launch.back().l0) {
+                LevelLaunch f{};
+                f.b0 = (int)blk.size();
+                g->lev_launch.push_back(f);
+            }
+            LevelLaunch &f = g->lev_launch.back();
+            q.first = f.blocks;
+            f.blocks = q.end = f.blocks + level_blocks(q.nn + q.nw, q.nr, nh);
+            blk.insert(blk.end(), (size_t)(q.end - q.first), (int32_t)shape.size());
+            shape.push_back(q);
+            ++f.levels;
             ++g->lev_big;
             ++l;
         }
-        g->lev_launch.push_back(q);
         if (E.nid > cap * 32 || (int64_t)E.L.vid.size() > cap) return false;
     }
     // the late lists: slices in vertex order, sorted by length within windows where rows are long
@@ -644,7 +787,10 @@ bool build_plan(bl_graph *g, int B, int D) {
         ~Temp() { e.release(), l.release(), go.release(); }
     } t;
     if (!E.L.upload(g->lev_early, gw, E.nid, E.nrid, st) || !L.L.upload(g->lev_late, gw, L.nid, L.nrid, st) ||
-        !put(g->lev_start, start) || !put(t.e, E.slot) || !put(t.l, L.slot) || !put(t.go, go))
+        !put(g->lev_start, start) || !put(g->lev_blk, blk) || !put(g->lev_shape, shape) ||
+        g->lev_moved.ensure(sizeof(double2) * (size_t)n) ||
+        g->lev_ticket.ensure(4 * (g->lev_launch.size() + 1) * LV_TICKET_INTS) || !put(t.e, E.slot) ||
+        !put(t.l, L.slot) || !put(t.go, go))
         return false;
     const auto fill = [&](const DevBuf &slot, const LevelLists &d) {
         return FillList{slot.as<int64_t>(), d.ids.as<unsigned>(), d.rids.as<unsigned>(),
@@ -691,25 +837,39 @@ LevelArgs level_args(const bl_graph *g, const LevelLists &d, double2 *pos, const
     a.step = step;
     a.pos = pos;
     a.rep = g->bh.rep.as<double2>();
+    a.moved = g->lev_moved.as<double2>();
     a.eterm = g->eterm.as<double>();
     a.status = g->bh.misc.as<int>();
+    a.blk = nullptr;
+    a.shape = g->lev_shape.as<LevelShape>();
+    a.ticket = nullptr;
+    a.err = g->bh.misc.as<int>() + BH_LEVEL_ERR;
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g->device) != hipSuccess || khz <= 0)
+        khz = 100000;
+    a.ticks = (long long)khz * 10000;  // 10 s
+    if (const char *w = getenv("BL_LEVEL_WAIT_US")) a.ticks = (long long)khz * atoll(w) / 1000;  // tests
     return a;
 }
-int level_blocks(int slices, int rows, int hubs) {
-    return (slices + LV_WAVES - 1) / LV_WAVES + (rows + LV_WAVES - 1) / LV_WAVES + hubs;
-}
+bool is_flow(const LevelLaunch &q) { return q.blocks > 0; }
 }  // namespace
 
-// The late sums, before any vertex moves.
-int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, hipStream_t s) {
+// The late sums, before any vertex moves (and the marks for k_level_flow).
+int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, int it, hipStream_t s) {
     const LevelArgs a = level_args(g, g->lev_late, pos, p, 0.0);
     const int ns = g->lev_late_slices, nr = g->lev_late_rows;
-    const int grid = level_blocks(ns, nr, g->lev_late_hubs);
+    LevelClear q{level_blocks(ns, nr, g->lev_late_hubs), 0, 0, g->lev_ticket.as<int>(), it == 0};
+    const int flows = (int)std::count_if(g->lev_launch.begin(), g->lev_launch.end(), is_flow);
+    if (flows) {
+        q.n = g->n;
+        q.nt = flows * LV_TICKET_INTS;
+    }
+    const int grid = q.late + (q.n + LV_T - 1) / LV_T;
     if (grid > 0) {
         const bool ieee = g->lev_d > 0;
         auto k = g->has_w ? (ieee ? k_level_late<true, true> : k_level_late<true, false>)
                           : (ieee ? k_level_late<false, true> : k_level_late<false, false>);
-        hipLaunchKernelGGL(k, dim3(grid), dim3(LV_T), 0, s, a, ns, nr);
+        hipLaunchKernelGGL(k, dim3(grid), dim3(LV_T), 0, s, a, ns, nr, q);
     }
     BL_HIP(hipGetLastError());
     return BL_OK;
@@ -717,16 +877,23 @@ int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, hipStream_t
 
 // One iteration's walk (after launch_level_late).
 int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, double step, hipStream_t s) {
-    const LevelArgs a = level_args(g, g->lev_early, pos, p, step);
-    auto k = g->has_w ? (g->lev_d > 0 ? k_level<true, true> : k_level<true, false>)
-                      : (g->lev_d > 0 ? k_level<false, true> : k_level<false, false>);
+    LevelArgs a = level_args(g, g->lev_early, pos, p, step);
+    int left = (int)std::count_if(g->lev_launch.begin(), g->lev_launch.end(), is_flow);
+    int *ticket = g->lev_ticket.as<int>();
+    auto k = g->has_w ? (g->lev_d > 0 ? k_level_flow<true, true> : k_level_flow<true, false>)
+                      : (g->lev_d > 0 ? k_level_flow<false, true> : k_level_flow<false, false>);
     for (const LevelLaunch &q : g->lev_launch) {
-        if (q.l1 > q.l0)
+        if (is_flow(q)) {
+            a.blk = g->lev_blk.as<int>() + q.b0;
+            a.ticket = q.levels > 1 ? ticket : nullptr;
+            ticket += LV_TICKET_INTS;
+            --left;
+            hipLaunchKernelGGL(k, dim3(q.blocks), dim3(LV_T), 0, s, a);
+        } else {
+            if (!left) a.moved = nullptr;
             hipLaunchKernelGGL(g->has_w ? k_level_run<true> : k_level_run<false>, dim3(1), dim3(1024), 0, s, a, q.l0,
                                q.l1, q.v0, q.e0);
-        else
-            hipLaunchKernelGGL(k, dim3(level_blocks(q.nn + q.nw, q.nr, q.nh)), dim3(LV_T), 0, s, a,
-                               LevelShape{q.v0, q.nn, q.nw, q.r0, q.nr, q.e0});
+        }
     }
     BL_HIP(hipGetLastError());
     return BL_OK;
