@@ -295,7 +295,9 @@ __global__ __launch_bounds__(1024) void k_scan_single(const int *__restrict__ in
 }
 
 // ---------------------------------------------------------------------------------------
-// 3. LSD radix sort, 8-bit digits.  hist is digit-major: hist[d * nblk + blk].
+// 3. LSD radix sort, 8-bit digits.  hist is digit-major, hist[d * nblk + blk], or with few tiles (SUM)
+// tile-major, hist[blk * 256 + d].
+template <bool SUM>
 __global__ __launch_bounds__(WG) void k_sort_hist(const uint64_t *__restrict__ keys, int n, int shift, int nblk,
                                                   int rounds, int *__restrict__ hist) {
     __shared__ int h[256];
@@ -308,7 +310,7 @@ __global__ __launch_bounds__(WG) void k_sort_hist(const uint64_t *__restrict__ k
         if (i < n) atomicAdd(&h[(int)((keys[i] >> shift) & 255u)], 1);
     }
     __syncthreads();
-    hist[threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
+    hist[SUM ? blockIdx.x * 256 + threadIdx.x : threadIdx.x * nblk + blockIdx.x] = h[threadIdx.x];
 }
 
 // Per-digit scan of the histogram: workgroup d turns row d (the blocks' counts of digit d) into
@@ -361,7 +363,9 @@ __global__ __launch_bounds__(WG) void k_sort_rowscan(int *__restrict__ hist, int
 // thread t then writes entries t, t + WG, ... to the digit's global bucket, which starts at the
 // keys of all smaller digits (the exclusive scan of dtot) plus the tile's row prefix.  GATHER
 // (the last pass): also spos[g] = pos[id], the positions in sorted order.
-template <int R, bool GATHER>
+// SUM: every workgroup adds up all tiles' counts (offs as k_sort_hist left them) and the launch of
+// k_sort_rowscan goes: 1 KB a tile from the L2, 64 lanes a tile, sixteen tiles a wave in flight.
+template <int R, bool GATHER, bool SUM>
 __global__ __launch_bounds__(WG) void k_sort_scatter(const uint64_t *__restrict__ kin, const int *__restrict__ vin,
                                                      uint64_t *__restrict__ kout, int *__restrict__ vout, int n,
                                                      int shift, int nblk, const int *__restrict__ offs,
@@ -377,7 +381,7 @@ __global__ __launch_bounds__(WG) void k_sort_scatter(const uint64_t *__restrict_
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int base = blockIdx.x * TILE;
     const int cnt = min(TILE, n - base);
-    const int cd = dtot[tid], row = offs[tid * nblk + blockIdx.x];
+    int cd = SUM ? 0 : dtot[tid], row = SUM ? 0 : offs[tid * nblk + blockIdx.x];
     const int wb = w * 64 * R + lane;
     uint64_t k[R];
     int v[R];
@@ -387,9 +391,37 @@ __global__ __launch_bounds__(WG) void k_sort_scatter(const uint64_t *__restrict_
         k[r] = e < cnt ? kin[base + e] : 0ull;
         v[r] = e < cnt ? vin[base + e] : 0;
     }
+    // [total, before this tile][wave][digit]; sk is staged two barriers after they are read
+    int *const part = reinterpret_cast<int *>(sk);
+    if constexpr (SUM) {
+        constexpr int U = 16;
+        const int4 *h4 = reinterpret_cast<const int4 *>(offs) + lane;  // digits 4 lane .. 4 lane + 3
+        int4 all = make_int4(0, 0, 0, 0), bef = all;
+        for (int q0 = w; q0 < nblk; q0 += NW * U) {
+            int4 h[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) h[u] = h4[64 * min(q0 + NW * u, nblk - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int q = q0 + NW * u;
+                const int a = q < nblk ? -1 : 0, b = q < (int)blockIdx.x ? -1 : 0;
+                all.x += h[u].x & a, all.y += h[u].y & a, all.z += h[u].z & a, all.w += h[u].w & a;
+                bef.x += h[u].x & b, bef.y += h[u].y & b, bef.z += h[u].z & b, bef.w += h[u].w & b;
+            }
+        }
+        reinterpret_cast<int4 *>(part)[w * 64 + lane] = all;
+        reinterpret_cast<int4 *>(part)[(NW + w) * 64 + lane] = bef;
+    }
 #pragma unroll
     for (int q = 0; q < NW; ++q) wrun[q][tid] = 0;
     __syncthreads();
+    if constexpr (SUM) {
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            cd += part[q * 256 + tid];
+            row += part[(NW + q) * 256 + tid];
+        }
+    }
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     int rk[R];
 #pragma unroll
@@ -2363,6 +2395,12 @@ int ensure_bh(BHWork &w, int n) {
     return BL_OK;
 }
 
+// Tiles up to which every tile's workgroup sums all tiles' counts itself (1 KB each), in place of a launch
+// that scans them: the launch is 3.5 us of each of the six passes, the sum grows with the tiles.  Tree in us,
+// scan / sum: 20,000 points (10 tiles) 143 / 130, 60,000 150 / 137, 120,000 160 / 147, 250,000 (123) 175 / 166,
+// 400,000 (196) 199 / 199, 800,000 (391) 259 / 289.
+constexpr int SORT_SUM = 128;
+
 // Steps 1 to 4: the points in Morton order (keys_a, idx_a, spos), for any n.
 int sort_points(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t *d_xs, uint32_t *d_ys) {
     int *misc = w.misc.as<int>();
@@ -2381,16 +2419,16 @@ int sort_points(BHWork &w, const double2 *d_pos, int n, hipStream_t s, uint32_t 
     double2 *spos = w.spos.as<double2>();
     int *hist = w.hist.as<int>();
     int *dtot = w.scan_tmp.as<int>();
+    const char *senv = getenv("BL_SORT_SUM");  // 0: with the scan's launch (tests)
+    const bool sum = nblk <= SORT_SUM && !(senv && !strcmp(senv, "0"));
     for (int pass = SORT_SKIP / 8; pass < 8; ++pass) {
         const int shift = 8 * pass;
-        hipLaunchKernelGGL(k_sort_hist, dim3(nblk), dim3(WG), 0, s, ka, n, shift, nblk, rounds, hist);
-        hipLaunchKernelGGL(k_sort_rowscan, dim3(256), dim3(WG), 0, s, hist, nblk, dtot);
-        if (pass < 7)
-            hipLaunchKernelGGL((k_sort_scatter<SORT_ROUNDS, false>), dim3(nblk), dim3(WG), 0, s, ka, ia, kb, ib, n,
-                               shift, nblk, hist, dtot, d_pos, spos);
-        else
-            hipLaunchKernelGGL((k_sort_scatter<SORT_ROUNDS, true>), dim3(nblk), dim3(WG), 0, s, ka, ia, kb, ib, n,
-                               shift, nblk, hist, dtot, d_pos, spos);
+        hipLaunchKernelGGL(sum ? k_sort_hist<true> : k_sort_hist<false>, dim3(nblk), dim3(WG), 0, s, ka, n, shift, nblk,
+                           rounds, hist);
+        if (!sum) hipLaunchKernelGGL(k_sort_rowscan, dim3(256), dim3(WG), 0, s, hist, nblk, dtot);
+        const auto scatter = sum        ? pass < 7 ? k_sort_scatter<SORT_ROUNDS, false, true> : k_sort_scatter<SORT_ROUNDS, true, true>
+                             : pass < 7 ? k_sort_scatter<SORT_ROUNDS, false, false> : k_sort_scatter<SORT_ROUNDS, true, false>;
+        hipLaunchKernelGGL(scatter, dim3(nblk), dim3(WG), 0, s, ka, ia, kb, ib, n, shift, nblk, hist, dtot, d_pos, spos);
         std::swap(ka, kb);
         std::swap(ia, ib);
     }
