@@ -52,6 +52,7 @@
 
 #include "bh_common.h"
 #include "pair_math.h"
+#include "traverse.h"
 
 namespace bl {
 namespace {
@@ -151,12 +152,16 @@ __device__ __forceinline__ double2 chunk_sums(Src src, int n, int c0, int cpt, i
             for (int k = 0; k < 8; ++k) qx[k] = src[2 * (j + k)], qy[k] = src[2 * (j + k) + 1];
             pair_rep_group<REFINE, 8>(qx, qy, p.x, p.y, ax, ay);
         }
-        if (j < j1) dense_tail<REFINE, 8>(src, j, j1, p.x, p.y, ax, ay), j = j1;
+        if constexpr (REFINE) {
+            if (j < j1) add_group<8, false>(interleaved(src), j, 1, j1, p.x, p.y, ax, ay), j = j1;
+        } else {
+            for (; j < j1; ++j) pair_rep<false>(src[2 * j], src[2 * j + 1], p.x, p.y, ax, ay);
+        }
         t.add(ax, ay);
     }
     const double2 v = t.total(__builtin_ctz(cpt));
     if (isfinite(v.x) && isfinite(v.y)) return v;
-    PairTree u;  // a group's product left the range: each such chunk again, pair by pair
+    PairTree u;  // a group's product left the range: each such chunk again, with care
     for (int c = c0; c < c0 + cpt; ++c) {
         double ax, ay;
         dense_sum<REFINE, 8, true>(src, min(n, c * sub), min(n, (c + 1) * sub), p.x, p.y, ax, ay);
@@ -218,11 +223,12 @@ __device__ void layout_graph(const BatchedArgs &a, int g, int me, int T, double2
     double2 *parts = a.parts + (size_t)at * 2 * MAXTEAM * B;
     const int share = max(1, T / L);          // members whose subtrees a lane of a row adds
     int need = 0;
-    double step = a.step0, E = 0.0;
+    double step = scalar(a.step0), E = 0.0;  // in scalar registers: the vector ones are short
     auto ends = [&](int b) {  // this row's entries in batch b
         const int i = v0 + min(n - 1, b * B + row);
         return make_int2(a.rp[i], a.rend[i]);
     };
+    const auto posn = [=](int j) { return gp[j]; };
     auto first = [&](int2 e) { return e.x + k < e.y ? a.ci[e.x + k] : 0; };
     int2 er = ends(0);
     int jn = first(er);
@@ -232,9 +238,21 @@ __device__ void layout_graph(const BatchedArgs &a, int g, int me, int T, double2
             const bool mine = row < bc;
             const double2 pr = gp[b0 + (mine ? row : 0)];
             double cx = 0.0, cy = 0.0;
+            const int law = a.law == LAW_FA ? LAW_FA : LAW_FR;
+            bool close = false;
             for (int e = er.x + k; e < er.y; e += L) {
-                const double2 pj = gp[e == er.x + k ? jn : a.ci[e]];
-                correct_pair<REFINE>(a.law == LAW_FA ? LAW_FA : LAW_FR, a.W, pj.x - pr.x, pj.y - pr.y, cx, cy);
+                const int j = e == er.x + k ? jn : a.ci[e];
+                const double2 pj = gp[j];
+                const double dx = pj.x - pr.x, dy = pj.y - pr.y;
+                const double inv = linked_factor<REFINE>(posn, true, j & ~(GROUP - 1), j & (GROUP - 1), 1, n, pr.x, pr.y,
+                                                         dx, dy);  // chunks begin at whole groups
+                correct_pair(law, a.W, dx, dy, inv, cx, cy);
+                close = close || too_close<REFINE>(dx, dy);
+            }
+            const bool apart = REFINE && (__ballot(close) >> (tid & 63 & ~(L - 1)) & ((1ull << L) - 1)) != 0;
+            if (apart) {
+                const double2 f = apart_share(posn, n, k, L, pr.x, pr.y, a.ci, er.x, er.y, [&](int) { return a.W; }, law);
+                cx = f.x, cy = f.y;
             }
             // the next batch's entries are loaded behind this batch's dense sum
             er = ends(b + 1 < nb ? b + 1 : 0);
@@ -291,8 +309,8 @@ __device__ void layout_graph(const BatchedArgs &a, int g, int me, int T, double2
                 f.x = lanes_sum(f.x, T / share);
                 f.y = lanes_sum(f.y, T / share);
             }
-            f.x += cx;
-            f.y += cy;
+            f.x = apart ? cx : f.x + cx;
+            f.y = apart ? cy : f.y + cy;
             // the move (every force of the batch is formed from the positions before it)
             if (mine && k == 0) gp[b0 + row] = moved(gp[b0 + row], f.x, f.y, step);
             if (it == a.iters - 1) {  // the energy: wave sums, then the 16 wave sums in order
@@ -304,11 +322,11 @@ __device__ void layout_graph(const BatchedArgs &a, int g, int me, int T, double2
                 double eb_sum = 0.0;
 #pragma unroll
                 for (int q = 0; q < BT / 64; ++q) eb_sum += eb[q];
-                E += eb_sum;  // batches added in order
+                E = scalar(E + eb_sum);  // batches added in order
             }
             ++need;
         }
-        step = step * a.decay;
+        step = scalar(step * a.decay);
     }
     if (me == 0) {
         if (in_lds) {

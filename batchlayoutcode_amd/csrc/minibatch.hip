@@ -15,7 +15,9 @@
 // 1/|d|^2 (mixed: FP64, one reciprocal for eight pairs; FP32: v_rcp_f32), and the term -d/|d|^2
 // accumulated in FP64 (one FMA per component with the FP64 difference).  The dense loop runs over all j; neighbours are not
 // branched on: a correction adds, in FP64, each neighbour's attraction and removes the
-// repulsion product the dense loop accumulated for it (the same operands, so it cancels).
+// repulsion product the dense loop accumulated for it, for close ones from the same factor bit for bit
+// (linked_factor), so that what is left of it is the sum's own rounding.  A vertex with a neighbour closer than 2^-40 has its
+// force formed without that neighbour's repulsion (apart_share).
 //   * k_step32 (small graphs): one launch per batch step, a workgroup per batch vertex.
 //   * k_pairs32 + k_move32: two launches per batch step.  The pair kernel's
 //     chunk workgroups write each batch vertex's chunk partials; its correction waves take
@@ -69,14 +71,16 @@ __device__ __forceinline__ void move_one(double2 *pos, int i, double fx, double 
 // Workgroups x >= G (row 0 only): one wave per correction piece of the batch (pieces
 // [pc0, pc0+npc): at most CORR_PIECE neighbour entries of one vertex, so a hub's correction
 // is spread over many waves instead of holding up the step).
-// part[slot * P + x] receives the chunk partial; part[slot * P + G + k] piece k's correction.
+// part[slot * P + x] receives the chunk partial; part[slot * P + G + k] piece k's correction, or a NaN of
+// the bits APART and the x of the vertex's whole force, whose y is then in eterm.
+constexpr long long APART = 0x7ffa6d6f72746170;
 template <int JS, bool REFINE>
 __global__ __launch_bounds__(WG) void k_pairs32(const double2 *__restrict__ pos, int n, int b0, int bc, int chunk,
                                                 int G, double2 *__restrict__ part, int P,
                                                 const int *__restrict__ erp, const int *__restrict__ eci,
                                                 const float *__restrict__ ew, double W, int law,
                                                 const int *__restrict__ cpre, const int *__restrict__ cpv, int pc0,
-                                                int npc) {
+                                                int npc, double *__restrict__ eterm) {
     constexpr int IPW = WG / JS;
     __shared__ double2 red[WG];
     const int tid = threadIdx.x;
@@ -91,13 +95,33 @@ __global__ __launch_bounds__(WG) void k_pairs32(const double2 *__restrict__ pos,
         double cx = 0.0, cy = 0.0;
         const int kbeg = erp[i] + k * CORR_PIECE;
         const int kend = min(erp[i + 1], kbeg + CORR_PIECE);
+        const int grouped = n / UNROLL * UNROLL;  // a subgroup's range begins and ends at whole UNROLLs, or at n
+        const auto at = [=](int j) { return pos[j]; };
+        bool close = false;
         for (int e = kbeg + lane; e < kend; e += 64) {
-            const double2 pj = pos[eci[e]];
-            correct_pair<REFINE>(law, ew ? W * (double)ew[e] : W, pj.x - pi.x, pj.y - pi.y, cx, cy);
+            const int j = eci[e];
+            const double2 pj = pos[j];
+            const double dx = pj.x - pi.x, dy = pj.y - pi.y;
+            const double inv = linked_factor<REFINE>(at, j < grouped, j & ~(GROUP - 1), j & (GROUP - 1), 1, n, pi.x,
+                                                     pi.y, dx, dy);
+            correct_pair(law, ew ? W * (double)ew[e] : W, dx, dy, inv, cx, cy);
+            close = close || too_close<REFINE>(dx, dy);
+        }
+        double2 *mine = part + (size_t)(i - b0) * P + G + k;
+        if (__ballot(close)) {  // the whole force, for k_move32 to take instead of the sum
+            const double2 f = apart_share(at, n, lane, 64, pi.x, pi.y, eci, erp[i], erp[i + 1],
+                                          [=](int e) { return ew ? W * (double)ew[e] : W; }, law);
+            cx = wave_sum(f.x);
+            cy = wave_sum(f.y);
+            if (lane == 0) {
+                *mine = make_double2(__longlong_as_double(APART), cx);
+                eterm[i] = cy;
+            }
+            return;
         }
         cx = wave_sum(cx);
         cy = wave_sum(cy);
-        if (lane == 0) part[(size_t)(i - b0) * P + G + k] = make_double2(cx, cy);
+        if (lane == 0) *mine = make_double2(cx, cy);
         return;
     }
     const int li = tid % IPW;
@@ -112,6 +136,9 @@ __global__ __launch_bounds__(WG) void k_pairs32(const double2 *__restrict__ pos,
     const int j0 = min(je, jb + js * sub);
     const int j1 = min(je, j0 + sub);
     double ax, ay;
+    // lgkmcnt(0): with arguments still on their way the compiler waits between the loop's scalar loads, in every
+    // round (1 us a step)
+    __builtin_amdgcn_s_waitcnt(0xc07f);
     dense_sum<REFINE, UNROLL>(cpos, j0, j1, px, py, ax, ay);
     if constexpr (JS > 1) {
         red[tid] = make_double2(ax, ay);
@@ -140,6 +167,7 @@ __global__ __launch_bounds__(NT) void k_step32(const double2 *__restrict__ src, 
                                                int law, const double *__restrict__ stepp, double step,
                                                double *__restrict__ eterm) {
     __shared__ double2 red[NT / 64];
+    __shared__ uint64_t near[NT / 64];
     const int tid = threadIdx.x;
     const int i = b0 + (int)blockIdx.x;
     const double2 pi = src[i];
@@ -148,14 +176,37 @@ __global__ __launch_bounds__(NT) void k_step32(const double2 *__restrict__ src, 
     double ax = 0.0, ay = 0.0;
     strided_sum<REFINE, NT>(src, tid, n, pi.x, pi.y, ax, ay);
     double cx = 0.0, cy = 0.0;
+    bool close = false;
+    const auto at = [=](int j) { return src[j]; };
     for (int e = e0 + tid; e < e1; e += NT) {
-        const double2 pj = src[e == e0 + tid ? jn : eci[e]];
-        correct_pair<REFINE>(law, ew ? W * (double)ew[e] : W, pj.x - pi.x, pj.y - pi.y, cx, cy);
+        const int j = e == e0 + tid ? jn : eci[e];
+        const double2 pj = src[j];
+        const double dx = pj.x - pi.x, dy = pj.y - pi.y;
+        const int q = j / NT;  // the position's place in thread j % NT
+        const double inv = linked_factor<REFINE>(at, true, j - (q & (GROUP - 1)) * NT, q & (GROUP - 1), NT, n, pi.x, pi.y,
+                                                 dx, dy);
+        correct_pair(law, ew ? W * (double)ew[e] : W, dx, dy, inv, cx, cy);
+        close = close || too_close<REFINE>(dx, dy);
     }
     ax = wave_sum(ax + cx);
     ay = wave_sum(ay + cy);
-    if ((tid & 63) == 0) red[tid >> 6] = make_double2(ax, ay);
+    const uint64_t any = __ballot(close);
+    if ((tid & 63) == 0) red[tid >> 6] = make_double2(ax, ay), near[tid >> 6] = any;
     __syncthreads();
+    if constexpr (REFINE) {
+        uint64_t apart = 0;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) apart |= near[w];
+        if (apart) {
+            const double2 f = apart_share(at, n, tid, NT, pi.x, pi.y, eci, e0, e1,
+                                          [=](int e) { return ew ? W * (double)ew[e] : W; }, law);
+            ax = wave_sum(f.x);
+            ay = wave_sum(f.y);
+            __syncthreads();
+            if ((tid & 63) == 0) red[tid >> 6] = make_double2(ax, ay);
+            __syncthreads();
+        }
+    }
     if (tid == 64)
         for (int k = (int)blockIdx.x; k < pc; k += (int)gridDim.x) dst[p0 + k] = src[p0 + k];
     if (tid == 0) {
@@ -293,8 +344,11 @@ __global__ __launch_bounds__(WG) void k_move32(const double2 *__restrict__ part,
     if (lane == 0) red[w] = make_double2(sx, sy);
     __syncthreads();
     if (tid == 0) {
-        const double fx = (red[0].x + red[1].x) + (red[2].x + red[3].x);
-        const double fy = (red[0].y + red[1].y) + (red[2].y + red[3].y);
+        double fx = (red[0].x + red[1].x) + (red[2].x + red[3].x);
+        double fy = (red[0].y + red[1].y) + (red[2].y + red[3].y);
+        if (isnan(fx))
+            for (p = G; p < pe; ++p)
+                if (__double_as_longlong(row[p].x) == APART) fx = row[p].y, fy = eterm[i];
         pos[i] = moved(x0, fx, fy, stepp ? *stepp : step);
         eterm[i] = fx * fx + fy * fy;
     }
@@ -624,20 +678,20 @@ int run_minibatch(bl_graph *g, double *d_xy, const bl_params *p, int law, double
                     prof.ext(0, &e0, &e1);
                     if (p->precision == BL_PREC_FP32)
                         hipExtLaunchKernelGGL((k_pairs32<4, false>), grid, dim3(WG), 0, s, e0, e1, 0, pos, n, b0, bc,
-                                              chunk, G, part, P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc);
+                                              chunk, G, part, P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc, eterm);
                     else
                         hipExtLaunchKernelGGL((k_pairs32<4, true>), grid, dim3(WG), 0, s, e0, e1, 0, pos, n, b0, bc,
-                                              chunk, G, part, P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc);
+                                              chunk, G, part, P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc, eterm);
                     prof.ext(1, &e0, &e1);
                     hipExtLaunchKernelGGL(k_move32, dim3(bc), dim3(WG), 0, s, e0, e1, 0, part, P, G, cpre, pos, b0, bc,
                                           d_step, STEP, eterm);
                 } else {
                     if (p->precision == BL_PREC_FP32)
                         hipLaunchKernelGGL((k_pairs32<4, false>), grid, dim3(WG), 0, s, pos, n, b0, bc, chunk, G, part,
-                                           P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc);
+                                           P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc, eterm);
                     else
                         hipLaunchKernelGGL((k_pairs32<4, true>), grid, dim3(WG), 0, s, pos, n, b0, bc, chunk, G, part,
-                                           P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc);
+                                           P, erp, eci, ew, p->weight, law, cpre, cpv, pc0, npc, eterm);
                     hipLaunchKernelGGL(k_move32, dim3(bc), dim3(WG), 0, s, part, P, G, cpre, pos, b0, bc, d_step,
                                        STEP, eterm);
                 }

@@ -3,7 +3,8 @@
 // Reference semantics (sample/algorithms.cpp:758-768): a neighbour j of i contributes the
 // attraction A(d) with d = x_j - x_i; any other j with |d|^2 > 0 contributes -d/|d|^2.
 // The dense loops add -d/|d|^2 for every j (the self pair gives 0); correct_pair() then
-// removes, for each neighbour, the product the dense loop added and adds A(d).
+// removes, for each neighbour, the product the dense loop added and adds A(d).  Neighbours almost
+// on top of a vertex, whose product would drown its force, are left out instead (apart_share).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -138,42 +139,57 @@ __device__ __forceinline__ void pair_rep_group(const double *qx, const double *q
     }
 }
 
-// The positions [j, j1) past the last whole group of N, added in order.  REFINE: one more group, filled
-// up with pairs of distance 0 and |d|^2 = 1 (a serial chain of reciprocals took 5 us of a batch step).
-template <bool REFINE, int N, class Src>
-__device__ __forceinline__ void dense_tail(Src src, const int j, const int j1, const double px, const double py,
-                                           double &ax, double &ay) {
-    if constexpr (REFINE) {
-        double dx[N], dy[N], r[N];
+// A group's differences to (px, py) and |d|^2: positions at(j), at(j + D), ... below end; those past it stand
+// for a pair of distance 0 and |d|^2 = 1.
+template <int N, class At>
+__device__ __forceinline__ void load_group(At at, const int j, const int D, const int end, const double px,
+                                           const double py, double *dx, double *dy, double *r) {
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-            const int q = min(j + k, j1 - 1);
-            const double qx = src[2 * q], qy = src[2 * q + 1];
-            const bool in = j + k < j1;
-            dx[k] = in ? qx - px : 0.0;
-            dy[k] = in ? qy - py : 0.0;
-            r[k] = in ? fma(dy[k], dy[k], fma(dx[k], dx[k], kTiny64)) : 1.0;
-        }
-        recip_all<N>(r);
-#pragma unroll
-        for (int k = 0; k < N; ++k) {
-            ax = fma(-dx[k], r[k], ax);
-            ay = fma(-dy[k], r[k], ay);
-        }
-    } else {
-        for (int k = j; k < j1; ++k) pair_rep<false>(src[2 * k], src[2 * k + 1], px, py, ax, ay);
+    for (int k = 0; k < N; ++k) {
+        const bool in = j + k * D < end;
+        const double2 q = at(in ? j + k * D : j);
+        dx[k] = in ? q.x - px : 0.0;
+        dy[k] = in ? q.y - py : 0.0;
+        r[k] = in ? fma(dy[k], dy[k], fma(dx[k], dx[k], kTiny64)) : 1.0;
     }
 }
 
+// Adds the terms of a group.  CAREFUL: a product of |d|^2 may have left the FP64 range; where a pair's factor
+// is not finite, it has one of its own.
+template <int N, bool CAREFUL, class At>
+__device__ __forceinline__ void add_group(At at, const int j, const int D, const int end, const double px,
+                                          const double py, double &ax, double &ay) {
+    double dx[N], dy[N], r[N], own[N];
+    load_group<N>(at, j, D, end, px, py, dx, dy, r);
+#pragma unroll
+    for (int k = 0; k < N; ++k) own[k] = r[k];
+    recip_all<N>(r);
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const double f = CAREFUL && !isfinite(r[k]) ? recip(own[k]) : r[k];
+        ax = fma(-dx[k], f, ax);
+        ay = fma(-dy[k], f, ay);
+    }
+}
+
+// x, y interleaved as positions.
+template <class Src>
+__device__ __forceinline__ auto interleaved(Src src) {
+    return [=](int j) { return make_double2(src[2 * j], src[2 * j + 1]); };
+}
+
+constexpr int GROUP = 8;  // pairs that share a reciprocal
+
 // The dense repulsion of position (px, py) against positions [j0, j1) of src (x, y interleaved),
-// U positions loaded at a time, in (ax, ay).  A sum that is not finite is formed again pair by
-// pair: a group's product may have left the FP64 range where no single |d|^2 does.
-// PAD: the positions past the last whole group by dense_tail (for short ranges; otherwise one by one, in less code).
+// U positions loaded at a time, in (ax, ay).  A sum that is not finite is formed again with care: a
+// group's product may have left the FP64 range where no single |d|^2 does.
+// PAD: the positions past the last U in one more group filled up (for short ranges; a serial chain of
+// reciprocals took 5 us of a batch step); otherwise one by one, in less code.
 template <bool REFINE, int U, bool PAD = false, class Src>
 __device__ __forceinline__ void dense_sum(Src src, const int j0, const int j1, const double px, const double py,
                                           double &ax, double &ay) {
-    constexpr int N = 8;  // pairs that share a reciprocal
-    static_assert(U % N == 0, "whole groups");
+    constexpr int N = GROUP;
+    static_assert(U % N == 0 && (!PAD || U == N), "whole groups");
     ax = ay = 0.0;
     int j = j0;
     for (; j + U <= j1; j += U) {
@@ -186,23 +202,25 @@ __device__ __forceinline__ void dense_sum(Src src, const int j0, const int j1, c
 #pragma unroll
         for (int k = 0; k < U; k += N) pair_rep_group<REFINE, N>(qx + k, qy + k, px, py, ax, ay);
     }
-    if constexpr (PAD) {
-        if (j < j1) dense_tail<REFINE, N>(src, j, j1, px, py, ax, ay);
-        j = j1;
+    if constexpr (PAD && REFINE) {
+        if (j < j1) add_group<N, false>(interleaved(src), j, 1, j1, px, py, ax, ay);
+    } else {
+        for (; j < j1; ++j) pair_rep<REFINE>(src[2 * j], src[2 * j + 1], px, py, ax, ay);
     }
-    for (; j < j1; ++j) pair_rep<REFINE>(src[2 * j], src[2 * j + 1], px, py, ax, ay);
     if (REFINE && !(isfinite(ax) && isfinite(ay))) {
         ax = ay = 0.0;
-        for (j = j0; j < j1; ++j) pair_rep<REFINE>(src[2 * j], src[2 * j + 1], px, py, ax, ay);
+        const int grouped = PAD ? j1 : j0 + (j1 - j0) / U * U;
+        for (j = j0; j < grouped; j += N) add_group<N, true>(interleaved(src), j, 1, j1, px, py, ax, ay);
+        for (; j < j1; ++j) pair_rep<REFINE>(src[2 * j], src[2 * j + 1], px, py, ax, ay);
     }
 }
 
 // The dense repulsion of (px, py) against positions j0, j0 + D, ... below n, added to (ax, ay): groups of 8
-// as dense_sum, the last one filled up as dense_tail.
+// as dense_sum, the last one filled up.
 template <bool REFINE, int D>
 __device__ __forceinline__ void strided_sum(const double2 *__restrict__ src, const int j0, const int n, const double px,
                                             const double py, double &ax, double &ay) {
-    constexpr int N = 8;
+    constexpr int N = GROUP;
     double sx = 0.0, sy = 0.0;
     int j = j0;
     for (; j + (N - 1) * D < n; j += N * D) {
@@ -215,26 +233,11 @@ __device__ __forceinline__ void strided_sum(const double2 *__restrict__ src, con
         pair_rep_group<REFINE, N>(qx, qy, px, py, sx, sy);
     }
     if constexpr (REFINE) {
-        if (j < n) {
-            double dx[N], dy[N], r[N];
-#pragma unroll
-            for (int k = 0; k < N; ++k) {
-                const bool in = j + k * D < n;
-                const double2 q = src[in ? j + k * D : j];
-                dx[k] = in ? q.x - px : 0.0;
-                dy[k] = in ? q.y - py : 0.0;
-                r[k] = in ? fma(dy[k], dy[k], fma(dx[k], dx[k], kTiny64)) : 1.0;
-            }
-            recip_all<N>(r);
-#pragma unroll
-            for (int k = 0; k < N; ++k) {
-                sx = fma(-dx[k], r[k], sx);
-                sy = fma(-dy[k], r[k], sy);
-            }
-        }
+        const auto at = [=](int q) { return src[q]; };
+        if (j < n) add_group<N, false>(at, j, D, n, px, py, sx, sy);
         if (!(isfinite(sx) && isfinite(sy))) {
             sx = sy = 0.0;
-            for (j = j0; j < n; j += D) pair_rep<true>(src[j].x, src[j].y, px, py, sx, sy);
+            for (j = j0; j < n; j += N * D) add_group<N, true>(at, j, D, n, px, py, sx, sy);
         }
     } else {
         for (; j < n; j += D) pair_rep<false>(src[j].x, src[j].y, px, py, sx, sy);
@@ -243,14 +246,80 @@ __device__ __forceinline__ void strided_sum(const double2 *__restrict__ src, con
     ay += sy;
 }
 
-// Neighbour correction for one (i, j) pair: removes the dense loop's product (dx * inv; with REFINE
-// to its last bits, of the order of the dense sum's own rounding) and adds the attraction.
+// The factor 1/|d|^2 that a dense sum gave the pair at place m of the group at(first), at(first + D), ...
+// below end, bit for bit: the products of recip_all, which are the same from every place of the group.
+template <class At>
+__device__ __forceinline__ double group_factor(At at, const int first, const int m, const int D, const int end,
+                                               const double px, const double py) {
+    double r[GROUP];
+    static_assert(GROUP == 8, "three levels of products");
+#pragma unroll
+    for (int k = 0; k < GROUP; ++k) {
+        const int j = first + (m ^ k) * D;
+        const double2 q = at(j < end ? j : first);
+        const double dx = q.x - px, dy = q.y - py;
+        r[k] = j < end ? fma(dy, dy, fma(dx, dx, kTiny64)) : 1.0;
+    }
+    const double two = r[2] * r[3], four = (r[4] * r[5]) * (r[6] * r[7]);
+    const double f = recip(((r[0] * r[1]) * two) * four) * four * two * r[1];
+    return isfinite(f) ? f : recip(r[0]);
+}
+
+// The factor to remove a linked pair (dx, dy) with: bit for bit the dense sum's where the pair is close (group:
+// whether it was in one).  Further away than 2^-4 one of its own, which differs by about 2^-52: less than the
+// roundings of the dense sum's additions after the pair.  (Eight loads for every neighbour made the step of the
+// 250k random geometric graph 4% longer: the correction's workgroups hold up the last of the others.)
+constexpr double kNear2 = 0x1p-8;
+template <bool REFINE, class At>
+__device__ __forceinline__ double linked_factor(At at, const bool group, const int first, const int m, const int D,
+                                                const int end, const double px, const double py, const double dx,
+                                                const double dy) {
+    if (REFINE && group && fma(dy, dy, dx * dx) < kNear2) return group_factor(at, first, m, D, end, px, py);
+    return inv_r2<REFINE>(dx, dy);
+}
+
+// A linked pair closer than 2^-40 (coincident ones aside, whose terms are 0): its repulsion, which the
+// reference never forms, would take the force's low digits with it when it is added and removed again.
+constexpr double kApart2 = 0x1p-80;
 template <bool REFINE>
-__device__ __forceinline__ void correct_pair(int law, double W, double dx, double dy, double &cx, double &cy) {
-    const double inv = inv_r2<REFINE>(dx, dy);
+__device__ __forceinline__ bool too_close(const double dx, const double dy) {
+    return REFINE && fma(dy, dy, dx * dx) < kApart2 && (dx != 0.0 || dy != 0.0);
+}
+
+// Neighbour correction for one (i, j) pair: removes the dense loop's product, formed from the same factor
+// `inv`, and adds the attraction.
+__device__ __forceinline__ void correct_pair(int law, double W, double dx, double dy, double inv, double &cx, double &cy) {
     cx += dx * inv;
     cy += dy * inv;
     attract64(law, W, dx, dy, cx, cy);
+}
+
+// A thread's share t, t + D, ... of the whole force on position (px, py) of a vertex whose neighbours are
+// entries [e0, e1) of ci (ascending), one of them too close: such neighbours are not added at all.  Rare,
+// so a pair at a time.
+template <class At, class Weight>
+__device__ __forceinline__ double2 apart_share(At at, const int n, const int t, const int D, const double px,
+                                               const double py, const int *__restrict__ ci, const int e0, const int e1,
+                                               Weight weight, const int law) {
+    double fx = 0.0, fy = 0.0;
+    for (int j = t; j < n; j += D) {
+        const double2 q = at(j);
+        if (too_close<true>(q.x - px, q.y - py)) {
+            int lo = e0, hi = e1;  // the first neighbour >= j
+            while (lo < hi) {
+                const int m = (lo + hi) >> 1;
+                if (ci[m] < j) lo = m + 1; else hi = m;
+            }
+            if (lo < e1 && ci[lo] == j) continue;
+        }
+        pair_rep<true>(q.x, q.y, px, py, fx, fy);
+    }
+    for (int e = e0 + t; e < e1; e += D) {
+        const double2 q = at(ci[e]);
+        const double dx = q.x - px, dy = q.y - py;
+        correct_pair(law, weight(e), dx, dy, too_close<true>(dx, dy) ? 0.0 : inv_r2<true>(dx, dy), fx, fy);
+    }
+    return make_double2(fx, fy);
 }
 
 // x_i += (F/|F|) * STEP, algorithms.cpp:775-779 / Coordinate.h:57-65.
