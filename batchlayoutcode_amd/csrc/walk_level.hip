@@ -18,13 +18,15 @@
 // needs it reads it until it has come.  So a level costs one store and one load through memory, about
 // 2.4 us, where a launch of its own cost 5 (two dependent loads past caches that a launch leaves empty, the
 // dispatch, the write-back), and the next levels' rows are loaded while they wait.  Workgroups take their
-// level and place in it by a ticket in level order: what a workgroup waits for was given to one that
-// started before it, so some workgroup can always go on.  Eight counters, one for each residue of the
-// workgroup's number (workgroups start in order on each XCD): with a single one the tickets themselves took
-// 13 ns each, 215 us on the triangulation.  A wait ends at a deadline, and the run with an error.
-//   - rows of up to 4 entries take 4 lanes each, rows of up to 8 take 8, at an address that the lane's
-//     number gives: a lane forms the factors of one entry, and the lanes' products are added one after
-//     another by DPP moves;
+// level and place in it by a ticket in level order, from one counter: what a workgroup waits for was given to
+// one that started before it, so some workgroup can always go on, whatever else runs on the device (with a
+// counter for each XCD two launches side by side can each fill the XCD whose next ticket the other waits
+// for).  A ticket takes 13 ns, one after another, so a workgroup takes as many rows as its lanes have
+// places for.  A wait ends at a deadline, and the run with an error.
+//   - rows of up to 4 entries take 4 lanes each, rows of up to 8 take 8, of up to 16 16, at an address that
+//     the lane's number gives: a lane forms the factors of one entry, and the lanes' products are added one
+//     after another by DPP moves (with rows of 9 to 16 entries one a wave the random geometric graph's walk
+//     took 5,183 tickets and 75 us, now 64; R-MAT 486 -> 460);
 //   - rows of up to LV_WAVE entries one a wave, longer ones (hubs) one a workgroup.
 // What bounds the walk: on R-MAT the hand-off of 188 levels; on the triangulation random 16-byte reads and
 // writes (1.66M moves in 195 us).  k_level_flow against a launch a level: R-MAT scale 20 at -batch 1024
@@ -54,27 +56,30 @@
 namespace bl {
 namespace {
 
-constexpr int LV_NARROW = 4, LV_WIDE = 8;  // lanes of a short row
+constexpr int LV_NARROW = 4, LV_WIDE = 8, LV_BROAD = 16;  // lanes of a short row
 constexpr int LV_WAVE = 512;      // longest row of one wave: 8 entries a lane (1, in list order)
 constexpr int LV_T = 512;         // threads of a level's workgroups: 8 slices or rows, or one hub
 constexpr int LV_WAVES = LV_T / 64;
 constexpr int LV_RUN = 2048;      // largest level of a run: 2 slices per wave of 1024 threads
 constexpr int LV_RUNS = 8;        // shortest run: a level in it takes 2-3 us, after about 15 us to start
-constexpr int LV_TICKETS = 8, LV_LINE = 32;  // ticket counters of a launch, ints between them
-constexpr int LV_TICKET_INTS = LV_TICKETS * LV_LINE;
+constexpr int LV_TICKET_INTS = 32;  // between the ticket counters of the launches
+// Blocks of a level from which a ticket stands for two: the triangulation's walk takes 232 us with one, 198 with
+// two, 214 with up to eight (from 256 blocks a ticket more), whose rows then wait for each other.
+constexpr int LV_PAIR = 512;
 constexpr int LV_MAXLEVELS = 1 << 16;
 constexpr int LV_LATE = 32;       // longest row of a slice of the late lists
 constexpr int LV_WINDOW = 4096;   // where rows are longer, these lists are sorted by length within such windows
 constexpr unsigned LV_PAD = 0x7fffffffu, LV_RECENT = 0x80000000u;
 constexpr int64_t LV_SHORT = (int64_t)1 << 62;  // host: marks a short row's place
 
-// A level in k_level_flow, its workgroups [first, end) from the last: nn waves of rows of 4 lanes (16 a
-// wave), then nw of rows of 8 (8 a wave), from vertex slot v0 and entry block e0 (64 entries each),
-// then nr rows from row r0, one a wave, then hubs, one a workgroup.
+// A level in k_level_flow, its `blocks` of 8 waves' work from the last, `per` of them to a workgroup from
+// the launch's number `first` on: nn waves of rows of 4 lanes (16 a wave), then nw of rows of 8 (8 a
+// wave) and nb of rows of 16, from vertex slot v0 and entry block e0 (64 entries each), then nr rows from
+// row r0, one a wave, then hubs, one a workgroup.
 struct LevelShape {
-    int v0, nn, nw, r0, nr;
+    int v0, nn, nw, nb, r0, nr;
     unsigned e0;
-    int first, end;
+    int first, blocks, per;
 };
 
 struct LevelArgs {
@@ -230,18 +235,18 @@ __device__ __forceinline__ void slice_pos(const LevelArgs &a, const unsigned *c,
     for (int g = 0; g < N; ++g) p[g] = a.pos[c[g] == LV_PAD ? own : (int)(c[g] & LV_PAD)];
 }
 
-// v of the lane before (row_shr:1; lane 0 of 16 gets 0, which no short row's lane takes).
+// v of the lane before (row_shr:1; lane 0 of 16 gets 0, and the first lane of a short row takes none).
 __device__ __forceinline__ double lane_before(double v) {
     const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x111, 0xF, 0xF, false);
     const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x111, 0xF, 0xF, false);
     return __hiloint2double(hi, lo);
 }
 
-// A wave of short rows, N lanes each: entry block `block`, the rows' vertices from slot vs.  Lane k
+// A wave of short rows (false: given up), N lanes each: entry block `block`, the rows' vertices from slot vs.  Lane k
 // of a row forms entry k's factors and adds its product to the sum of the lanes before it, in the
 // k-th of N steps; the repulsion is subtracted before the first recent entry, else at the end.
 template <bool HAS_W, int N>
-__device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t block) {
+__device__ __forceinline__ bool short_rows(const LevelArgs &a, int vs, size_t block) {
     const int lane = threadIdx.x & 63, k = lane & (N - 1);
     const int id = a.vid[vs + lane / N], i = max(id, 0);
     const size_t e = block * 64 + lane;
@@ -251,7 +256,7 @@ __device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t bl
     const double2 v = a.pos[i], r = a.rep[i];
     const int j = real ? (int)(c & LV_PAD) : i;
     double2 pj;
-    if (!moved_pos<1>(a, &j, &real, &pj)) return;
+    if (!moved_pos<1>(a, &j, &real, &pj)) return false;
     double dx, dy, sc;
     attr_factors(pj, v, Wk, dx, dy, sc);
     const unsigned rec = (unsigned)(__ballot(c >= LV_RECENT) >> (lane - k)) & ((1u << N) - 1);
@@ -266,9 +271,9 @@ __device__ __forceinline__ void short_rows(const LevelArgs &a, int vs, size_t bl
         const double sx = fma(dx, sc, px), sy = fma(dy, sc, py);
         if (k == g) f = make_double2(real ? sx : px, real ? sy : py);
     }
-    if (k != N - 1 || id < 0) return;
     if (rec == 0) f = make_double2(f.x - r.x, f.y - r.y);
-    move_vertex<true>(a, i, v, f);
+    if (k == N - 1 && id >= 0) move_vertex<true>(a, i, v, f);
+    return true;
 }
 
 // This thread's share of a row's sum: entries t, t + T, ..., eight loads in flight.
@@ -343,68 +348,77 @@ __device__ __forceinline__ void finish_row(const LevelArgs &a, bool one, int i, 
         move_vertex<true>(a, i, v, make_double2(f.x - r.x, f.y - r.y));
 }
 
-// Rows by workgroup b past the slices' workgroups: nr rows from row r0 one a wave, then hubs (a
-// fixed order of the sums: per lane, over the wave by DPP, over the waves in turn).
+// Rows by block b past the slices' blocks: nr rows from row r0 one a wave, then hubs (a
+// fixed order of the sums: per lane, over the wave by DPP, over the waves in turn).  False: given up (a
+// hub in all waves).
 template <bool HAS_W, bool LATE, bool SEQ>
-__device__ __forceinline__ void long_rows(const LevelArgs &a, int b, int r0, int nr, int bad) {
+__device__ __forceinline__ bool long_rows(const LevelArgs &a, int b, int r0, int nr, int bad) {
     __shared__ double2 red[LV_WAVES];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int rb = (nr + LV_WAVES - 1) / LV_WAVES;
     if (b < rb) {
         const int k = b * LV_WAVES + wave;
-        if (k >= nr) return;
+        if (k >= nr) return true;
         const int4 row = a.row[r0 + k];  // wave-uniform
         const double2 v = a.pos[row.x], r = a.rep[row.x];
         if constexpr (SEQ) {
             const double2 f = row_in_order<HAS_W>(a, row, lane, v, r, bad);
             if (lane == 0 && !bad) move_vertex<true>(a, row.x, v, f);
-            return;
+            return !bad;
         }
         double2 f = row_share<HAS_W, LATE, 64>(a, row, lane, v, bad);
         bad = __any(bad);
         f.x = wave_sum(f.x);
         f.y = wave_sum(f.y);
         finish_row<LATE>(a, lane == 0, row.x, v, r, f, bad);
-        return;
+        return !bad;
     }
     const int4 row = a.row[r0 + nr + b - rb];
     const double2 v = a.pos[row.x], r = a.rep[row.x];
     double2 f = row_share<HAS_W, LATE, LV_T>(a, row, (int)threadIdx.x, v, bad);
     f.x = wave_sum(f.x);
     f.y = wave_sum(f.y);
+    __syncthreads();  // the hub before has been added up
     if (lane == 0) red[wave] = f;
     bad = __syncthreads_or(bad);
     f = red[0];
 #pragma unroll
     for (int k = 1; k < LV_WAVES; ++k) f = add2(f, red[k]);
     finish_row<LATE>(a, threadIdx.x == 0, row.x, v, r, f, bad);
+    return !bad;
 }
 
 // Consecutive levels (SEQ: every row's sum in list order), the longest rows of each first.
 template <bool HAS_W, bool SEQ>
 __global__ __launch_bounds__(LV_T) void k_level_flow(LevelArgs a) {
     __shared__ int tk;
-    if (threadIdx.x == 0) tk = (int)blockIdx.x;
-    if (threadIdx.x == 0 && a.ticket) {  // nullptr: a single level, nothing to wait for
-        const int x = (int)blockIdx.x % LV_TICKETS;
-        tk = x + LV_TICKETS * __hip_atomic_fetch_add(a.ticket + LV_LINE * x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (threadIdx.x == 0)  // nullptr: a single level, nothing to wait for
+        tk = a.ticket ? __hip_atomic_fetch_add(a.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (int)blockIdx.x;
     const int bad = *a.status;
     __syncthreads();
     if (bad) return;
     const int t = __builtin_amdgcn_readfirstlane(tk);
     const LevelShape q = a.shape[a.blk[t]];
-    const int b = q.end - 1 - t, nsb = (q.nn + q.nw + LV_WAVES - 1) / LV_WAVES;
-    if (b < nsb) {
-        const int k = __builtin_amdgcn_readfirstlane(b * LV_WAVES + ((int)threadIdx.x >> 6));
-        constexpr int RN = 64 / LV_NARROW, RW = 64 / LV_WIDE;  // rows a wave
-        if (k < q.nn)
-            short_rows<HAS_W, LV_NARROW>(a, q.v0 + RN * k, (size_t)q.e0 + k);
-        else if (k < q.nn + q.nw)
-            short_rows<HAS_W, LV_WIDE>(a, q.v0 + RN * q.nn + RW * (k - q.nn), (size_t)q.e0 + k);
-        return;
+    const int nsb = (q.nn + q.nw + q.nb + LV_WAVES - 1) / LV_WAVES;
+    const int end = q.blocks - (t - q.first) * q.per;
+    // hubs first, whose barriers every wave reaches: one that gives up at a row or slice meets no more of them
+    for (int b = end - 1; b >= max(0, end - q.per); --b) {
+        bool ok = true;
+        if (b < nsb) {
+            const int k = __builtin_amdgcn_readfirstlane(b * LV_WAVES + ((int)threadIdx.x >> 6));
+            constexpr int RN = 64 / LV_NARROW, RW = 64 / LV_WIDE, RB = 64 / LV_BROAD;  // rows a wave
+            const int wide = q.v0 + RN * q.nn, broad = wide + RW * q.nw;
+            if (k < q.nn)
+                ok = short_rows<HAS_W, LV_NARROW>(a, q.v0 + RN * k, (size_t)q.e0 + k);
+            else if (k < q.nn + q.nw)
+                ok = short_rows<HAS_W, LV_WIDE>(a, wide + RW * (k - q.nn), (size_t)q.e0 + k);
+            else if (k < q.nn + q.nw + q.nb)
+                ok = short_rows<HAS_W, LV_BROAD>(a, broad + RB * (k - q.nn - q.nw), (size_t)q.e0 + k);
+        } else {
+            ok = long_rows<HAS_W, false, SEQ>(a, b - nsb, q.r0, q.nr, 0);
+        }
+        if (!ok) return;
     }
-    long_rows<HAS_W, false, SEQ>(a, b - nsb, q.r0, q.nr, 0);
 }
 
 // What k_level_late leaves for an iteration's k_level_flow: no vertex has moved, no workgroup has a ticket.
@@ -649,12 +663,12 @@ bool build_plan(bl_graph *g, int B, int D) {
             nl = std::max(nl, top + 2);
         }
     if (nl > LV_MAXLEVELS) return false;
-    // within a level: rows for slices of 4 and of 8 columns, rows of a wave, hubs (the lagged walk's
-    // rows, whose sums stay in list order, have at most 64 entries)
-    constexpr int K = 4;
+    // within a level: rows of 4, 8 and 16 lanes, rows of a wave, hubs (the lagged walk's rows, whose sums
+    // stay in list order, have at most 64 entries)
+    constexpr int K = 5;
     if (D > 0 && g->max_row > 64) return false;
     auto cls = [&](int i) {
-        return (size_t)lev[i] * K + (ec[i] <= LV_NARROW ? 0 : ec[i] <= LV_WIDE ? 1 : ec[i] <= LV_WAVE ? 2 : 3);
+        return (size_t)lev[i] * K + (ec[i] <= LV_NARROW ? 0 : ec[i] <= LV_WIDE ? 1 : ec[i] <= LV_BROAD ? 2 : ec[i] <= LV_WAVE ? 3 : 4);
     };
     std::vector<int32_t> first((size_t)nl * K + 1, 0), order(n);
     for (int i = 0; i < n; ++i) ++first[cls(i) + 1];
@@ -702,7 +716,9 @@ bool build_plan(bl_graph *g, int B, int D) {
     // the levels' launches: on their own, or runs of small levels without longer rows
     std::vector<int32_t> start;  // of each level of the runs, its first slice in its run, and the run's end
     auto count = [&](int l, int c) { return first[(size_t)l * K + c + 1] - first[(size_t)l * K + c]; };
-    auto small = [&](int l) { return count(l, 0) + count(l, 1) <= LV_RUN && count(l, 2) + count(l, 3) == 0; };
+    auto small = [&](int l) {
+        return count(l, 0) + count(l, 1) <= LV_RUN && count(l, 2) + count(l, 3) + count(l, 4) == 0;
+    };
     std::vector<LevelShape> shape;
     std::vector<int32_t> blk;  // of each workgroup of k_level_flow, its level
     g->lev_launch.clear();
@@ -734,11 +750,12 @@ bool build_plan(bl_graph *g, int B, int D) {
             q.v0 = v0;
             q.e0 = e0;
             q.nn = E.short_rows(vs, count(l, 0), LV_NARROW);
-            q.nw = E.short_rows(vs + count(l, 0), count(l, 1), LV_WIDE);
-            vs += count(l, 0) + count(l, 1);
+            q.nw = E.short_rows(vs += count(l, 0), count(l, 1), LV_WIDE);
+            q.nb = E.short_rows(vs += count(l, 1), count(l, 2), LV_BROAD);
+            vs += count(l, 2);
             q.r0 = (int)E.L.row.size();
-            q.nr = count(l, 2);
-            const int nh = count(l, 3);
+            q.nr = count(l, 3);
+            const int nh = count(l, 4);
             for (int t = 0; t < q.nr + nh; ++t) E.row(vs[t], ec[vs[t]]);
             if (g->lev_launch.empty() || g->lev_launch.back().l1 > g->lev_launch.back().l0) {
                 LevelLaunch f{};
@@ -747,8 +764,10 @@ bool build_plan(bl_graph *g, int B, int D) {
             }
             LevelLaunch &f = g->lev_launch.back();
             q.first = f.blocks;
-            f.blocks = q.end = f.blocks + level_blocks(q.nn + q.nw, q.nr, nh);
-            blk.insert(blk.end(), (size_t)(q.end - q.first), (int32_t)shape.size());
+            q.blocks = level_blocks(q.nn + q.nw + q.nb, q.nr, nh);
+            q.per = q.blocks < LV_PAIR ? 1 : 2;
+            f.blocks += (q.blocks + q.per - 1) / q.per;
+            blk.insert(blk.end(), (size_t)(f.blocks - q.first), (int32_t)shape.size());
             shape.push_back(q);
             ++f.levels;
             ++g->lev_big;
