@@ -35,7 +35,7 @@
 // writes a buffer again only after the next step's count, when all have read it.  The teams take the
 // first places of the queue and together at most the workgroups that run at once, so their members
 // start together.  Where they don't (the device is busy with other launches), a wait ends at a
-// deadline, the teams give up, and a second launch without teams lays out their graphs, whose
+// deadline, its team gives up (the others go on), and a second launch without teams lays out its graph, whose
 // positions in memory are still the initial ones.  Launches of graphs of 64..8192
 // vertices, 20 iterations, without and with teams: 16 graphs 97.0 and 16.1 ms, 200 (-batch 64) 108 and
 // 35.7, 1,500 107 and 83.9.
@@ -88,7 +88,7 @@ struct BatchedArgs {
     const int *team_at;        // a team's place in parts and arrived
     double2 *parts;            // [team][2][MAXTEAM][B] members' partials, by step parity
     int *arrived;              // [team] members that stored their partials, summed over the steps
-    int *err;                  // a wait that ran out
+    int *err;                  // [team] a wait that ran out
     long long ticks;           // longest wait
     const int *voff;           // vertex offsets [count+1]
     const int *rp;             // row pointers over all vertices (global entry ids)
@@ -180,14 +180,14 @@ __device__ __forceinline__ double lanes_sum(double v, int count) {
     return v;
 }
 
-// Waits until `need` arrivals are counted, in thread 0; false at the deadline or
-// after another wait's.
-__device__ __forceinline__ bool team_wait(const BatchedArgs &a, int *arrived, int need) {
+// Waits until `need` arrivals of team `at` are counted, in thread 0; false at the deadline or
+// after another member's.
+__device__ __forceinline__ bool team_wait(const BatchedArgs &a, int at, int need) {
     const long long t0 = wall_clock64();
-    while (__hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
-        if (__hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
+    while (__hip_atomic_load(a.arrived + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
+        if (__hip_atomic_load(a.err + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
         if (wall_clock64() - t0 > a.ticks) {
-            atomicOr(a.err, 1);
+            atomicOr(a.err + at, 1);
             return false;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -293,7 +293,7 @@ __device__ void layout_graph(const BatchedArgs &a, int g, int me, int T, double2
                 __syncthreads();
                 if (tid == 0) {
                     __hip_atomic_fetch_add(a.arrived + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    *go = team_wait(a, a.arrived + at, (need + 1) * T);
+                    *go = team_wait(a, at, (need + 1) * T);
                 }
                 __syncthreads();
                 if (!__builtin_amdgcn_readfirstlane(*go)) return;
@@ -523,7 +523,7 @@ int run_batched(int32_t count, const int32_t *voff, const int64_t *eoff, const i
     const size_t b_order = 8 * items.size(), b_voff = 4 * (size_t)(count + 1), b_erp = 4 * (size_t)(N + 1),
                  b_eci = 4 * std::max<size_t>(1, nnz), b_pos = 16 * (size_t)N, b_en = 8 * (size_t)count,
                  b_fin = 8 * (size_t)count, b_wg = 8 * (size_t)grid, b_q = 64, b_ipw = 4 * (size_t)count,
-                 b_arr = 4 * (size_t)(teams + 1),
+                 b_arr = 4 * (size_t)std::max(1, 2 * teams),
                  b_parts = sizeof(double2) * 2 * MAXTEAM * p->batch * (size_t)teams;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
     const size_t total = al(b_order) + al(b_voff) + 2 * al(b_erp) + al(b_eci) + al(b_pos) + al(b_en) + al(b_fin) +
@@ -543,7 +543,7 @@ int run_batched(int32_t count, const int32_t *voff, const int64_t *eoff, const i
     int *d_ipw = reinterpret_cast<int *>(c); c += al(b_ipw);
     int *d_team = reinterpret_cast<int *>(c); c += al(b_ipw);
     int *d_team_at = reinterpret_cast<int *>(c); c += al(b_ipw);
-    int *d_arr = reinterpret_cast<int *>(c); c += al(b_arr);  // the teams' counts, then the error flag
+    int *d_arr = reinterpret_cast<int *>(c); c += al(b_arr);  // the teams' counts, then their error flags
     double2 *d_parts = reinterpret_cast<double2 *>(c); c += al(b_parts);
     int2 *d_titems = reinterpret_cast<int2 *>(c);  // a size class's sample graphs (tuning)
     BL_HIP(hipMemcpyAsync(d_items, items.data(), b_order, hipMemcpyHostToDevice, s));
@@ -686,22 +686,18 @@ int run_batched(int32_t count, const int32_t *voff, const int64_t *eoff, const i
     std::vector<long long> fin(count), wg(grid);
     BL_HIP(hipMemcpyAsync(wg.data(), d_wg, b_wg, hipMemcpyDeviceToHost, s));
     if (teams) {
-        int gave_up = 0;
-        BL_HIP(hipMemcpyAsync(&gave_up, a.err, sizeof(int), hipMemcpyDeviceToHost, s));
         BL_HIP(hipMemcpyAsync(fin.data(), d_fin, b_fin, hipMemcpyDeviceToHost, s));
         BL_HIP(hipStreamSynchronize(s));
-        if (gave_up) {  // the graphs that no team finished, without teams
-            items.clear();
-            for (int q = 0; q < count; ++q)
-                if (!fin[order[q]]) items.push_back(make_int2(order[q], 0));
-            if (!items.empty()) {
-                BL_HIP(hipMemcpyAsync(d_items, items.data(), 8 * items.size(), hipMemcpyHostToDevice, s));
-                BL_HIP(hipMemsetAsync(d_q, 0, b_q, s));
-                a.count = (int)items.size();
-                a.team = nullptr;
-                hipLaunchKernelGGL(kernel, dim3(std::min((int)items.size(), grid)), dim3(BT), dyn, s, a);
-                BL_HIP(hipGetLastError());
-            }
+        items.clear();  // the graphs of the teams that gave up, without teams
+        for (int q = 0; q < count; ++q)
+            if (!fin[order[q]]) items.push_back(make_int2(order[q], 0));
+        if (!items.empty()) {
+            BL_HIP(hipMemcpyAsync(d_items, items.data(), 8 * items.size(), hipMemcpyHostToDevice, s));
+            BL_HIP(hipMemsetAsync(d_q, 0, b_q, s));
+            a.count = (int)items.size();
+            a.team = nullptr;
+            hipLaunchKernelGGL(kernel, dim3(std::min((int)items.size(), grid)), dim3(BT), dyn, s, a);
+            BL_HIP(hipGetLastError());
         }
     }
     BL_HIP(hipEventRecord(e1, s));

@@ -1,5 +1,5 @@
 """Two handles at once from two threads, as the C ABI allows: kernels whose workgroups wait for each other
-(the level walk) side by side on the device.  Every result is the one that the
+(the level walk, the batched launch's teams) side by side on the device.  Every result is the one that the
 same call gives alone, and none runs into a deadline."""
 import threading
 
@@ -48,3 +48,20 @@ def test_two_level_walks_at_once(bl):
         for xy, st in got[k]:
             assert np.array_equal(xy, alone[k][0]) and st.energy == alone[k][1].energy
         handles[k].close()
+
+
+def test_two_batched_launches_at_once(bl):
+    sets = []
+    for seed in (1, 2):
+        rng = np.random.default_rng(seed)
+        gs, xs = [], []
+        for n in rng.integers(200, 8192, 60):
+            e = rng.integers(0, n, (4 * n, 2))
+            gs.append(graphs.csr_from_edges(int(n), e[e[:, 0] != e[:, 1]]))
+            xs.append(rng.random((int(n), 2)))
+        sets.append((gs, xs))
+    print("[case] two batched launches at once", flush=True)
+    alone, got = _both([lambda s=s: bl.run_batched(*s, algo=2, iters=10, batch=128) for s in sets], 4)
+    for k in (0, 1):
+        for out, en, _, _ in got[k]:
+            assert all(np.array_equal(a, b) for a, b in zip(out, alone[k][0])) and np.array_equal(en, alone[k][1])
