@@ -180,11 +180,11 @@ __device__ __forceinline__ double lanes_sum(double v, int count) {
     return v;
 }
 
-// Waits until `need` arrivals of team `at` are counted, in thread 0; false at the deadline or
-// after another member's.
-__device__ __forceinline__ bool team_wait(const BatchedArgs &a, int at, int need) {
+// Waits until `need` arrivals of team `at` are counted (modulo 2^32, which 134 million steps of a team of 16
+// reach), in thread 0; false at the deadline or after another member's.
+__device__ __forceinline__ bool team_wait(const BatchedArgs &a, int at, unsigned need) {
     const long long t0 = wall_clock64();
-    while (__hip_atomic_load(a.arrived + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
+    while ((int)((unsigned)__hip_atomic_load(a.arrived + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - need) < 0) {
         if (__hip_atomic_load(a.err + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
         if (wall_clock64() - t0 > a.ticks) {
             atomicOr(a.err + at, 1);
@@ -222,7 +222,7 @@ __device__ void layout_graph(const BatchedArgs &a, int g, int me, int T, double2
     const int at = T > 1 ? __builtin_amdgcn_readfirstlane(a.team_at[g]) : 0;
     double2 *parts = a.parts + (size_t)at * 2 * MAXTEAM * B;
     const int share = max(1, T / L);          // members whose subtrees a lane of a row adds
-    int need = 0;
+    unsigned need = 0;
     double step = scalar(a.step0), E = 0.0;  // in scalar registers: the vector ones are short
     auto ends = [&](int b) {  // this row's entries in batch b
         const int i = v0 + min(n - 1, b * B + row);
@@ -293,7 +293,7 @@ __device__ void layout_graph(const BatchedArgs &a, int g, int me, int T, double2
                 __syncthreads();
                 if (tid == 0) {
                     __hip_atomic_fetch_add(a.arrived + at, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    *go = team_wait(a, at, (need + 1) * T);
+                    *go = team_wait(a, at, (unsigned)(need + 1) * (unsigned)T);
                 }
                 __syncthreads();
                 if (!__builtin_amdgcn_readfirstlane(*go)) return;
