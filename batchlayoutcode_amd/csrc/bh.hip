@@ -2756,7 +2756,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         if (rc) return rc;
         if (use_level) {
             prof.begin(5);
-            rc = launch_level_late(g, pos, p, it, s);
+            rc = launch_level_late(g, pos, p, use_wide, it, s);
             prof.end();
             if (rc) return rc;
         } else if (p->precision != BL_PREC_FP64 && !use_grid && use_row) {
@@ -2777,7 +2777,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         } else if (use_level) {
             walk = use_wide ? BL_WALK_WIDE : use_grid ? BL_WALK_GRID : use_lag ? BL_WALK_LAG
                    : use_row ? BL_WALK_ROW : p->batch <= WALK_MAXB ? BL_WALK_PF : BL_WALK_SPLIT;
-            rc = launch_walk_level(g, pos, p, STEP, s);
+            rc = launch_walk_level(g, pos, p, use_wide, STEP, s);
             if (rc) return rc;
         } else if (use_wide) {
             walk = BL_WALK_WIDE;

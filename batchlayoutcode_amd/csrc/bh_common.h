@@ -140,10 +140,11 @@ void batch_scan(bl_graph *g, int B);
 
 // The walk by dependence levels (walk_level.hip): level_walk_plan builds the plan for batch size B
 // (D > 0: with the sums of the lagged walk at lag D); launch_level_late sums the late attraction
-// into the repulsion, launch_walk_level runs one iteration's walk after it.
+// into the repulsion, launch_walk_level runs one iteration's walk after it (fast: the operations of the
+// wide walk, else with D = 0 those of the row walk).
 bool level_walk_plan(bl_graph *g, int B, int D);
-int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, int it, hipStream_t s);
-int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, double step, hipStream_t s);
+int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, bool fast, int it, hipStream_t s);
+int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, bool fast, double step, hipStream_t s);
 constexpr int BH_LEVEL_ERR = 10;  // of BHWork::misc: the level walk gave up (cleared in iteration 0)
 
 // The lagged batch walk (walk_lag.hip): lag_walk_choose gives the default lag for batches of B

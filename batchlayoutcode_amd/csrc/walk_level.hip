@@ -42,7 +42,9 @@
 //
 // Graphs for which the lagged walk (walk_lag.hip) is chosen keep its sums bit for bit: the
 // early neighbours at least D groups back ("settled") are summed first, the repulsion is
-// subtracted, then the others ("recent", marked in the entry) are added.
+// subtracted, then the others ("recent", marked in the entry) are added; |d| and the unit vector by rsqrt2
+// (late terms by the IEEE square root).  Those for which the wide walk (walk_wide.hip) is chosen have all by
+// rsqrt2, as it has.  All others have IEEE roots and divisions, as the row, entry-split and split walks.
 #include <math.h>
 #include <stdlib.h>
 
@@ -141,14 +143,20 @@ __device__ __forceinline__ void store_moved(double2 *p, double2 q) {
     __asm__ volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
 }
 
-// x_i += (F/|F|) * STEP (:1062-1066), the unit vector F * rsqrt2(|F|^2): the lagged walk's operations.
+// x_i += (F/|F|) * STEP (:1062-1066).  IEEE: root and divisions as the row, entry-split and split walks form
+// them; else the unit vector F * rsqrt2(|F|^2), the lagged and the wide walk's operations.
 // FLOW: published for the workgroups of the same launch, else for later launches if there are any that
 // read it (a.moved).
-template <bool FLOW>
+template <bool FLOW, bool IEEE>
 __device__ __forceinline__ void move_vertex(const LevelArgs &a, int i, double2 v, double2 f) {
     const double m2 = f.x * f.x + f.y * f.y;
-    const double r = rsqrt2(m2) * a.step;
-    const double2 q = make_double2(fma(f.x, r, v.x), fma(f.y, r, v.y));
+    double2 q;
+    if constexpr (IEEE) {
+        q = moved(v, f.x, f.y, a.step);
+    } else {
+        const double r = rsqrt2(m2) * a.step;
+        q = make_double2(fma(f.x, r, v.x), fma(f.y, r, v.y));
+    }
     const double2 m = make_double2(is_none(q.x) ? NAN : q.x, is_none(q.y) ? NAN : q.y);
     if constexpr (FLOW) store_moved(a.moved + i, m);
     else if (a.moved) a.moved[i] = m;
@@ -178,28 +186,30 @@ __device__ __forceinline__ bool moved_pos(const LevelArgs &a, const int *j, cons
     }
 }
 
-// The late term: |d| by the IEEE square root where the graph keeps the lagged walk's sums.
+// A neighbour's difference and the factor of its attraction W|d| d, |d| by the IEEE square root or rsqrt2.
 template <bool IEEE>
-__device__ __forceinline__ void late_add(double2 pj, double2 v, double Wk, double &ax, double &ay) {
+__device__ __forceinline__ void factors(double2 pj, double2 v, double Wk, double &dx, double &dy, double &sc) {
     if constexpr (IEEE) {
-        const double dx = pj.x - v.x, dy = pj.y - v.y;
-        const double sc = Wk * sqrt(dx * dx + dy * dy);
-        ax = fma(dx, sc, ax);
-        ay = fma(dy, sc, ay);
+        dx = pj.x - v.x;
+        dy = pj.y - v.y;
+        sc = Wk * sqrt(dx * dx + dy * dy);
     } else {
-        attr_add(pj, v, Wk, ax, ay);
+        attr_factors(pj, v, Wk, dx, dy, sc);
     }
 }
 
 // The sums so far and one more term, kept if `on`.
+template <bool IEEE>
 __device__ __forceinline__ void add_if(bool on, double2 pj, double2 v, double Wk, double2 &f) {
-    double x = f.x, y = f.y;
-    attr_add(pj, v, Wk, x, y);
+    double dx, dy, sc;
+    factors<IEEE>(pj, v, Wk, dx, dy, sc);
+    const double x = fma(dx, sc, f.x), y = fma(dy, sc, f.y);
     f.x = on ? x : f.x;
     f.y = on ? y : f.y;
 }
 
 // Early sum of one vertex: settled entries, then - r at the first recent one (or at the end).
+template <bool IEEE>
 struct EarlySum {
     double2 f{0.0, 0.0};
     bool less = false;
@@ -210,7 +220,7 @@ struct EarlySum {
     }
     __device__ __forceinline__ void add(unsigned c, double2 pj, double2 v, double2 r, double Wk) {
         subtract(c >= LV_RECENT && !less, r);
-        add_if(c != LV_PAD, pj, v, Wk, f);
+        add_if<IEEE>(c != LV_PAD, pj, v, Wk, f);
     }
     __device__ __forceinline__ double2 total(double2 r) {
         subtract(!less, r);
@@ -245,7 +255,7 @@ __device__ __forceinline__ double lane_before(double v) {
 // A wave of short rows (false: given up), N lanes each: entry block `block`, the rows' vertices from slot vs.  Lane k
 // of a row forms entry k's factors and adds its product to the sum of the lanes before it, in the
 // k-th of N steps; the repulsion is subtracted before the first recent entry, else at the end.
-template <bool HAS_W, int N>
+template <bool HAS_W, int N, bool IEEE>
 __device__ __forceinline__ bool short_rows(const LevelArgs &a, int vs, size_t block) {
     const int lane = threadIdx.x & 63, k = lane & (N - 1);
     const int id = a.vid[vs + lane / N], i = max(id, 0);
@@ -258,7 +268,7 @@ __device__ __forceinline__ bool short_rows(const LevelArgs &a, int vs, size_t bl
     double2 pj;
     if (!moved_pos<1>(a, &j, &real, &pj)) return false;
     double dx, dy, sc;
-    attr_factors(pj, v, Wk, dx, dy, sc);
+    factors<IEEE>(pj, v, Wk, dx, dy, sc);
     const unsigned rec = (unsigned)(__ballot(c >= LV_RECENT) >> (lane - k)) & ((1u << N) - 1);
     const bool first = rec != 0 && (int)__builtin_ctz(rec) == k;
     const double rx = first ? r.x : 0.0, ry = first ? r.y : 0.0;
@@ -272,13 +282,13 @@ __device__ __forceinline__ bool short_rows(const LevelArgs &a, int vs, size_t bl
         if (k == g) f = make_double2(real ? sx : px, real ? sy : py);
     }
     if (rec == 0) f = make_double2(f.x - r.x, f.y - r.y);
-    if (k == N - 1 && id >= 0) move_vertex<true>(a, i, v, f);
+    if (k == N - 1 && id >= 0) move_vertex<true, IEEE>(a, i, v, f);
     return true;
 }
 
 // This thread's share of a row's sum: entries t, t + T, ..., eight loads in flight.
 // LATE: their iteration-start positions, else the new ones (bad: given up).
-template <bool HAS_W, bool LATE, int T>
+template <bool HAS_W, bool LATE, bool IEEE, int T>
 __device__ __forceinline__ double2 row_share(const LevelArgs &a, int4 row, int t, double2 v, int &bad) {
     constexpr int N = 8;
     double2 f = make_double2(0.0, 0.0);
@@ -303,7 +313,7 @@ __device__ __forceinline__ double2 row_share(const LevelArgs &a, int4 row, int t
         }
 #pragma unroll
         for (int g = 0; g < N; ++g)
-            add_if(on[g], p[g], v, HAS_W ? a.W * (double)w[g] : a.W, f);
+            add_if<IEEE>(on[g], p[g], v, HAS_W ? a.W * (double)w[g] : a.W, f);
     }
     return f;
 }
@@ -339,19 +349,19 @@ __device__ __forceinline__ double2 row_in_order(const LevelArgs &a, int4 row, in
 }
 
 // A row's wave or workgroup has its sum f in `one` thread: the late sum, or the move.
-template <bool LATE>
+template <bool LATE, bool IEEE>
 __device__ __forceinline__ void finish_row(const LevelArgs &a, bool one, int i, double2 v, double2 r, double2 f, int bad) {
     if (!one || bad) return;
     if constexpr (LATE)
         a.rep[i] = make_double2(r.x - f.x, r.y - f.y);
     else
-        move_vertex<true>(a, i, v, make_double2(f.x - r.x, f.y - r.y));
+        move_vertex<true, IEEE>(a, i, v, make_double2(f.x - r.x, f.y - r.y));
 }
 
 // Rows by block b past the slices' blocks: nr rows from row r0 one a wave, then hubs (a
 // fixed order of the sums: per lane, over the wave by DPP, over the waves in turn).  False: given up (a
 // hub in all waves).
-template <bool HAS_W, bool LATE, bool SEQ>
+template <bool HAS_W, bool LATE, bool SEQ, bool IEEE>
 __device__ __forceinline__ bool long_rows(const LevelArgs &a, int b, int r0, int nr, int bad) {
     __shared__ double2 red[LV_WAVES];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -363,19 +373,19 @@ __device__ __forceinline__ bool long_rows(const LevelArgs &a, int b, int r0, int
         const double2 v = a.pos[row.x], r = a.rep[row.x];
         if constexpr (SEQ) {
             const double2 f = row_in_order<HAS_W>(a, row, lane, v, r, bad);
-            if (lane == 0 && !bad) move_vertex<true>(a, row.x, v, f);
+            if (lane == 0 && !bad) move_vertex<true, IEEE>(a, row.x, v, f);
             return !bad;
         }
-        double2 f = row_share<HAS_W, LATE, 64>(a, row, lane, v, bad);
+        double2 f = row_share<HAS_W, LATE, IEEE, 64>(a, row, lane, v, bad);
         bad = __any(bad);
         f.x = wave_sum(f.x);
         f.y = wave_sum(f.y);
-        finish_row<LATE>(a, lane == 0, row.x, v, r, f, bad);
+        finish_row<LATE, IEEE>(a, lane == 0, row.x, v, r, f, bad);
         return !bad;
     }
     const int4 row = a.row[r0 + nr + b - rb];
     const double2 v = a.pos[row.x], r = a.rep[row.x];
-    double2 f = row_share<HAS_W, LATE, LV_T>(a, row, (int)threadIdx.x, v, bad);
+    double2 f = row_share<HAS_W, LATE, IEEE, LV_T>(a, row, (int)threadIdx.x, v, bad);
     f.x = wave_sum(f.x);
     f.y = wave_sum(f.y);
     __syncthreads();  // the hub before has been added up
@@ -384,13 +394,13 @@ __device__ __forceinline__ bool long_rows(const LevelArgs &a, int b, int r0, int
     f = red[0];
 #pragma unroll
     for (int k = 1; k < LV_WAVES; ++k) f = add2(f, red[k]);
-    finish_row<LATE>(a, threadIdx.x == 0, row.x, v, r, f, bad);
+    finish_row<LATE, IEEE>(a, threadIdx.x == 0, row.x, v, r, f, bad);
     return !bad;
 }
 
 // Consecutive levels (SEQ: every row's sum in list order), the longest rows of each first.
-template <bool HAS_W, bool SEQ>
-__global__ __launch_bounds__(LV_T) void k_level_flow(LevelArgs a) {
+template <bool HAS_W, bool SEQ, bool IEEE>
+__global__ __launch_bounds__(LV_T, 4) void k_level_flow(LevelArgs a) {
     __shared__ int tk;
     if (threadIdx.x == 0)  // nullptr: a single level, nothing to wait for
         tk = a.ticket ? __hip_atomic_fetch_add(a.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (int)blockIdx.x;
@@ -409,13 +419,13 @@ __global__ __launch_bounds__(LV_T) void k_level_flow(LevelArgs a) {
             constexpr int RN = 64 / LV_NARROW, RW = 64 / LV_WIDE, RB = 64 / LV_BROAD;  // rows a wave
             const int wide = q.v0 + RN * q.nn, broad = wide + RW * q.nw;
             if (k < q.nn)
-                ok = short_rows<HAS_W, LV_NARROW>(a, q.v0 + RN * k, (size_t)q.e0 + k);
+                ok = short_rows<HAS_W, LV_NARROW, IEEE>(a, q.v0 + RN * k, (size_t)q.e0 + k);
             else if (k < q.nn + q.nw)
-                ok = short_rows<HAS_W, LV_WIDE>(a, wide + RW * (k - q.nn), (size_t)q.e0 + k);
+                ok = short_rows<HAS_W, LV_WIDE, IEEE>(a, wide + RW * (k - q.nn), (size_t)q.e0 + k);
             else if (k < q.nn + q.nw + q.nb)
-                ok = short_rows<HAS_W, LV_BROAD>(a, broad + RB * (k - q.nn - q.nw), (size_t)q.e0 + k);
+                ok = short_rows<HAS_W, LV_BROAD, IEEE>(a, broad + RB * (k - q.nn - q.nw), (size_t)q.e0 + k);
         } else {
-            ok = long_rows<HAS_W, false, SEQ>(a, b - nsb, q.r0, q.nr, 0);
+            ok = long_rows<HAS_W, false, SEQ, IEEE>(a, b - nsb, q.r0, q.nr, 0);
         }
         if (!ok) return;
     }
@@ -453,7 +463,7 @@ __global__ __launch_bounds__(LV_T) void k_level_late(LevelArgs a, int ns, int nr
         const int2 h = a.head[s];
         const int id = a.vid[s * 64 + lane], i = max(id, 0);
         const double2 v = a.pos[i], r = a.rep[i];
-        double ax = 0.0, ay = 0.0;
+        double2 f = make_double2(0.0, 0.0);
         for (int k0 = 0; k0 < h.y; k0 += N) {
             unsigned c[N];
             float w[N];
@@ -462,12 +472,12 @@ __global__ __launch_bounds__(LV_T) void k_level_late(LevelArgs a, int ns, int nr
             slice_pos<N>(a, c, i, p);
 #pragma unroll
             for (int g = 0; g < N; ++g)
-                if (c[g] != LV_PAD) late_add<IEEE>(p[g], v, HAS_W ? a.W * (double)w[g] : a.W, ax, ay);
+                add_if<IEEE>(c[g] != LV_PAD, p[g], v, HAS_W ? a.W * (double)w[g] : a.W, f);
         }
-        if (id >= 0 && !bad) a.rep[i] = make_double2(r.x - ax, r.y - ay);
+        if (id >= 0 && !bad) a.rep[i] = make_double2(r.x - f.x, r.y - f.y);
         return;
     }
-    long_rows<HAS_W, true, false>(a, (int)blockIdx.x - nsb, 0, nr, bad);
+    long_rows<HAS_W, true, false, IEEE>(a, (int)blockIdx.x - nsb, 0, nr, bad);
 }
 
 // Levels [l0, l1) of at most LV_RUN vertices in slices of 8 columns (the run's first vertex slot is
@@ -476,7 +486,7 @@ __global__ __launch_bounds__(LV_T) void k_level_late(LevelArgs a, int ns, int nr
 // own position (only its own level moves it) and repulsion one; after the barrier a level is one
 // round trip for its neighbours' positions, the sums and the stores.  The workgroup's waves share
 // one L1, so a barrier after the stores is all the order they need.
-template <bool HAS_W>
+template <bool HAS_W, bool IEEE>
 __global__ __launch_bounds__(1024) void k_level_run(LevelArgs a, int l0, int l1, int v0, unsigned e0) {
     constexpr int PER = LV_RUN / 1024, G = LV_WIDE;
     if (__builtin_amdgcn_readfirstlane(*a.status)) return;
@@ -524,7 +534,7 @@ __global__ __launch_bounds__(1024) void k_level_run(LevelArgs a, int l0, int l1,
             if (__builtin_amdgcn_readfirstlane(__ballot(ido[j] >= 0) != 0)) {
                 double2 p[G];
                 slice_pos<G>(a, cur[j].c, max(ido[j], 0), p);
-                EarlySum sum;
+                EarlySum<IEEE> sum;
 #pragma unroll
                 for (int g = 0; g < G; ++g) {
                     if (!__ballot(cur[j].c[g] != LV_PAD)) break;  // rows fill the columns in order
@@ -539,7 +549,7 @@ __global__ __launch_bounds__(1024) void k_level_run(LevelArgs a, int l0, int l1,
         entries(l + 2, nxt);
 #pragma unroll
         for (int j = 0; j < PER; ++j)
-            if (ido[j] >= 0) move_vertex<false>(a, ido[j], vo[j], f[j]);
+            if (ido[j] >= 0) move_vertex<false, IEEE>(a, ido[j], vo[j], f[j]);
         __syncthreads();
     }
 }
@@ -873,8 +883,8 @@ LevelArgs level_args(const bl_graph *g, const LevelLists &d, double2 *pos, const
 bool is_flow(const LevelLaunch &q) { return q.blocks > 0; }
 }  // namespace
 
-// The late sums, before any vertex moves (and the marks for k_level_flow).
-int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, int it, hipStream_t s) {
+// The late sums, before any vertex moves (and the marks for k_level_flow).  fast: the wide walk's operations.
+int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, bool fast, int it, hipStream_t s) {
     const LevelArgs a = level_args(g, g->lev_late, pos, p, 0.0);
     const int ns = g->lev_late_slices, nr = g->lev_late_rows;
     LevelClear q{level_blocks(ns, nr, g->lev_late_hubs), 0, 0, g->lev_ticket.as<int>(), it == 0};
@@ -885,9 +895,8 @@ int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, int it, hip
     }
     const int grid = q.late + (q.n + LV_T - 1) / LV_T;
     if (grid > 0) {
-        const bool ieee = g->lev_d > 0;
-        auto k = g->has_w ? (ieee ? k_level_late<true, true> : k_level_late<true, false>)
-                          : (ieee ? k_level_late<false, true> : k_level_late<false, false>);
+        auto k = g->has_w ? (fast ? k_level_late<true, false> : k_level_late<true, true>)
+                          : (fast ? k_level_late<false, false> : k_level_late<false, true>);
         hipLaunchKernelGGL(k, dim3(grid), dim3(LV_T), 0, s, a, ns, nr, q);
     }
     BL_HIP(hipGetLastError());
@@ -895,12 +904,19 @@ int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, int it, hip
 }
 
 // One iteration's walk (after launch_level_late).
-int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, double step, hipStream_t s) {
+int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, bool fast, double step, hipStream_t s) {
     LevelArgs a = level_args(g, g->lev_early, pos, p, step);
     int left = (int)std::count_if(g->lev_launch.begin(), g->lev_launch.end(), is_flow);
     int *ticket = g->lev_ticket.as<int>();
-    auto k = g->has_w ? (g->lev_d > 0 ? k_level_flow<true, true> : k_level_flow<true, false>)
-                      : (g->lev_d > 0 ? k_level_flow<false, true> : k_level_flow<false, false>);
+    const bool seq = g->lev_d > 0, ieee = !seq && !fast;
+    auto k = g->has_w ? (seq    ? k_level_flow<true, true, false>
+                         : fast ? k_level_flow<true, false, false>
+                                : k_level_flow<true, false, true>)
+                      : (seq    ? k_level_flow<false, true, false>
+                         : fast ? k_level_flow<false, false, false>
+                                : k_level_flow<false, false, true>);
+    auto run = g->has_w ? (ieee ? k_level_run<true, true> : k_level_run<true, false>)
+                        : (ieee ? k_level_run<false, true> : k_level_run<false, false>);
     for (const LevelLaunch &q : g->lev_launch) {
         if (is_flow(q)) {
             a.blk = g->lev_blk.as<int>() + q.b0;
@@ -910,8 +926,7 @@ int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, double step
             hipLaunchKernelGGL(k, dim3(q.blocks), dim3(LV_T), 0, s, a);
         } else {
             if (!left) a.moved = nullptr;
-            hipLaunchKernelGGL(g->has_w ? k_level_run<true> : k_level_run<false>, dim3(1), dim3(1024), 0, s, a, q.l0,
-                               q.l1, q.v0, q.e0);
+            hipLaunchKernelGGL(run, dim3(1), dim3(1024), 0, s, a, q.l0, q.l1, q.v0, q.e0);
         }
     }
     BL_HIP(hipGetLastError());
