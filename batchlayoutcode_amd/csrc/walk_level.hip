@@ -70,6 +70,7 @@ constexpr int LV_TICKET_INTS = 32;  // between the ticket counters of the launch
 constexpr int LV_PAIR = 512;
 constexpr int LV_MAXLEVELS = 1 << 16;
 constexpr int LV_LATE = 32;       // longest row of a slice of the late lists
+constexpr int LV_ROW = 64;        // longest row whose sums are kept in list order (the lagged walk's)
 constexpr int LV_WINDOW = 4096;   // where rows are longer, these lists are sorted by length within such windows
 constexpr unsigned LV_PAD = 0x7fffffffu, LV_RECENT = 0x80000000u;
 constexpr int64_t LV_SHORT = (int64_t)1 << 62;  // host: marks a short row's place
@@ -676,7 +677,7 @@ bool build_plan(bl_graph *g, int B, int D) {
     // within a level: rows of 4, 8 and 16 lanes, rows of a wave, hubs (the lagged walk's rows, whose sums
     // stay in list order, have at most 64 entries)
     constexpr int K = 5;
-    if (D > 0 && g->max_row > 64) return false;
+    if (D > 0 && g->max_row > LV_ROW) return false;
     auto cls = [&](int i) {
         return (size_t)lev[i] * K + (ec[i] <= LV_NARROW ? 0 : ec[i] <= LV_WIDE ? 1 : ec[i] <= LV_BROAD ? 2 : ec[i] <= LV_WAVE ? 3 : 4);
     };
@@ -785,7 +786,9 @@ bool build_plan(bl_graph *g, int B, int D) {
         }
         if (E.nid > cap * 32 || (int64_t)E.L.vid.size() > cap) return false;
     }
-    // the late lists: slices in vertex order, sorted by length within windows where rows are long
+    // the late lists: slices in vertex order, sorted by length within windows where rows are long (the lagged
+    // walk's sums all in slices, which add in list order)
+    const int sliced = D > 0 ? LV_ROW : LV_LATE;
     std::vector<int32_t> win, rows, hubs;
     auto late_len = [&](int i) { return rp[i + 1] - rp[i] - ec[i]; };
     const bool sorted = g->max_row > LV_LATE;
@@ -794,7 +797,7 @@ bool build_plan(bl_graph *g, int B, int D) {
         for (int i = w0; i < std::min(n, w0 + LV_WINDOW); ++i) {
             const int c = late_len(i);
             if (c > LV_WAVE) hubs.push_back(i);
-            else if (c > LV_LATE) rows.push_back(i);
+            else if (c > sliced) rows.push_back(i);
             else if (c > 0) win.push_back(i);
         }
         if (sorted)
@@ -806,7 +809,7 @@ bool build_plan(bl_graph *g, int B, int D) {
             L.L.head.push_back(make_int2((int)L.nid, W));
             L.slices(win.data() + t, m, W);
         }
-        if (L.nid > cap - 2 * LV_WINDOW * LV_LATE) return false;
+        if (L.nid > cap - 2 * LV_WINDOW * LV_ROW) return false;
     }
     for (int i : rows) L.row(i, late_len(i));
     for (int i : hubs) L.row(i, late_len(i));
