@@ -401,7 +401,7 @@ __device__ __forceinline__ bool long_rows(const LevelArgs &a, int b, int r0, int
 
 // Consecutive levels (SEQ: every row's sum in list order), the longest rows of each first.
 template <bool HAS_W, bool SEQ, bool IEEE>
-__global__ __launch_bounds__(LV_T, 4) void k_level_flow(LevelArgs a) {
+__global__ __launch_bounds__(LV_T) void k_level_flow(LevelArgs a) {
     __shared__ int tk;
     if (threadIdx.x == 0)  // nullptr: a single level, nothing to wait for
         tk = a.ticket ? __hip_atomic_fetch_add(a.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (int)blockIdx.x;
