@@ -43,7 +43,8 @@ class bl_params(C.Structure):
 class bl_stats(C.Structure):
     _fields_ = [("energy", C.c_double), ("iters_done", C.c_int32), ("status", C.c_int32),
                 ("seconds", C.c_double), ("step_final", C.c_double), ("kernel_ms", C.c_double * 8),
-                ("kernel_launches", C.c_int32 * 8), ("walk", C.c_int32), ("far_cells", C.c_int64),
+                ("kernel_launches", C.c_int32 * 8), ("walk", C.c_int32), ("walk_levels", C.c_int32),
+                ("far_cells", C.c_int64),
                 ("far_model_iters", C.c_int32), ("far_judge_err", C.c_float * 2), ("walk_helped", C.c_int32),
                 ("walk_lag", C.c_int32), ("nonfinite", C.c_int32)]
 
@@ -126,12 +127,13 @@ class Stats:
     walk_helped: int = 0
     walk_lag: int = 0
     nonfinite: int = 0
+    walk_levels: int = 0  # > 0: the walk moved by that many dependence levels
 
 
 def _stats(st: bl_stats) -> Stats:
     return Stats(st.energy, st.iters_done, st.seconds, st.step_final, tuple(st.kernel_ms),
                  tuple(st.kernel_launches), st.walk, st.far_cells, st.far_model_iters, tuple(st.far_judge_err),
-                 st.walk_helped, st.walk_lag, st.nonfinite)
+                 st.walk_helped, st.walk_lag, st.nonfinite, st.walk_levels)
 
 
 class Graph:

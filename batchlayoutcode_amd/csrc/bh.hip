@@ -2818,7 +2818,7 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
         STEP = STEP * 0.999;  // :1070
     }
     prof.report(st);
-    if (st) st->walk = walk;
+    if (st) st->walk = walk, st->walk_levels = use_level ? g->lev_big + g->lev_small : 0;
     unsigned long long cells = 0;
     if (far_mode && far_mode != FAR_EXACT && iters > 0)
         BL_HIP(hipMemcpyAsync(&cells, ncells, sizeof(cells), hipMemcpyDeviceToHost, s));

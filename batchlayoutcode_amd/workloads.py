@@ -41,7 +41,8 @@ def _run(tag, rp, ci, w, iters, profile, **kw):
                vertex_updates_per_s=n * iters / st.seconds, energy=st.energy, params=kw)
     if profile:
         rec["kernel_ms_per_iter"] = dict(zip(CLASSES, [m / iters for m in st.kernel_ms]))
-        rec.update(walk=st.walk, walk_lag=st.walk_lag, walk_batches_helped=st.walk_helped, far_cells=st.far_cells)
+        rec.update(walk=st.walk, walk_levels=st.walk_levels, walk_lag=st.walk_lag, walk_batches_helped=st.walk_helped,
+                   far_cells=st.far_cells)
     return rec
 
 

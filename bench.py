@@ -206,7 +206,7 @@ def c4_leg(args, torch, api, graphs):
             secs, st, sp, per_iter = timed(algo, q["theta"])
             res[name] = dict(theta=q["theta"], value=n * K / secs, ms_per_step=secs * 1e3 / K, energy=st.energy,
                              kernel_ms_per_iter=per_iter, far_cells_per_iter=sp.far_cells, walk=sp.walk,
-                             walk_lag=sp.walk_lag, walk_batches_helped=sp.walk_helped,
+                             walk_levels=sp.walk_levels, walk_lag=sp.walk_lag, walk_batches_helped=sp.walk_helped,
                              model_iterations=sp.far_model_iters if algo == api.ALGO_FAR_LEARNED else None,
                              judge_median_errors=(dict(learned=sp.far_judge_err[0], analytic=sp.far_judge_err[1])
                                                   if algo == api.ALGO_FAR_LEARNED else None))
@@ -219,7 +219,8 @@ def c4_leg(args, torch, api, graphs):
 
 
 WALK_KERNELS = {1: "k_attract_move", 2: "k_walk_pf", 3: "k_walk_split", 4: "k_late_attract + k_walk_row",
-                5: "k_walk_grid", 6: "k_level_late + k_level"}
+                5: "k_walk_grid", 6: "k_late_attract + k_walk_lag", 7: "k_walk_wide"}
+LEVEL_KERNELS = "k_level_late + k_level_flow + k_level_run"  # bl_stats.walk_levels > 0
 
 
 def c4_roofline(n, nnz, lp):
@@ -248,13 +249,15 @@ def c4_roofline(n, nnz, lp):
     bytes_per_iter = n * (4 + 16 + 16 + 16 + 8) + nnz * (4 + 16)
     achieved = bytes_per_iter / (walk_ms / 1e3) / 1e9
     traffic = None
-    return dict(bound="hbm", kernel=WALK_KERNELS.get(sp.walk, "walk"), achieved=achieved, peak=PEAK_HBM_GBS, unit="GB/s",
-                frac=achieved / PEAK_HBM_GBS, traffic=traffic, mean_launch_us=walk_ms * 1e3,
+    return dict(bound="hbm", kernel=LEVEL_KERNELS if sp.walk_levels else WALK_KERNELS.get(sp.walk, "walk"),
+                achieved=achieved, peak=PEAK_HBM_GBS, unit="GB/s", frac=achieved / PEAK_HBM_GBS, traffic=traffic,
+                mean_launch_us=walk_ms * 1e3,
                 launches=sp.kernel_launches[1], bytes_per_launch=bytes_per_iter,
                 note="algorithmic bytes of one iteration's attraction and move (4 B rowptr + 16 B own position + "
                      "16 B repulsion + 16 B written position + 8 B energy term per vertex, 4 B column id + 16 B "
                      "neighbour position per CSR entry) / mean time of the walk and its pre-pass; the walk is bound "
-                     "by the launches and the memory latency of its dependence levels, not by bytes")
+                     "by the memory latency of " + ("its dependence levels" if sp.walk_levels else "its steps") +
+                     ", not by bytes")
 
 
 def algo2_leg(args, torch, api, graphs):

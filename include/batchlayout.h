@@ -102,9 +102,11 @@ typedef struct {
     int32_t kernel_launches[8];
     /* Barnes-Hut family (algos 4, 6, 40-43): the batch walk that the graph's shape and the batch size
        select, one of BL_WALK_* (0 for the all-pairs algorithms).  Outside FP64 mode its batches move
-       by dependence levels where these are few (the same layout up to the order of partial sums;
-       for BL_WALK_LAG the same bits); the value names the selected walk either way */
+       by dependence levels where these are few (the same arithmetic; the same layout up to the order
+       of partial sums, for BL_WALK_LAG the same bits): walk_levels is then the number of levels, and
+       the walk named did not run itself; else it is 0 */
     int32_t walk;
+    int32_t walk_levels;
     /* algos 40, 42, 43: cells the far-field traversal accepted in the last iteration (with the
        learned model, the number of model evaluations); 0 otherwise */
     int64_t far_cells;
