@@ -287,7 +287,7 @@ __device__ void far_flush(const MlpLds &L, FarQueue &Q, int count, int lane, uin
 // one load of its line.  Accepting: 4^-depth < (theta / MAXMIN)^2 |c - p|^2.  On a triangulation of
 // 1.66M points, monopole at theta 0.4 2.02 -> 1.48 ms (754 nodes and 211 points a wave; 77% of the
 // cycles vector instructions), second order at theta 0.8 0.88 -> 0.67 ms.
-#define BL_FAR_NODE                                    \
+#define BL_FARTRAV_NODE                                \
     "s_lshl_b64 s[82:83], s[80:81], 6\n\t"             \
     "s_add_u32 s82, s82, %[cells0]\n\t"                \
     "s_addc_u32 s83, s83, %[cells1]\n\t"               \
@@ -296,10 +296,10 @@ __device__ void far_flush(const MlpLds &L, FarQueue &Q, int count, int lane, uin
     BL_TRAV_TEST("%[open2]")                           \
     "s_bcnt1_i32_b64 s92, s[86:87]\n\t"                \
     "s_add_u32 %[cnt], %[cnt], s92\n\t"
-#define BL_FAR_POINT BL_TRAV_RECIP("s_nop 0\n\t") BL_TRAV_ADD
+#define BL_FARTRAV_POINT BL_TRAV_RECIP("s_nop 0\n\t") BL_TRAV_ADD
 // the second-order term in d itself: |d|^-6 (A d + B d_perp), A = (dx^2 - dy^2)(Mxx - Myy) +
 // 4 dx dy Mxy, B = -2 (dx dy (Myy - Mxx) + (dx^2 - dy^2) Mxy); %[s] = |d|^-2
-#define BL_FAR_QUAD                                \
+#define BL_FARTRAV_QUAD                            \
     "v_mul_f64 %[t], %[dy], %[dy]\n\t"             \
     "v_fma_f64 %[t], %[dx], %[dx], -%[t]\n\t"      \
     "v_mul_f64 %[u], %[dx], %[dy]\n\t"             \
@@ -319,14 +319,14 @@ __device__ void far_flush(const MlpLds &L, FarQueue &Q, int count, int lane, uin
     "v_mul_f64 %[u], %[t], %[dx]\n\t"              \
     "v_fma_f64 %[u], %[r2], %[dy], %[u]\n\t"       \
     "v_fma_f64 %[fy], %[v], %[u], %[fy]\n\t"
-#define BL_FAR_MONO                                \
+#define BL_FARTRAV_MONO                            \
     BL_TRAV_RECIP("v_cvt_f64_i32 %[w], s74\n\t")   \
     "v_mul_f64 %[w], %[s], %[w]\n\t"               \
     "v_fma_f64 %[fx], %[dx], %[w], %[fx]\n\t"      \
     "v_fma_f64 %[fy], %[dy], %[w], %[fy]\n\t"
-#define BL_FAR_LOOP(term)                                                                                            \
-    __asm__ volatile(BL_TRAV_POP BL_FAR_NODE BL_TRAV_TAKE(term)                                                      \
-                     BL_TRAV_OPEN("s76", "s77", "s78", "s79", BL_FAR_POINT)                                          \
+#define BL_FARTRAV_LOOP(term)                                                                                        \
+    __asm__ volatile(BL_TRAV_POP BL_FARTRAV_NODE BL_TRAV_TAKE(term)                                                  \
+                     BL_TRAV_OPEN("s76", "s77", "s78", "s79", BL_FARTRAV_POINT)                                      \
                      "Lout%=:"                                                                                      \
                      : [node] "+v"(stk.node), [lo] "+v"(stk.lo), [hi] "+v"(stk.hi), [sp] "+s"(sp),                   \
                        [fx] "+v"(fx), [fy] "+v"(fy), [cnt] "+s"(cnt), [why] "=&s"(why), [dx] "=&v"(dx),              \
@@ -344,9 +344,9 @@ __device__ __forceinline__ void far_walk(WaveStack &stk, const FarCell *cells, c
         int why, sp = scalar(stk.sp), cnt = scalar(accepted);
         double dx, dy, r2, sv, t, u, v, w;
         if constexpr (QUAD)
-            BL_FAR_LOOP(BL_FAR_MONO BL_FAR_QUAD);
+            BL_FARTRAV_LOOP(BL_FARTRAV_MONO BL_FARTRAV_QUAD);
         else
-            BL_FAR_LOOP(BL_FAR_MONO);
+            BL_FARTRAV_LOOP(BL_FARTRAV_MONO);
         stk.sp = sp;
         accepted = cnt;
         why = scalar(why);

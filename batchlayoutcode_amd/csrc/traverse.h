@@ -106,9 +106,13 @@ struct WaveStack {
 // Wait states of gfx950 that an assembler does not insert: one between a reciprocal (or root) and its
 // use, one between the write of a vector register and its v_readlane, two between a vector
 // instruction's scalar result and its use as a vector operand; none of these pairs is closer here.
+// Four between a vector instruction's scalar result and its use as the lane of a v_readlane: %[sp]
+// comes in by v_readfirstlane, so the block begins with them; inside it %[sp] and m0 are the
+// scalar unit's.
 enum TravStop : int { TRAV_END = 0, TRAV_FULL = 1, TRAV_NEAR = 2 };
 
 #define BL_TRAV_POP                          \
+    "s_nop 3\n\t"                            \
     "s_mov_b32 s81, 0\n\t"                   \
     "s_mov_b32 s90, 0\n\t"                   \
     "s_mov_b32 %[why], 0\n"                  \
@@ -204,8 +208,9 @@ enum TravStop : int { TRAV_END = 0, TRAV_FULL = 1, TRAV_NEAR = 2 };
     "v_fma_f64 %[fx], %[dx], %[s], %[fx]\n\t"  \
     "v_fma_f64 %[fy], %[dy], %[s], %[fy]\n\t"
 
-#define BL_TRAV_CLOBBERS                                                                                          \
-    "vcc", "scc", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75", "s76",      \
-        "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89", "s90", "s91", "s92"
+#define BL_TRAV_CLOBBERS                                                                                     \
+    "vcc", "scc", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75",  \
+    "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89", "s90", \
+    "s91", "s92"
 
 }  // namespace bl
