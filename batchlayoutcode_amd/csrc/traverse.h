@@ -209,7 +209,7 @@ enum TravStop : int { TRAV_END = 0, TRAV_FULL = 1, TRAV_NEAR = 2 };
     "v_fma_f64 %[fy], %[dy], %[s], %[fy]\n\t"
 
 #define BL_TRAV_CLOBBERS                                                                                     \
-    "vcc", "scc", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75",  \
+    "vcc", "scc", "m0", "s64", "s65", "s66", "s67", "s68", "s69", "s70", "s71", "s72", "s73", "s74", "s75",  \
     "s76", "s77", "s78", "s79", "s80", "s81", "s82", "s83", "s84", "s85", "s86", "s87", "s88", "s89", "s90", \
     "s91", "s92"
 
