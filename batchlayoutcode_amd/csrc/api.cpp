@@ -182,9 +182,7 @@ extern "C" int bl_graph_destroy(bl_graph *g) {
                      &g->wide_npa, &g->wide_npb, &g->wide_ring_of, &g->wide_far_rp, &g->wide_far_ci, &g->wide_far_w,
                      &g->wide_chunks, &g->wide_cfr, &g->wide_nch, &g->wide_pre, &g->wide_cnt, &g->wide_sink};
     for (DevBuf *b : all) b->release();
-    g->lev_early.release();
-    g->lev_late.release();
-    for (DevBuf *b : {&g->lev_start, &g->lev_blk, &g->lev_shape, &g->lev_moved, &g->lev_ticket}) b->release();
+    level_walk_release(g);
     g->bh.release();
     if (g->stream) (void)hipStreamDestroy(g->stream);
     delete g;

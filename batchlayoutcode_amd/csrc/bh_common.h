@@ -143,6 +143,7 @@ void batch_scan(bl_graph *g, int B);
 // into the repulsion, launch_walk_level runs one iteration's walk after it (fast: the operations of the
 // wide walk, else with D = 0 those of the row walk).
 bool level_walk_plan(bl_graph *g, int B, int D);
+void level_walk_release(bl_graph *g);
 int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, bool fast, int it, hipStream_t s);
 int launch_walk_level(bl_graph *g, double2 *pos, const bl_params *p, bool fast, double step, hipStream_t s);
 constexpr int BH_LEVEL_ERR = 10;  // of BHWork::misc: the level walk gave up (cleared in iteration 0)

@@ -813,6 +813,8 @@ bool build_plan(bl_graph *g, int B, int D) {
     }
     for (int i : rows) L.row(i, late_len(i));
     for (int i : hubs) L.row(i, late_len(i));
+    const char *penv = getenv("BL_LEVEL_PAD_GIB");  // tests: more than there is
+    const size_t pad = penv ? (size_t)std::max(0, atoi(penv)) << 30 : 0;
     hipStream_t st = g->stream;
     struct Temp {
         DevBuf e, l, go;
@@ -820,7 +822,7 @@ bool build_plan(bl_graph *g, int B, int D) {
     } t;
     if (!E.L.upload(g->lev_early, gw, E.nid, E.nrid, st) || !L.L.upload(g->lev_late, gw, L.nid, L.nrid, st) ||
         !put(g->lev_start, start) || !put(g->lev_blk, blk) || !put(g->lev_shape, shape) ||
-        g->lev_moved.ensure(sizeof(double2) * (size_t)n) ||
+        g->lev_moved.ensure(sizeof(double2) * (size_t)n + pad) ||
         g->lev_ticket.ensure(4 * (g->lev_launch.size() + 1) * LV_TICKET_INTS) || !put(t.e, E.slot) ||
         !put(t.l, L.slot) || !put(t.go, go))
         return false;
@@ -839,9 +841,16 @@ bool build_plan(bl_graph *g, int B, int D) {
 }
 }  // namespace
 
+void level_walk_release(bl_graph *g) {
+    g->lev_early.release();
+    g->lev_late.release();
+    for (DevBuf *b : {&g->lev_start, &g->lev_blk, &g->lev_shape, &g->lev_moved, &g->lev_ticket}) b->release();
+}
+
 // The plan for batches of B vertices (cached per batch size and lag): levels, their slices and
 // hubs, the late lists, and the launches.  D > 0: the sums of the lagged walk with lag D and
-// the groups of lag_walk_groups.  False: too many levels, or lists past 2^31 entries.
+// the groups of lag_walk_groups.  False: too many levels, lists past 2^31 entries, or no memory for them, and
+// then no memory held.
 bool level_walk_plan(bl_graph *g, int B, int D) {
     if (g->lev_batch == B && g->lev_d == D) return g->lev_ok;
     g->lev_batch = B;
@@ -850,6 +859,10 @@ bool level_walk_plan(bl_graph *g, int B, int D) {
         g->lev_ok = build_plan(g, B, D);
     } catch (const std::bad_alloc &) {
         g->lev_ok = false;
+    }
+    if (!g->lev_ok) {
+        level_walk_release(g);
+        (void)hipGetLastError();  // the walk in its place runs without it
     }
     return g->lev_ok;
 }
