@@ -2681,13 +2681,14 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     const char *lenv = getenv("BL_LEVELS");
     bool use_level = p->precision != BL_PREC_FP64 && iters > 0 && !wenv && !getenv("BL_LAG_D") && !getenv("BL_LAG_H") &&
                      !getenv("BL_WIDE_D") && !getenv("BL_WIDE_H") && !(lenv && !strcmp(lenv, "0")) &&
-                     level_walk_plan(g, p->batch, use_lag ? lag_d : 0);
+                     level_walk_levels(g, p->batch);
     // The lagged walk stays on graphs whose ids follow the edges with large batches (a 1000 x 1000 grid in
     // row order at -batch 256: 1.99 ms against 2.19; at -batch 64 7.85 against 2.17), the row walk on
     // those of few batches.
     if (use_level && (use_lag || use_row) && !lenv)
         use_level = level_us(n, g->lev_big, g->lev_small) <
                     (use_lag ? lag_us(lag_steps, lag_w, g->lev_small > 0) : row_us(nbt));
+    use_level = use_level && level_walk_plan(g, p->batch, use_lag ? lag_d : 0);
     if (!use_level) {
         if (use_wide) use_wide = wide_walk_fits(g, p->batch);
         if (use_wide) {

@@ -138,10 +138,12 @@ int bh_build_tree(BHWork &w, const double2 *d_pos, int n, hipStream_t s);
 // largest early neighbour (-1: none; g->batch_top).  Cached per batch size.
 void batch_scan(bl_graph *g, int B);
 
-// The walk by dependence levels (walk_level.hip): level_walk_plan builds the plan for batch size B
-// (D > 0: with the sums of the lagged walk at lag D); launch_level_late sums the late attraction
+// The walk by dependence levels (walk_level.hip): level_walk_levels counts the levels for batch size B
+// (g->lev_big, g->lev_small; false: too many); level_walk_plan builds the plan
+// (D > 0: with the sums of the lagged walk at lag D; false: no memory); launch_level_late sums the late attraction
 // into the repulsion, launch_walk_level runs one iteration's walk after it (fast: the operations of the
 // wide walk, else with D = 0 those of the row walk).
+bool level_walk_levels(bl_graph *g, int B);
 bool level_walk_plan(bl_graph *g, int B, int D);
 void level_walk_release(bl_graph *g);
 int launch_level_late(bl_graph *g, double2 *pos, const bl_params *p, bool fast, int it, hipStream_t s);

@@ -121,6 +121,11 @@ struct bl_graph {
     int32_t lev_batch = 0, lev_d = 0, lev_big = 0, lev_small = 0, lev_late_slices = 0, lev_late_rows = 0,
             lev_late_hubs = 0;
     bool lev_ok = false;
+    // its levels at batch size lev_scan: of every vertex, its early entries, and the vertices of each level and
+    // class of row, up to the plan
+    int32_t lev_scan = 0, lev_count = 0;
+    bool lev_scan_ok = false;
+    std::vector<int32_t> lev_of, lev_early_n, lev_first;
     bl::LevelLists lev_early, lev_late;
     bl::DevBuf lev_start, lev_blk, lev_shape, lev_moved, lev_ticket;
     std::vector<bl::LevelLaunch> lev_launch;

@@ -652,14 +652,32 @@ int level_blocks(int slices, int rows, int hubs) {
     return (slices + LV_WAVES - 1) / LV_WAVES + (rows + LV_WAVES - 1) / LV_WAVES + hubs;
 }
 
-bool build_plan(bl_graph *g, int B, int D) {
+// Classes of a level's rows: of 4, 8 and 16 lanes, of a wave, hubs.
+constexpr int LV_CLASSES = 5;
+int row_class(int early) {
+    return early <= LV_NARROW ? 0 : early <= LV_WIDE ? 1 : early <= LV_BROAD ? 2 : early <= LV_WAVE ? 3 : 4;
+}
+int count(const bl_graph *g, int l, int c) {
+    const int32_t *f = g->lev_first.data() + (size_t)l * LV_CLASSES + c;
+    return f[1] - f[0];
+}
+// The end of the run of small levels without rows of more than 8 entries from level l on.
+int run_end(const bl_graph *g, int l) {
+    const auto small = [&](int e) {
+        return count(g, e, 0) + count(g, e, 1) <= LV_RUN && count(g, e, 2) + count(g, e, 3) + count(g, e, 4) == 0;
+    };
+    while (l < g->lev_count && small(l)) ++l;
+    return l;
+}
+
+// Levels and numbers of early entries of all vertices, and the rows of each level and class.
+bool scan_levels(bl_graph *g, int B) {
     const int n = g->n;
     if ((int)g->h_rowptr.size() != n + 1 || (int64_t)g->h_colids.size() != g->nnz) return false;
     const int32_t *rp = g->h_rowptr.data(), *ci = g->h_colids.data();
-    const float *gw = g->h_w.empty() ? nullptr : g->h_w.data();
-    const std::vector<int32_t> go = D > 0 ? lag_walk_groups(g, B) : std::vector<int32_t>();
-    // levels and numbers of early entries
-    std::vector<int32_t> lev(n), ec(n);
+    g->lev_of.resize(n);
+    g->lev_early_n.resize(n);
+    int32_t *lev = g->lev_of.data(), *ec = g->lev_early_n.data();
     int nl = 0;
     for (int b0 = 0; b0 < n; b0 += B)
         for (int i = b0; i < std::min(n, b0 + B); ++i) {
@@ -674,19 +692,36 @@ bool build_plan(bl_graph *g, int B, int D) {
             nl = std::max(nl, top + 2);
         }
     if (nl > LV_MAXLEVELS) return false;
-    // within a level: rows of 4, 8 and 16 lanes, rows of a wave, hubs (the lagged walk's rows, whose sums
-    // stay in list order, have at most 64 entries)
-    constexpr int K = 5;
-    if (D > 0 && g->max_row > LV_ROW) return false;
-    auto cls = [&](int i) {
-        return (size_t)lev[i] * K + (ec[i] <= LV_NARROW ? 0 : ec[i] <= LV_WIDE ? 1 : ec[i] <= LV_BROAD ? 2 : ec[i] <= LV_WAVE ? 3 : 4);
-    };
-    std::vector<int32_t> first((size_t)nl * K + 1, 0), order(n);
-    for (int i = 0; i < n; ++i) ++first[cls(i) + 1];
-    for (size_t k = 0; k < (size_t)nl * K; ++k) first[k + 1] += first[k];
+    g->lev_count = nl;
+    g->lev_first.assign((size_t)nl * LV_CLASSES + 1, 0);
+    int32_t *first = g->lev_first.data();
+    for (int i = 0; i < n; ++i) ++first[(size_t)lev[i] * LV_CLASSES + row_class(ec[i]) + 1];
+    for (size_t k = 0; k < (size_t)nl * LV_CLASSES; ++k) first[k + 1] += first[k];
+    g->lev_big = g->lev_small = 0;
+    for (int l = 0; l < nl;) {
+        const int e = run_end(g, l);
+        if (e - l >= LV_RUNS) g->lev_small += e - l, l = e;
+        else ++g->lev_big, ++l;
+    }
+    return true;
+}
+
+// A plan's host lists, which the launches don't need.
+void forget_levels(bl_graph *g) {
+    for (std::vector<int32_t> *v : {&g->lev_of, &g->lev_early_n, &g->lev_first}) std::vector<int32_t>().swap(*v);
+}
+
+bool build_plan(bl_graph *g, int B, int D) {
+    const int n = g->n, nl = g->lev_count;
+    if (D > 0 && g->max_row > LV_ROW) return false;  // the lagged walk's rows, whose sums stay in list order
+    const int32_t *rp = g->h_rowptr.data(), *lev = g->lev_of.data(), *ec = g->lev_early_n.data();
+    const float *gw = g->h_w.empty() ? nullptr : g->h_w.data();
+    const std::vector<int32_t> go = D > 0 ? lag_walk_groups(g, B) : std::vector<int32_t>();
+    const std::vector<int32_t> &first = g->lev_first;
+    std::vector<int32_t> order(n);
     {
         std::vector<int32_t> at(first.begin(), first.end() - 1);
-        for (int i = 0; i < n; ++i) order[at[cls(i)]++] = i;
+        for (int i = 0; i < n; ++i) order[at[(size_t)lev[i] * LV_CLASSES + row_class(ec[i])]++] = i;
     }
     constexpr int64_t cap = ((int64_t)1 << 31) - 1;
     // Where every vertex's entries go: slot >= 0 the first of its column in a slice (stride 64), < 0
@@ -726,20 +761,14 @@ bool build_plan(bl_graph *g, int B, int D) {
     L.slot.resize(n);
     // the levels' launches: on their own, or runs of small levels without longer rows
     std::vector<int32_t> start;  // of each level of the runs, its first slice in its run, and the run's end
-    auto count = [&](int l, int c) { return first[(size_t)l * K + c + 1] - first[(size_t)l * K + c]; };
-    auto small = [&](int l) {
-        return count(l, 0) + count(l, 1) <= LV_RUN && count(l, 2) + count(l, 3) + count(l, 4) == 0;
-    };
     std::vector<LevelShape> shape;
     std::vector<int32_t> blk;  // of each workgroup of k_level_flow, its level
     g->lev_launch.clear();
-    g->lev_big = g->lev_small = 0;
     for (int l = 0; l < nl;) {
-        int e = l;
-        while (e < nl && small(e)) ++e;
+        const int e = run_end(g, l);
         const int v0 = (int)E.L.vid.size();
         const uint32_t e0 = (uint32_t)(E.nid / 64);
-        const int32_t *vs = order.data() + first[(size_t)l * K];
+        const int32_t *vs = order.data() + first[(size_t)l * LV_CLASSES];
         if (e - l >= LV_RUNS) {
             LevelLaunch q{};
             q.v0 = v0;
@@ -748,25 +777,24 @@ bool build_plan(bl_graph *g, int B, int D) {
             q.l1 = q.l0 + e - l;
             int at = 0;  // slices of the run
             for (; l < e; ++l) {
-                const int m = count(l, 0) + count(l, 1);
+                const int m = count(g, l, 0) + count(g, l, 1);
                 start.push_back(at);
-                E.slices(order.data() + first[(size_t)l * K], m, LV_WIDE);
+                E.slices(order.data() + first[(size_t)l * LV_CLASSES], m, LV_WIDE);
                 at += (m + 63) / 64;
             }
             start.push_back(at);
-            g->lev_small += q.l1 - q.l0;
             g->lev_launch.push_back(q);
         } else {
             LevelShape q{};
             q.v0 = v0;
             q.e0 = e0;
-            q.nn = E.short_rows(vs, count(l, 0), LV_NARROW);
-            q.nw = E.short_rows(vs += count(l, 0), count(l, 1), LV_WIDE);
-            q.nb = E.short_rows(vs += count(l, 1), count(l, 2), LV_BROAD);
-            vs += count(l, 2);
+            q.nn = E.short_rows(vs, count(g, l, 0), LV_NARROW);
+            q.nw = E.short_rows(vs += count(g, l, 0), count(g, l, 1), LV_WIDE);
+            q.nb = E.short_rows(vs += count(g, l, 1), count(g, l, 2), LV_BROAD);
+            vs += count(g, l, 2);
             q.r0 = (int)E.L.row.size();
-            q.nr = count(l, 3);
-            const int nh = count(l, 4);
+            q.nr = count(g, l, 3);
+            const int nh = count(g, l, 4);
             for (int t = 0; t < q.nr + nh; ++t) E.row(vs[t], ec[vs[t]]);
             if (g->lev_launch.empty() || g->lev_launch.back().l1 > g->lev_launch.back().l0) {
                 LevelLaunch f{};
@@ -781,7 +809,6 @@ bool build_plan(bl_graph *g, int B, int D) {
             blk.insert(blk.end(), (size_t)(f.blocks - q.first), (int32_t)shape.size());
             shape.push_back(q);
             ++f.levels;
-            ++g->lev_big;
             ++l;
         }
         if (E.nid > cap * 32 || (int64_t)E.L.vid.size() > cap) return false;
@@ -841,6 +868,21 @@ bool build_plan(bl_graph *g, int B, int D) {
 }
 }  // namespace
 
+// The levels for batches of B vertices, in g->lev_big (of launches of consecutive levels) and g->lev_small (of
+// runs); cached per batch size.  False: too many.  What the plan's making takes beyond it is spent only
+// where the levels are chosen.
+bool level_walk_levels(bl_graph *g, int B) {
+    if (g->lev_scan == B && (!g->lev_scan_ok || g->lev_batch == B || !g->lev_of.empty())) return g->lev_scan_ok;
+    g->lev_scan = B;
+    try {
+        g->lev_scan_ok = scan_levels(g, B);
+    } catch (const std::bad_alloc &) {
+        g->lev_scan_ok = false;
+    }
+    if (!g->lev_scan_ok) forget_levels(g);
+    return g->lev_scan_ok;
+}
+
 void level_walk_release(bl_graph *g) {
     g->lev_early.release();
     g->lev_late.release();
@@ -849,17 +891,19 @@ void level_walk_release(bl_graph *g) {
 
 // The plan for batches of B vertices (cached per batch size and lag): levels, their slices and
 // hubs, the late lists, and the launches.  D > 0: the sums of the lagged walk with lag D and
-// the groups of lag_walk_groups.  False: too many levels, lists past 2^31 entries, or no memory for them, and
-// then no memory held.
+// the groups of lag_walk_groups.  False: lists past 2^31 entries, or no memory for them, and then no memory held.
 bool level_walk_plan(bl_graph *g, int B, int D) {
     if (g->lev_batch == B && g->lev_d == D) return g->lev_ok;
-    g->lev_batch = B;
-    g->lev_d = D;
+    g->lev_batch = 0;  // scanned again if the last plan has used the levels up
+    if (!level_walk_levels(g, B)) return false;
     try {
         g->lev_ok = build_plan(g, B, D);
     } catch (const std::bad_alloc &) {
         g->lev_ok = false;
     }
+    g->lev_batch = B;
+    g->lev_d = D;
+    forget_levels(g);
     if (!g->lev_ok) {
         level_walk_release(g);
         (void)hipGetLastError();  // the walk in its place runs without it

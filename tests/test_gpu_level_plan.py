@@ -1,5 +1,5 @@
-"""A level plan that there is no memory for leaves none behind: the walk in its place runs, with the same
-layout."""
+"""The level walk's plan takes device memory only where the levels are chosen, and a plan that there is no
+memory for leaves none behind: the walk in its place runs, with the same layout."""
 import numpy as np
 import pytest
 import torch
@@ -16,6 +16,26 @@ def _taken(g, x0, **kw):
     out = g.run(x0, algo=4, iters=1, bht=1.2, **kw)
     torch.cuda.synchronize()
     return before - torch.cuda.mem_get_info()[0], out
+
+
+def test_rejected_levels_take_no_memory(bl, monkeypatch):
+    """A grid in row order at -batch 256: the lagged walk is the faster one."""
+    rp, ci = graphs.csr_from_edges(*graphs.grid(700, 700))
+    x0 = np.random.default_rng(8).random((len(rp) - 1, 2))
+    print("[case] plan of levels that are not chosen", flush=True)
+    monkeypatch.delenv("BL_LEVELS", raising=False)
+    with bl.Graph(rp, ci) as g:  # the library's first use
+        g.run(x0, algo=4, iters=1, batch=256)
+    taken = {}
+    for levels in ("0", None):
+        if levels:
+            monkeypatch.setenv("BL_LEVELS", levels)
+        else:
+            monkeypatch.delenv("BL_LEVELS")
+        with bl.Graph(rp, ci) as g:
+            taken[levels], (_, st) = _taken(g, x0, batch=256)
+            assert st.walk == bl.WALK_LAG and st.walk_levels == 0
+    assert taken[None] == taken["0"], taken
 
 
 @pytest.mark.parametrize("kind,batch,walk", [("rgg", 64, "LAG"), ("rmat", 1024, "WIDE")])
