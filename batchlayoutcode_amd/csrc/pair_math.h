@@ -302,19 +302,25 @@ __device__ __forceinline__ double2 apart_share(At at, const int n, const int t, 
                                                const double py, const int *__restrict__ ci, const int e0, const int e1,
                                                Weight weight, const int law) {
     double fx = 0.0, fy = 0.0;
+    int e = e0, next = -1;  // ci[e], once read
     for (int j = t; j < n; j += D) {
         const double2 q = at(j);
         if (too_close<true>(q.x - px, q.y - py)) {
-            int lo = e0, hi = e1;  // the first neighbour >= j
-            while (lo < hi) {
-                const int m = (lo + hi) >> 1;
-                if (ci[m] < j) lo = m + 1; else hi = m;
+            if (next < j) {  // on to the first neighbour >= j, in growing steps
+                int step = 1;
+                for (; e < e1 && ci[min(e + step, e1) - 1] < j; step <<= 1) e = min(e + step, e1);
+                int hi = min(e + step, e1);
+                while (e < hi) {
+                    const int m = (e + hi) >> 1;
+                    if (ci[m] < j) e = m + 1; else hi = m;
+                }
+                next = e < e1 ? ci[e] : 0x7fffffff;
             }
-            if (lo < e1 && ci[lo] == j) continue;
+            if (next == j) continue;
         }
         pair_rep<true>(q.x, q.y, px, py, fx, fy);
     }
-    for (int e = e0 + t; e < e1; e += D) {
+    for (e = e0 + t; e < e1; e += D) {
         const double2 q = at(ci[e]);
         const double dx = q.x - px, dy = q.y - py;
         correct_pair(law, weight(e), dx, dy, too_close<true>(dx, dy) ? 0.0 : inv_r2<true>(dx, dy), fx, fy);

@@ -136,3 +136,28 @@ def test_coincident_vertices_in_one_group(bl, monkeypatch, kernel):
         bound = 2 * (n + 16) * eps * tot / mag + 8 * eps * (1 + np.abs(x).max(1))
         worst = (np.abs(got - F / mag[:, None]).max(1) / bound).max()
         assert worst <= 1.0, (n, m, float(worst))
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+def test_all_vertices_in_a_tiny_ball(bl, monkeypatch, kernel):
+    """Every pair is closer than 2^-40, linked or not: a vertex's neighbours, up to all others, are found among
+    them all.  No attraction: |F| against extended precision as above."""
+    eps = 2.0 ** -53
+    rng = np.random.default_rng(4)
+    for n, deg in ((7, 2), (130, 4), (1000, 9), (1024, 40)):
+        print(f"[case] tiny ball, {kernel} n {n} degree {deg}", flush=True)
+        x = 1e-14 * rng.random((n, 2))
+        e = np.concatenate([rng.integers(0, n, (n * deg // 2, 2)), np.stack([np.full(n, n // 2), np.arange(n)], 1)])
+        e = np.unique(np.sort(e[e[:, 0] != e[:, 1]], 1), axis=0)
+        e = e[~((e == 0).any(1) & (e == n // 2).any(1))]  # the hub keeps one repulsion: a direction
+        rp, ci = _linked(n, e)
+        xy, en = _run(bl, monkeypatch, kernel, rp, ci, x, algo=8, iters=1, weight=0.0, batch=1024, step0=1e-14)
+        _, _, t = _terms(x)
+        t[_met(rp, ci)] = 0
+        F = -t.sum(1)
+        mag = np.sqrt((F * F).sum(-1))
+        tot = np.sqrt((t * t).sum(-1)).sum(1)
+        got = (xy.astype(np.longdouble) - x) / 1e-14
+        bound = 2 * (n + 16) * eps * tot / mag + 16 * eps
+        worst = (np.abs(got - F / mag[:, None]).max(1) / bound).max()
+        assert worst <= 1.0, (n, float(worst))
