@@ -84,7 +84,7 @@ __global__ __launch_bounds__(WG) void k_pairs32(const double2 *__restrict__ pos,
     constexpr int IPW = WG / JS;
     __shared__ double2 red[WG];
     const int tid = threadIdx.x;
-    if ((int)blockIdx.x >= G) {
+    if (__builtin_expect((int)blockIdx.x >= G, 0)) {  // its code last: 0.5 us a step with it before the dense sum's
         if (blockIdx.y != 0) return;
         const int w = ((int)blockIdx.x - G) * (WG / 64) + tid / 64;
         const int lane = tid & 63;
@@ -167,7 +167,6 @@ __global__ __launch_bounds__(NT) void k_step32(const double2 *__restrict__ src, 
                                                int law, const double *__restrict__ stepp, double step,
                                                double *__restrict__ eterm) {
     __shared__ double2 red[NT / 64];
-    __shared__ uint64_t near[NT / 64];
     const int tid = threadIdx.x;
     const int i = b0 + (int)blockIdx.x;
     const double2 pi = src[i];
@@ -190,29 +189,28 @@ __global__ __launch_bounds__(NT) void k_step32(const double2 *__restrict__ src, 
     }
     ax = wave_sum(ax + cx);
     ay = wave_sum(ay + cy);
-    const uint64_t any = __ballot(close);
-    if ((tid & 63) == 0) red[tid >> 6] = make_double2(ax, ay), near[tid >> 6] = any;
+    const double mark = __longlong_as_double(APART);
+    if (__ballot(close)) ax = mark;
+    if ((tid & 63) == 0) red[tid >> 6] = make_double2(ax, ay);
     __syncthreads();
-    if constexpr (REFINE) {
-        uint64_t apart = 0;
-#pragma unroll
-        for (int w = 0; w < NT / 64; ++w) apart |= near[w];
-        if (apart) {
-            const double2 f = apart_share(at, n, tid, NT, pi.x, pi.y, eci, e0, e1,
-                                          [=](int e) { return ew ? W * (double)ew[e] : W; }, law);
-            ax = wave_sum(f.x);
-            ay = wave_sum(f.y);
-            __syncthreads();
-            if ((tid & 63) == 0) red[tid >> 6] = make_double2(ax, ay);
-            __syncthreads();
-        }
-    }
     if (tid == 64)
         for (int k = (int)blockIdx.x; k < pc; k += (int)gridDim.x) dst[p0 + k] = src[p0 + k];
-    if (tid == 0) {
-        double fx = red[0].x, fy = red[0].y;
+    if (tid >= 64) return;
+    double fx = red[0].x, fy = red[0].y;
 #pragma unroll
-        for (int w = 1; w < NT / 64; ++w) fx += red[w].x, fy += red[w].y;
+    for (int w = 1; w < NT / 64; ++w) fx += red[w].x, fy += red[w].y;
+    if (REFINE && isnan(fx)) {  // the same in all lanes
+        bool apart = false;
+#pragma unroll
+        for (int w = 0; w < NT / 64; ++w) apart = apart || __double_as_longlong(red[w].x) == APART;
+        if (apart) {
+            const double2 f = apart_share(at, n, tid, 64, pi.x, pi.y, eci, e0, e1,
+                                          [=](int e) { return ew ? W * (double)ew[e] : W; }, law);
+            fx = wave_sum(f.x);
+            fy = wave_sum(f.y);
+        }
+    }
+    if (tid == 0) {
         dst[i] = moved(pi, fx, fy, stepp ? *stepp : step);
         eterm[i] = fx * fx + fy * fy;
     }

@@ -266,10 +266,10 @@ __device__ __forceinline__ double group_factor(At at, const int first, const int
 }
 
 // The factor to remove a linked pair (dx, dy) with: bit for bit the dense sum's where the pair is close (group:
-// whether it was in one).  Further away than 2^-4 one of its own, which differs by about 2^-52: less than the
+// whether it was in one).  Further away than 2^-8 one of its own, which differs by about 2^-52: less than the
 // roundings of the dense sum's additions after the pair.  (Eight loads for every neighbour made the step of the
 // 250k random geometric graph 4% longer: the correction's workgroups hold up the last of the others.)
-constexpr double kNear2 = 0x1p-8;
+constexpr double kNear2 = 0x1p-16;
 template <bool REFINE, class At>
 __device__ __forceinline__ double linked_factor(At at, const bool group, const int first, const int m, const int D,
                                                 const int end, const double px, const double py, const double dx,
