@@ -48,8 +48,6 @@
 
 namespace bl {
 
-// out: 4 + 256 doubles, the sum in out[0] (minibatch.hip)
-
 namespace {
 
 constexpr int WG = 256;
@@ -2677,7 +2675,10 @@ int run_bh(bl_graph *g, double *d_xy, const bl_params *p, double step0, int iter
     int lag_steps = use_row && lag_d > 0 ? lag_walk_steps(g, p->batch, lag_d, &lag_w) : 0;
     if (wenv && (!strcmp(wenv, "row") || !strcmp(wenv, "single"))) lag_steps = 0;  // no helpers
     bool use_lag = lag_steps > 0;
-    // by dependence levels, whichever walk the graph's shape selects (its switches keep it)
+    // by dependence levels, whichever walk the graph's shape selects (its switches keep it); in place of the
+    // grid, wide, entry-split and split walks always: on bands of 16 to 300 neighbours, sorted geometric, R-MAT,
+    // random and grid graphs at -batch 32 to 8,192 the levels took 1.75 times less (a band of 64 at -batch 64,
+    // 1,563 levels for 1,563 batches: 3.4 against 6.0 ms) to 170
     const char *lenv = getenv("BL_LEVELS");
     bool use_level = p->precision != BL_PREC_FP64 && iters > 0 && !wenv && !getenv("BL_LAG_D") && !getenv("BL_LAG_H") &&
                      !getenv("BL_WIDE_D") && !getenv("BL_WIDE_H") && !(lenv && !strcmp(lenv, "0")) &&

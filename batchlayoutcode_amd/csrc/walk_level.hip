@@ -26,11 +26,11 @@
 //   - rows of up to 4 entries take 4 lanes each, rows of up to 8 take 8, of up to 16 16, at an address that
 //     the lane's number gives: a lane forms the factors of one entry, and the lanes' products are added one
 //     after another by DPP moves (with rows of 9 to 16 entries one a wave the random geometric graph's walk
-//     took 5,183 tickets and 75 us, now 64; R-MAT 486 -> 460);
+//     took 5,183 tickets and 75 us, now 64; R-MAT 486 -> 455);
 //   - rows of up to LV_WAVE entries one a wave, longer ones (hubs) one a workgroup.
 // What bounds the walk: on R-MAT the hand-off of 188 levels; on the triangulation random 16-byte reads and
-// writes (1.66M moves in 195 us).  k_level_flow against a launch a level: R-MAT scale 20 at -batch 1024
-// 989 -> 462 us, 250k random geometric graph 111 -> 65, triangulation 215 -> 195.
+// writes (1.66M moves in 198 us).  k_level_flow against a launch a level: R-MAT scale 20 at -batch 1024
+// 989 -> 455 us, 250k random geometric graph 111 -> 64, triangulation 215 -> 198.
 // Runs of levels of at most LV_RUN vertices without rows beyond 8 entries are one launch of one
 // workgroup, which takes the levels one after another with a barrier between them (1.2 to 3 us each) and
 // loads a level's vertices and entries two levels ahead.
